@@ -35,21 +35,17 @@ sweeps per step, and E_k / enstrophy at step 1000 against the FP64 form.
 The mixing workload runs the same series over 500 steps (--late-total).
 
 roofline: the dominant work of the headline form is the red-black SOR
-iteration (in the mixed forms the FP32 colour-split red and black launches,
-sor_split_kernel<0> and <1>).  Its algorithmic bytes per iteration are those
-of a red-black sweep that reads the whole iterate once per colour: (2 reads
-of p, 1 read of rhs, 1 write of p) = 4 values per cell, 16 B/cell in FP32 and
-32 B/cell in FP64, times the cell count; the floor of one read of p and rhs
-and one write of p (12 / 24 B/cell) is reported beside it.  Its average
-duration is measured with HIP events on the launch stream over complete
-batches of iterations inside the timed steps (the start event follows each
-batch's first iteration), and, for the FP32 iteration, right after the
-timed steps over 200 back-to-back iterations of the solver's own correction
-problem (o3d_solver_sor_period, one event interval of 199 iterations): the
-in-step intervals hold only 7 to 10 iterations each, and the two events'
-own processing adds about 3 us per iteration to them.  The roofline uses
-the back-to-back figure and reports the in-step one beside it; `traffic` is the measured HBM
-bytes of one iteration (both launches) from the committed rocprofv3 --pmc
+sweeps (sor_pair_kernel, two iterations per launch).  The algorithmic bytes
+of a launch are one read of the iterate and of the rhs and one write of the
+iterate, 12 B/cell in FP32 and 24 B/cell in FP64.  Its average duration is
+measured with HIP events on the launch stream over launches inside the timed
+steps (the start event follows each batch's first launch), and, for FP32,
+right after the timed steps over 200 back-to-back iterations of the solver's
+own correction problem (o3d_solver_sor_period, one event interval of 99
+launches): the in-step intervals hold only 3 to 7 launches each, and the two
+events' own processing adds to them.  The roofline uses the back-to-back
+figure and reports the in-step one beside it; `traffic` is the measured HBM
+bytes of one launch from the committed rocprofv3 --pmc
 summary.  The ceiling beside the nominal 8 TB/s is a hand-written streaming
 triad over three 1 GiB buffers (o3d_stream_probe).
 
@@ -113,7 +109,7 @@ def parse_args():
     return ap.parse_args()
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "sor_split_kernel_tgv256_pmc.md")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "sor_pair_kernel_tgv256_pmc.md")
 
 
 def measured_traffic(which):
@@ -238,32 +234,28 @@ def run_form(form, cfg, steps, warmup, model_path, init=None, coarse=(0, 0)):
         "enstrophy": st[4],
         "t_end": t_end,
     }
-    # SOR iterations: average duration from events over complete batches of
-    # launches (one launch = one red-black iteration: the red and the black
-    # colour-split launch, sor_split_kernel<0> and <1>).  Algorithmic bytes
-    # of an iteration: a red-black sweep reading the whole iterate once per
-    # colour, the rhs once and writing the iterate once, 4 values per cell
-    # (32 B/cell FP64, 16 B/cell FP32); the floor of one read of p and rhs
-    # and one write of p (24 / 12 B/cell) beside it.
-    for q, name, bpc, floor in ((0, "sor_f64", 32, 24), (1, "sor_f32", 16, 12)):
+    # SOR sweeps: average duration from events over launches that all ran (two
+    # red-black iterations each; the fused kernel of other grids one).
+    # Algorithmic bytes of a launch: one read of p and of the rhs and one
+    # write of p (24 B/cell FP64, 12 B/cell FP32).
+    for q, name, bpc in ((0, "sor_f64", 24), (1, "sor_f32", 12)):
         if sor_ln[q] > 0:
             avg_ms = sor_ms[q] / sor_ln[q]
-            gbs = bpc * n / (avg_ms * 1e-3) / 1e9
-            out[name] = {"in_step_us_per_iteration": 1e3 * avg_ms,
+            per = sor_sw[q] / sor_ln[q]
+            out[name] = {"in_step_us_per_iteration": 1e3 * sor_ms[q] / sor_sw[q],
                          "avg_launch_us": 1e3 * avg_ms, "launches_timed": sor_ln[q],
-                         "iterations_per_launch": sor_sw[q] / sor_ln[q],
+                         "iterations_per_launch": per,
                          "us_per_iteration": 1e3 * sor_ms[q] / sor_sw[q],
-                         "algorithmic_bytes_per_launch": bpc * n, "achieved_GBps": gbs,
-                         "floor_bytes_per_launch": floor * n,
-                         "floor_GBps": floor * n / (avg_ms * 1e-3) / 1e9}
+                         "algorithmic_bytes_per_launch": bpc * n,
+                         "achieved_GBps": bpc * n / (avg_ms * 1e-3) / 1e9}
             if q == 1 and period_us:
                 # The roofline figure: the back-to-back period, whose event
-                # interval spans 199 iterations.
-                avg_ms = period_us * 1e-3
+                # interval spans 99 launches.
+                avg_ms = period_us * per * 1e-3
                 out[name].update({
-                    "avg_launch_us": period_us, "timing": "back-to-back, 199 iterations",
-                    "achieved_GBps": bpc * n / (avg_ms * 1e-3) / 1e9,
-                    "floor_GBps": floor * n / (avg_ms * 1e-3) / 1e9})
+                    "us_per_iteration": period_us, "avg_launch_us": 1e3 * avg_ms,
+                    "timing": "back-to-back, 99 launches",
+                    "achieved_GBps": bpc * n / (avg_ms * 1e-3) / 1e9})
     if cc or gs:
         out["coarse_cycles"] = cc
         out["smooth_sweeps"] = gs
@@ -563,9 +555,9 @@ def main():
     dom = head.get("sor_" + which)
     roofline = None
     if dom:
-        kname = ("sor_split_kernel<float,0> + <float,1> (one colour-split red-black "
-                 "iteration, f32)" if which == "f32" else
-                 "sor_split_kernel<double,0> + <double,1> (one red-black iteration, f64)")
+        kname = ("sor_pair_kernel<float> (two colour-split red-black iterations, f32)"
+                 if which == "f32" else
+                 "sor_pair_kernel<double> (two red-black iterations, f64)")
         roofline = {"bound": "hbm", "kernel": kname,
                     "achieved": dom["achieved_GBps"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": dom["achieved_GBps"] / HBM_PEAK_GBS,
@@ -574,8 +566,6 @@ def main():
                     "avg_launch_us": dom["avg_launch_us"],
                     "timing": dom.get("timing", "in-step event batches"),
                     "in_step_us_per_iteration": dom["in_step_us_per_iteration"],
-                    "floor_bytes": dom["floor_bytes_per_launch"],
-                    "frac_floor": dom["floor_GBps"] / HBM_PEAK_GBS,
                     "frac_of_stream_probe": dom["achieved_GBps"] / copy_gbs,
                     "stream_probe_GBps": copy_gbs}
     late = None

@@ -132,8 +132,8 @@ int o3d_poisson(double *pp, const double *rhs, double dx, double dy, double dz, 
 /* The red-black SOR of o3d_poisson in FP32 (the sweeps of the mixed form),
  * same rules and outputs.  variant selects the kernels, both with
  * bit-identical iterates: 0 = one fused red+black iteration per launch;
- * 2 = colour-split storage, one in-place launch per colour (nx a multiple
- * of 8; the form the mixed solver uses).  No counterpart in the reference
+ * 2 = colour-split storage, two iterations per launch (nx a multiple of 8;
+ * the form the mixed solver uses).  No counterpart in the reference
  * (its solver is FP64). */
 int o3d_poisson_f32(float *pp, const float *rhs, double dx, double dy, double dz, int nx, int ny,
                     int nz, double *omega, double eps, int kmax, int idyn, int solver,
@@ -352,15 +352,15 @@ int o3d_copy(void *dst, const void *src, size_t bytes);
 /* Time of SOR sweeps measured with HIP events on the launch stream over the
  * last step: total ms of complete sweep batches, the number of sweeps
  * (iterations) and of kernel launches in them, per precision (index 0 FP64,
- * 1 FP32; one iteration per launch: a fused red+black launch, or with
- * colour-split storage the red and the black launch counted as one).
+ * 1 FP32; a launch is one iteration in the fused kernel and two with
+ * colour-split storage).
  * launches2 may be NULL. */
 int o3d_solver_sor_timing(void *handle, double *ms2, int *sweeps2, int *launches2);
 /* Mixed form with colour-split sweeps: `iterations` back-to-back FP32
- * red-black iterations (two launches each) of the solver's correction
+ * red-black iterations (two per launch, rounded up to at least two launches) of the solver's correction
  * problem, eps 0 so none stops, on its correction and residual buffers
  * (scratch between solves), timed with HIP events on the launch stream from
- * the end of the first iteration to the end of the last; us = the mean time
+ * the end of the first launch to the end of the last; us = the mean time
  * per iteration.  For measurement: the event interval spans many iterations,
  * so it holds the kernels and the gaps between back-to-back launches only.
  * No counterpart in the reference. */

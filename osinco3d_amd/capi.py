@@ -248,8 +248,8 @@ def multigrid(u, f, h, per, cycles):
 
 def poisson_f32(pp, rhs, d, omega, eps, kmax, idyn, solver, variant=0):
     """FP32 red-black SOR; returns (exit_iter, dmax, reason, omega).
-    variant: 0 fused iteration per launch, 1 two iterations per launch,
-    2 colour-split half sweeps (identical iterates)."""
+    variant: 0 fused iteration per launch, 2 colour-split storage and two
+    iterations per launch (identical iterates)."""
     nx, ny, nz = _dims(pp)
     om = C.c_double(omega)
     it = C.c_int(0)

@@ -292,16 +292,16 @@ SorConst sor_const(double dx, double dy, double dz) {
 
 // Batched launcher of red-black iterations with device-side stop control.
 // Buffers: buf[0] holds the start iterate; launch L reads buf[L & 1] and
-// writes buf[(L + 1) & 1].  With `split` (T == TR) each launch is one
-// iteration of the colour-split in-place sweeps on `sa` (buf unused).
+// writes buf[(L + 1) & 1].  With `pair` (T == TR) each launch is two
+// iterations on colour-split storage, the buffers in `pa` (buf unused).
 template <typename T, typename TR>
 struct SorRun {
   SorArgs<T, TR> a;
   SorState *st = nullptr;    // device
   SorState *hst = nullptr;   // pinned host copy
   T *buf[2] = {nullptr, nullptr};
-  bool split = false;
-  SorSplitArgs<T> sa{};
+  bool pair = false;
+  SorPairArgs<T> pa{};
   // Timing of complete batches (all launches did their iterations).  The
   // start event is recorded after a batch's first iteration, so it completes
   // while the queue is busy and the interval holds back-to-back iterations
@@ -316,22 +316,59 @@ struct SorRun {
   // solve that ends inside its first batch still times iterations 2..a.gs.
   hipEvent_t mid = nullptr;
 
-  hipError_t launch() {
-    if constexpr (std::is_same<T, TR>::value) {
-      if (split) {
-        sa.it = a.it;
-        return launch_sor_split_iteration<T>(sa, g_stream);
-      }
-    }
-    return launch_sor_iteration<T, TR>(a, g_stream);
-  }
-
   // Buffer holding the result after `sweeps` iterations.
   T *result(int sweeps) const { return buf[sweeps & 1]; }
 
+  // The pair kernel: first the launches of a solve of `expect` sweeps (an odd
+  // count takes its last pair back and runs one sweep alone, unless kmax ends
+  // it) and the one that sees the stop, then 8 at a time.
+  int run_pair(double omega, int expect, int *sweeps_out) {
+    HIPCHK(launch_sor_pair_init<T>(pa, omega, g_stream));
+    expect = std::min(std::max(1, expect), pa.kmax);
+    int batch = (expect + 1) / 2 + 1 + ((expect & 1) && expect < pa.kmax ? 1 : 0);
+    pa.launch = 0;
+    bool first = true;
+    while (true) {
+      hipEvent_t e0 = (*events)[0], e1 = (*events)[1];
+      bool mid_set = false;
+      for (int b = 0; b < batch; ++b) {
+        HIPCHK(launch_sor_pair<T>(pa, g_stream));
+        ++pa.launch;
+        if (b == 0) HIPCHK(hipEventRecord(e0, g_stream));
+        if (mid && first && b > 0 && pa.launch == pa.gs / 2) {
+          HIPCHK(hipEventRecord(mid, g_stream));
+          mid_set = true;
+        }
+      }
+      HIPCHK(hipEventRecord(e1, g_stream));
+      HIPCHK(hipMemcpyAsync(hst, st, sizeof(SorState), hipMemcpyDeviceToHost, g_stream));
+      HIPCHK(hipStreamSynchronize(g_stream));
+      // Timed are launches that ran two iterations each: a batch the solve
+      // did not end in, or the Gauss-Seidel opening.
+      const int timed = !hst->done ? batch - 1
+                                   : (mid_set && hst->sweeps >= pa.gs ? pa.gs / 2 - 1 : 0);
+      if (timed > 0) {
+        float ms = 0.f;
+        HIPCHK(hipEventElapsedTime(&ms, e0, hst->done ? mid : e1));
+        ms_full += ms;
+        sweeps_full += 2 * timed;
+        launches_full += timed;
+      }
+      if (hst->done) break;
+      // At most two launches per iteration (a pair and its first sweep again).
+      if (pa.launch > 2 * pa.kmax + 16) return fail("SOR state did not close after kmax");
+      first = false;
+      batch = 8;
+    }
+    *sweeps_out = hst->sweeps;
+    return 0;
+  }
+
   int run(double omega, int first_batch, int *sweeps_out) {
+    if constexpr (std::is_same<T, TR>::value) {
+      if (pair) return run_pair(omega, first_batch, sweeps_out);
+    }
     HIPCHK(launch_sor_init(st, omega, 0, g_stream));
-    if (split) HIPCHK(launch_sor_split_init(sa.dslot, g_stream));
     int it = 1, L = 0;
     int batch = std::max(1, first_batch);
     bool first = true, mid_set = false;
@@ -343,7 +380,7 @@ struct SorRun {
         a.it = it;
         a.pin = buf[L & 1];
         a.pout = buf[(L + 1) & 1];
-        HIPCHK(launch());
+        HIPCHK((launch_sor_iteration<T, TR>(a, g_stream)));
         ++L;
         ++it;
         if (b == 0 && batch > 1) {
@@ -774,35 +811,32 @@ extern "C" int o3d_predict_velocity(double *ux_pred, double *uy_pred, double *uz
   return s.finish();
 }
 
-// The colour-split sweep arguments matching `a` (red, black and the rhs
-// halves already in split storage).
+// The arguments of the pair kernel matching `a`, on the split buffers b0 (the
+// start iterate) and b1 and the split rhs.
 template <typename T>
-SorSplitArgs<T> split_args(const SorArgs<T, T> &a, T *red, T *black, const T *rhs_red,
-                           const T *rhs_black, unsigned long long *dslot) {
-  SorSplitArgs<T> sa{};
-  sa.red = red;
-  sa.black = black;
-  sa.rhs_red = rhs_red;
-  sa.rhs_black = rhs_black;
-  sa.st = a.st;
-  sa.dslot = dslot;
-  sa.log = a.log;
-  sa.log_len = a.log_len;
-  sa.nx = a.nx; sa.ny = a.ny; sa.nz = a.nz;
-  for (int q = 0; q < 3; ++q) sa.per[q] = a.per[q];
-  sa.ox = a.ox; sa.oy = a.oy; sa.oz = a.oz; sa.A = a.A;
-  sa.eps = a.eps;
-  sa.factor = a.factor;
-  sa.kmax = a.kmax;
-  sa.idyn = a.idyn;
-  sa.it = a.it;
-  sa.gs = a.gs;
-  return sa;
+SorPairArgs<T> pair_args(const SorArgs<T, T> &a, T *b0, T *b1, const T *rhs,
+                         unsigned long long *dslot) {
+  SorPairArgs<T> pa{};
+  pa.buf[0] = b0;
+  pa.buf[1] = b1;
+  pa.rhs = rhs;
+  pa.st = a.st;
+  pa.dslot = dslot;
+  pa.nx = a.nx; pa.ny = a.ny; pa.nz = a.nz;
+  for (int q = 0; q < 3; ++q) pa.per[q] = a.per[q];
+  pa.ox = a.ox; pa.oy = a.oy; pa.oz = a.oz; pa.A = a.A;
+  pa.eps = a.eps;
+  pa.factor = a.factor;
+  pa.kmax = a.kmax;
+  pa.idyn = a.idyn;
+  pa.gs = a.gs;
+  sor_pair_tiling<T>(pa);
+  return pa;
 }
 
 namespace {
-// variant: 0 one fused iteration per launch, 2 colour-split half sweeps,
-// -1 the colour-split sweeps where the grid allows them, else the fused
+// variant: 0 one fused iteration per launch, 2 colour-split sweeps, two
+// iterations per launch, -1 the colour-split sweeps where the grid allows them, else the fused
 // kernel (identical iterates in every case).
 template <typename T>
 int poisson_dev(T *pp, const T *rhs, double dx, double dy, double dz, int nx, int ny, int nz,
@@ -844,21 +878,23 @@ int poisson_dev(T *pp, const T *rhs, double dx, double dy, double dz, int nx, in
   a.gs = 0;
   int sweeps = 0;
   int rc = 0;
-  if (variant == 2 || (variant < 0 && sor_split_supported<T>(nx, ny, nz))) {
+  if (variant == 2 || (variant < 0 && sor_split_supported<T>(nx))) {
     // Colour-split copies of the iterate (in `other`) and of the rhs.
     T *rs;
     unsigned long long *dslot;
     CHK(s.scratch(n, &rs));
-    CHK(s.scratch(sor_split_slot_words(), &dslot));
+    CHK(s.scratch(sor_pair_slot_words(), &dslot));
     const int h = n / 2;
     HIPCHK(launch_split<T>(pp, other, other + h, nx, ny, nz, g_stream));
     HIPCHK(launch_split<T>(rhs, rs, rs + h, nx, ny, nz, g_stream));
-    r.split = true;
-    r.sa = split_args<T>(a, other, other + h, rs, rs + h, dslot);
+    // pp is free while its split copy is the iterate.
+    r.pair = true;
+    r.pa = pair_args<T>(a, other, pp, rs, dslot);
     rc = r.run(*omega, 16, &sweeps);
+    if (rc == 0 && r.hst->result == 1) HIPCHK(launch_copy<T>(other, pp, n, g_stream));
     if (rc == 0) HIPCHK(launch_unsplit<T>(pp, other, other + h, nx, ny, nz, g_stream));
   }
-  if (!r.split) {
+  if (!r.pair) {
     rc = r.run(*omega, 16, &sweeps);
     if (rc == 0 && r.result(sweeps) != pp)
       rc = launch_copy<T>(pp, other, n, g_stream) == hipSuccess ? 0 : fail("copy failed");
@@ -1083,7 +1119,7 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
   if (solver < 0 || solver >= SOR_KINDS)
     return fail("no Poisson solver bound for these boundaries");
   CHK(check_red_black(solver, nx, ny, nz));
-  if (!sor_split_supported<float>(nx, ny, nz) || ny % 2 || nz % 2)
+  if (!sor_split_supported<float>(nx) || ny % 2 || nz % 2)
     return fail("multigrid needs nx a multiple of 8 and ny, nz even (grid %dx%dx%d)", nx, ny,
                 nz);
   if (npre < 0 || npost < 0 || npre + npost < 1)
@@ -1128,9 +1164,10 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
   CHK(s.scratch(mg_plan(H, m0, h, per), &mgbuf));
   mg_bind(H, mgbuf);
   H.levels = std::min(H.levels, std::max(nlevels - 1, 0));
-  float *R, *E;
+  float *R, *E, *E2;
   CHK(s.scratch(n, &R));
   CHK(s.scratch(n, &E));
+  CHK(s.scratch(n, &E2));
   const int nb = residual_blocks(nx, ny, nz);
   double *part;
   CHK(s.scratch((size_t)4 * nb + 4, &part));
@@ -1140,7 +1177,7 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
   SorRun<float, float> run;
   CHK(s.scratch(1, &run.st));
   unsigned long long *dslot;
-  CHK(s.scratch(sor_split_slot_words(), &dslot));
+  CHK(s.scratch(sor_pair_slot_words(), &dslot));
   HIPCHK(hipHostMalloc((void **)&run.hst, sizeof(SorState)));
   double *hfin = nullptr;
   if (hipHostMalloc((void **)&hfin, 4 * sizeof(double)) != hipSuccess) {
@@ -1164,9 +1201,8 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
   a.idyn = 0;
   a.it = 0;
   a.gs = npre + npost;
-  const size_t half = n / 2;
-  run.split = true;
-  run.sa = split_args<float>(a, E, E + half, R, R + half, dslot);
+  run.pair = true;
+  run.pa = pair_args<float>(a, E, E2, R, dslot);
   int rc = 0, done = 0, why = 2;
   double rmax = 0.0, rmax_old = 1609.0;
   while (rc == 0) {
@@ -1198,7 +1234,11 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
       }
     }
     int sweeps = 0;
-    if ((rc = run.run(1.0, 16, &sweeps)) != 0) break;
+    if ((rc = run.run(1.0, npre + npost, &sweeps)) != 0) break;
+    if (run.hst->result == 1) {
+      std::swap(E, E2);
+      std::swap(run.pa.buf[0], run.pa.buf[1]);
+    }
     if (launch_fold_split(p, E, nx, ny, nz, g_stream) != hipSuccess) {
       rc = fail("multigrid: fold failed");
       break;
@@ -1223,7 +1263,7 @@ extern "C" int o3d_poisson_f32(float *pp, const float *rhs, double dx, double dy
   CHK(check_grid(nx, ny, nz));
   if (!omega) return fail("omega is NULL");
   if (variant != 0 && variant != 2) return fail("SOR kernel variant %d unknown", variant);
-  if (variant == 2 && !sor_split_supported<float>(nx, ny, nz))
+  if (variant == 2 && !sor_split_supported<float>(nx))
     return fail("colour-split sweeps need nx a multiple of 8 (nx = %d)", nx);
   const size_t n = (size_t)nx * ny * nz;
   Staged s;
@@ -1824,9 +1864,14 @@ int solver_poisson_f64(Solver &S, o3d_step_info *info) {
     HIPCHK(launch_split<double>(S.P[S.cur], q, q + h, nx, ny, nz, g_stream));
     HIPCHK(launch_split<double>((const double *)S.rhs, S.rhs_split, S.rhs_split + h, nx, ny, nz,
                                 g_stream));
-    r.split = true;
-    r.sa = split_args<double>(r.a, q, q + h, S.rhs_split, S.rhs_split + h, S.dslot);
+    // P[cur] is the second buffer: its split copy is the iterate.
+    r.pair = true;
+    r.pa = pair_args<double>(r.a, q, S.P[S.cur], S.rhs_split, S.dslot);
     CHK(r.run(S.omega, first, &sweeps));
+    if (S.hst->result == 1) {
+      S.cur = 1 - S.cur;
+      q = S.P[1 - S.cur];
+    }
     HIPCHK(launch_unsplit<double>(S.P[S.cur], q, q + h, nx, ny, nz, g_stream));
   } else {
     CHK(r.run(S.omega, first, &sweeps));
@@ -1955,17 +2000,18 @@ int solver_poisson_mixed(Solver &S, o3d_step_info *info) {
     // every one that starts from a coarse-grid correction.
     if (cycles == 0 || mgc) r.a.gs = p.smooth_sweeps;
     if (split) {
-      const int h = n / 2;
-      r.split = true;
-      r.sa = split_args<float>(r.a, S.E[0], S.E[0] + h, S.R, S.R + h, S.dslot);
+      r.pair = true;
+      r.pa = pair_args<float>(r.a, S.E[0], S.E[1], S.R, S.dslot);
     }
     int sweeps = 0;
     // The first solve of a step usually takes as many sweeps as the
     // previous step's: launch that many plus the launch that sees the stop,
     // so the solve ends without a second batch or unused launches.
-    const int first = cycles == 0 && S.last_first > 0 ? std::min(kin + 1, S.last_first + 1)
-                                                      : std::min(kin, 16);
+    const int first = cycles == 0 && S.last_first > 0
+                          ? std::min(kin + 1, S.last_first + (split ? 0 : 1))
+                          : std::min(kin, 16);
     CHK(r.run(S.omega, first, &sweeps));
+    if (r.pair && S.hst->result == 1) std::swap(S.E[0], S.E[1]);
     S.sor_ms[1] += r.ms_full;
     S.sor_sweeps[1] += r.sweeps_full;
     S.sor_launches[1] += r.launches_full;
@@ -2659,8 +2705,8 @@ extern "C" int o3d_solver_create(const o3d_params *p, void **handle) {
     rc |= S->alloc(&S->E[0], n);
     rc |= S->alloc(&S->E[1], n);
     rc |= S->alloc(&S->R, n);
-    if (!rc && sor_split_supported<float>(p->nx, p->ny, p->nz))
-      rc |= S->alloc(&S->dslot, sor_split_slot_words());
+    if (!rc && sor_split_supported<float>(p->nx))
+      rc |= S->alloc(&S->dslot, sor_pair_slot_words());
     int per[3];
     solver_periodic(kind, per);
     if (!rc && per[0] && per[1] && per[2]) {
@@ -2669,8 +2715,8 @@ extern "C" int o3d_solver_create(const o3d_params *p, void **handle) {
       if (!rc) rc |= S->alloc(&S->jpart, (size_t)S->jblocks);
     }
   }
-  if (!rc && !S->mixed && sor_split_supported<double>(p->nx, p->ny, p->nz)) {
-    rc |= S->alloc(&S->dslot, sor_split_slot_words());
+  if (!rc && !S->mixed && sor_split_supported<double>(p->nx)) {
+    rc |= S->alloc(&S->dslot, sor_pair_slot_words());
     rc |= S->alloc(&S->rhs_split, n);
   }
   if (!rc && p->adaptive_extrapolation) {
@@ -2900,24 +2946,22 @@ extern "C" int o3d_solver_sor_period(void *handle, int iterations, double *us) {
   r.events = &S.ev;
   r.buf[0] = S.E[0];
   r.buf[1] = S.E[1];
-  sor_args_common<float, float>(S, r.a, S.R, S.st, iterations);
+  // Two iterations per launch, at least two launches.
+  const int launches = std::max(2, (iterations + 1) / 2);
+  sor_args_common<float, float>(S, r.a, S.R, S.st, 2 * launches);
   r.a.eps = 0.0;  // never converged, never stagnant: every launch sweeps
-  const int h = S.n / 2;
-  r.split = true;
-  r.sa = split_args<float>(r.a, S.E[0], S.E[0] + h, S.R, S.R + h, S.dslot);
-  HIPCHK(launch_sor_init(S.st, S.omega, 0, g_stream));
-  HIPCHK(launch_sor_split_init(S.dslot, g_stream));
+  r.pa = pair_args<float>(r.a, S.E[0], S.E[1], S.R, S.dslot);
+  HIPCHK(launch_sor_pair_init<float>(r.pa, S.omega, g_stream));
   hipEvent_t e0 = S.ev[0], e1 = S.ev[1];
-  for (int it = 1; it <= iterations; ++it) {
-    r.a.it = it;
-    HIPCHK(r.launch());
-    if (it == 1) HIPCHK(hipEventRecord(e0, g_stream));
+  for (; r.pa.launch < launches; ++r.pa.launch) {
+    HIPCHK(launch_sor_pair<float>(r.pa, g_stream));
+    if (r.pa.launch == 0) HIPCHK(hipEventRecord(e0, g_stream));
   }
   HIPCHK(hipEventRecord(e1, g_stream));
   HIPCHK(hipEventSynchronize(e1));
   float ms = 0.f;
   HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-  *us = 1e3 * (double)ms / (iterations - 1);
+  *us = 1e3 * (double)ms / (2 * (launches - 1));
   return 0;
 }
 

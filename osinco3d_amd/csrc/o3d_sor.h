@@ -10,6 +10,13 @@ namespace o3d {
 // decides from the state written by earlier launches whether the reference's
 // stop rule has fired (src/poisson.f90:110-114), so the host can queue many
 // launches without reading anything back.
+// What a launch of the pair kernel did: iterations it0 .. it0 + n - 1 (n = 0:
+// none yet) from buffer src into the other, with their omegas; d_prev = dmax of
+// iteration it0 - 1.
+struct SorSched {
+  int it0, n, src, pad;
+  double d_prev, om_a, om_b;
+};
 struct SorState {
   unsigned long long dmax_bits[8];  // IEEE bits of dmax of iteration it, ring by it & 7
   double omega[8];                  // omega used by iteration it, ring by it & 7
@@ -20,7 +27,8 @@ struct SorState {
   int reason;                       // 0 eps, 1 stagnation, 2 kmax
   int sweeps;                       // sweeps applied to the field
   int base;                         // iteration offset for graph-replayed batches
-  int pad;
+  int result;                       // pair kernel: buffer that holds the iterate
+  SorSched sched[2];                // pair kernel: action of the launch before launch L at L & 1
 };
 
 // The three neighbour rules of src/poisson.f90 (chosen from x and y
@@ -93,34 +101,38 @@ inline bool sor_buffer_fits(int nx, int ny, int nz) {
 }
 hipError_t launch_sor_init(SorState *st, double omega, int base, hipStream_t s);
 
-// Colour-split sweeps: the iterate and the rhs stored per row as the red
-// nodes (i + j + k even) then the black ones, each compressed to nx / 2
-// entries; an iteration is a red and a black in-place launch with the point
-// update of sor_kernel (identical iterates).  dmax partials go to dslot
-// (sor_split_slot_words() words, zeroed by launch_sor_split_init).
+// Colour-split sweeps, two iterations per launch (o3d_sor_pair.hip).  Storage:
+// per row (j, k) the red nodes (i + j + k even) in the red half array and the
+// black ones in the black half array behind it, node i at entry i >> 1 of its
+// colour's row.  Launch L = 0, 1, ... of a solve reads one of buf[0..1] and
+// writes the other; buf[0] holds the start iterate, buf[st->result] the final
+// one.  The point update and the stop decisions are sor_kernel's (identical
+// iterates).  nx even; shape, ntx, nty, ntz, zc from sor_pair_tiling.
 template <typename T>
-struct SorSplitArgs {
-  T *red, *black;                   // iterate, updated in place
-  const T *rhs_red, *rhs_black;
+struct SorPairArgs {
+  T *buf[2];
+  const T *rhs;
   SorState *st;
-  unsigned long long *dslot;
-  double *log;  // dmax per iteration (may be null), log[it-1]
-  int log_len;
+  unsigned long long *dslot;  // sor_pair_slot_words() words: dmax of the last launches
   int nx, ny, nz, per[3];
+  int shape, ntx, nty, ntz, zc;
   double ox, oy, oz, A;
   double eps, factor;
-  int kmax, idyn;
-  int it;       // iteration number of this launch pair (added to st->base)
-  int gs;       // iterations 1..gs use omega = 1 (Gauss-Seidel smoothing) and
-                // end the solve only on kmax
+  int kmax, idyn, gs;
+  int launch;
 };
-// nx a multiple of 8 (FP32) or 4 (FP64): 16-byte vectors of one colour.
+// Where the solvers use it: nx even in FP64, a multiple of 8 in FP32.
 template <typename T>
-bool sor_split_supported(int nx, int ny, int nz);
-size_t sor_split_slot_words();
-hipError_t launch_sor_split_init(unsigned long long *dslot, hipStream_t s);
+bool sor_split_supported(int nx) { return nx % (sizeof(T) == 8 ? 2 : 8) == 0; }
+size_t sor_pair_slot_words();
 template <typename T>
-hipError_t launch_sor_split_iteration(const SorSplitArgs<T> &a, hipStream_t s);
+void sor_pair_tiling(SorPairArgs<T> &a);
+template <typename T>
+hipError_t launch_sor_pair_init(const SorPairArgs<T> &a, double omega, hipStream_t s);
+template <typename T>
+hipError_t launch_sor_pair(const SorPairArgs<T> &a, hipStream_t s);
+
+// Natural <-> colour-split storage (nx even).
 template <typename T>
 hipError_t launch_split(const T *f, T *red, T *black, int nx, int ny, int nz, hipStream_t s);
 template <typename T>

@@ -477,197 +477,6 @@ __global__ void __launch_bounds__(SNT, sor_waves<T>()) sor_kernel(const SorArgs<
   }
 }
 
-// ------------------------------------------------ colour-split half sweeps
-// The FP32 correction sweeps of the mixed form keep the iterate and the rhs
-// in colour-split storage: every row (j, k) stores its red nodes
-// (i + j + k even) in the red half-array and its black nodes in the black
-// one, node i at entry i >> 1 of its colour's row (nx even).  An iteration
-// is two in-place launches, red then black; each updates one colour from the
-// other with 16-byte loads and stores, no LDS and no halo recomputation
-// (16 B/cell per iteration instead of 12, at close to streaming rates).
-// Red node (c, j, k) of row parity q = (j + k) & 1 sits at i = 2c + q; its
-// x neighbours are black entries c - 1 + q and c + q; black node c sits at
-// i = 2c + 1 - q with red x neighbours c - q and c + 1 - q; the y and z
-// neighbours of either colour are entry c of the other colour's row.
-// Each launch applies the same point update (sor_gs, then the relaxation) in
-// the same operation order as sor_kernel, so the iterates are identical.
-// dmax is reduced per block and max-accumulated into one of kSplitSlots
-// words (on separate cache lines) so that thousands of blocks do not contend
-// for one address; the next red launch reduces the slots with one wave.
-// Entries per 16-byte vector: 4 in FP32, 2 in FP64.
-template <typename T>
-constexpr int split_v() { return 16 / (int)sizeof(T); }
-constexpr int kSplitZC = 2, kSplitBX = 32, kSplitBY = 8;
-constexpr int kSplitNT = kSplitBX * kSplitBY;
-constexpr int kSplitSlots = 64, kSplitStride = 16;
-
-template <typename T>
-bool sor_split_supported(int nx, int ny, int nz) {
-  (void)ny; (void)nz;
-  return nx % (2 * split_v<T>()) == 0;
-}
-size_t sor_split_slot_words() { return (size_t)8 * kSplitSlots * kSplitStride; }
-
-__device__ __forceinline__ int sor_ghost1(int q, int n, int periodic) {
-  if (q < 0) return periodic ? q + n : -q;
-  if (q >= n) return periodic ? q - n : 2 * (n - 1) - q;
-  return q;
-}
-
-template <typename T, int COLOUR>
-__global__ void __launch_bounds__(kSplitNT) sor_split_kernel(const SorSplitArgs<T> a) {
-  constexpr int kSplitV = split_v<T>();
-  typedef T vec __attribute__((ext_vector_type(kSplitV)));
-  __shared__ double scr[kSplitNT / O3D_WAVE];
-  SorState *st = a.st;
-  if (st->done) return;
-  const int it = a.it + st->base;
-  const int tl = threadIdx.x + kSplitBX * threadIdx.y;
-  const bool first = blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0;
-  T *__restrict__ X = COLOUR == 0 ? a.red : a.black;
-  const T *__restrict__ Y = COLOUR == 0 ? a.black : a.red;
-  const T *__restrict__ RX = COLOUR == 0 ? a.rhs_red : a.rhs_black;
-  const int hx = a.nx / 2, ny = a.ny, nz = a.nz;
-  const int px = a.per[0], py = a.per[1], pz = a.per[2];
-  const int nv = hx / kSplitV;
-  const int cv = blockIdx.x * kSplitBX + threadIdx.x;
-  const int j = blockIdx.y * kSplitBY + threadIdx.y;
-  const int k0 = blockIdx.z * kSplitZC;
-  const bool active = cv < nv && j < ny;
-  // The dmax slots of the two previous iterations are loaded first and
-  // every load of the sweep right after them, so the slot reduction and the
-  // stop decision overlap the sweep's loads (the load counter completes in
-  // order); the decision only gates the stores.
-  double sl1 = 0.0, sl2 = 0.0;
-  if (COLOUR == 0) {
-    const size_t lane = __lane_id();
-    sl1 = bits_to_double(a.dslot[((size_t)((it - 1) & 7) * kSplitSlots + lane) * kSplitStride]);
-    sl2 = bits_to_double(a.dslot[((size_t)((it - 2) & 7) * kSplitSlots + lane) * kSplitStride]);
-  }
-  const int c0 = active ? cv * kSplitV : 0;
-  const int jj = active ? j : 0;
-  const size_t pl = (size_t)hx * ny;
-  const size_t rj = (size_t)hx * jj + c0;
-  const size_t rjm = (size_t)hx * sor_ghost1(jj - 1, ny, py) + c0;
-  const size_t rjp = (size_t)hx * sor_ghost1(jj + 1, ny, py) + c0;
-  // Entry beside the vector: left for s = 0, right for s = 1 (periodic
-  // wrap, or the free-slip mirror, which keeps the colour).
-  const int cl = c0 - 1 < 0 ? (px ? hx - 1 : 0) : c0 - 1;
-  const int cr = c0 + kSplitV >= hx ? (px ? 0 : hx - 1) : c0 + kSplitV;
-  vec yz[kSplitZC + 2], ym[kSplitZC], yp[kSplitZC], pc[kSplitZC], rr[kSplitZC];
-  T side[kSplitZC];
-  yz[0] = *(const vec *)(Y + rj + pl * sor_ghost1(k0 - 1, nz, pz));
-#pragma unroll
-  for (int kk = 0; kk <= kSplitZC; ++kk)
-    yz[kk + 1] = *(const vec *)(Y + rj + pl * sor_ghost1(min(k0 + kk, nz), nz, pz));
-#pragma unroll
-  for (int kk = 0; kk < kSplitZC; ++kk) {
-    const int k = min(k0 + kk, nz - 1);  // planes past the end are not stored
-    const int sd = COLOUR == 0 ? ((jj + k) & 1) : 1 - ((jj + k) & 1);
-    const size_t pk = pl * k;
-    side[kk] = Y[pk + (rj - c0) + (sd == 0 ? cl : cr)];
-    ym[kk] = *(const vec *)(Y + rjm + pk);
-    yp[kk] = *(const vec *)(Y + rjp + pk);
-    pc[kk] = *(const vec *)(X + rj + pk);
-    rr[kk] = *(const vec *)(RX + rj + pk);
-  }
-  double om;
-  bool done = false;
-  if (COLOUR == 0) {
-    double dlast;
-    int reason;
-    done = sor_decide_with(st, it, a.eps, a.factor, a.kmax, a.idyn, om, reason, dlast,
-                           [&](int q) { return wave_max(q == it - 1 ? sl1 : sl2); });
-    // No eps or stagnation exit inside the Gauss-Seidel opening: its small
-    // updates say little about the smooth error that remains.
-    if (done && reason != 2 && it - 1 <= a.gs) done = false;
-    if (first && done && tl == 0) {
-      st->done = 1;
-      st->reason = reason;
-      st->exit_iter = reason == 2 ? a.kmax + 1 : it - 1;
-      st->sweeps = it - 1;
-      st->dmax_final = dlast;
-      st->omega_final = om;
-      if (a.log && it - 2 < a.log_len) a.log[it - 2] = dlast;
-    }
-    if (first && !done) {
-      if (tl < kSplitSlots)
-        a.dslot[((size_t)((it + 1) & 7) * kSplitSlots + tl) * kSplitStride] = 0ull;
-      if (tl == 0) {
-        st->omega[it & 7] = om;
-        if (a.log && it >= 2 && it - 2 < a.log_len) a.log[it - 2] = dlast;
-      }
-    }
-  } else {
-    om = st->omega[it & 7];
-  }
-  if (done) return;
-  const T ox = T(a.ox), oy = T(a.oy), oz = T(a.oz), A = T(a.A);
-  const T invA = T(1.0 / a.A);
-  // The first a.gs iterations are Gauss-Seidel sweeps (omega = 1); the
-  // omega ring keeps the solve's omega.
-  const double omu = it <= a.gs ? 1.0 : om;
-  const T w = T(omu), w1 = T(1.0 - omu);
-  T dmax = T(0);
-  if (active) {
-#pragma unroll
-    for (int kk = 0; kk < kSplitZC; ++kk) {
-      const int k = k0 + kk;
-      if (k < nz) {
-        const int sd = COLOUR == 0 ? ((j + k) & 1) : 1 - ((j + k) & 1);
-        const vec zm = yz[kk], zc = yz[kk + 1], zp = yz[kk + 2];
-        vec out;
-#pragma unroll
-        for (int v = 0; v < kSplitV; ++v) {
-          const T xm = sd == 0 ? (v == 0 ? side[kk] : zc[v - 1]) : zc[v];
-          const T xp = sd == 0 ? zc[v] : (v == kSplitV - 1 ? side[kk] : zc[v + 1]);
-          const T pn = sor_gs<T, T>(xm, xp, ym[kk][v], yp[kk][v], zm[v], zp[v], rr[kk][v], ox,
-                                    oy, oz, A, invA);
-          out[v] = w1 * pc[kk][v] + w * pn;
-          const T d = T(fabs(pn - pc[kk][v]));
-          dmax = d > dmax ? d : dmax;
-        }
-        *(vec *)(X + rj + pl * k) = out;
-      }
-    }
-  }
-  double dm = wave_max((double)dmax);
-  if (tl % O3D_WAVE == 0) scr[tl / O3D_WAVE] = dm;
-  __syncthreads();
-  dm = scr[0];
-#pragma unroll
-  for (int q = 1; q < kSplitNT / O3D_WAVE; ++q) dm = fmax(dm, scr[q]);
-  if (tl == 0 && dm != 0.0) {
-    const int b = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    atomicMax(&a.dslot[((size_t)(it & 7) * kSplitSlots + (b % kSplitSlots)) * kSplitStride],
-              (unsigned long long)__double_as_longlong(dm));
-  }
-}
-
-__global__ void sor_split_init_kernel(unsigned long long *dslot, int words) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < words) dslot[i] = 0ull;
-}
-
-hipError_t launch_sor_split_init(unsigned long long *dslot, hipStream_t s) {
-  const int words = (int)sor_split_slot_words();
-  sor_split_init_kernel<<<(words + 255) / 256, 256, 0, s>>>(dslot, words);
-  return hipGetLastError();
-}
-
-template <typename T>
-hipError_t launch_sor_split_iteration(const SorSplitArgs<T> &a, hipStream_t s) {
-  if (!sor_split_supported<T>(a.nx, a.ny, a.nz))
-    return hipErrorInvalidValue;
-  const int nv = a.nx / 2 / split_v<T>();
-  const dim3 grd((nv + kSplitBX - 1) / kSplitBX, (a.ny + kSplitBY - 1) / kSplitBY,
-                 (a.nz + kSplitZC - 1) / kSplitZC);
-  const dim3 blk(kSplitBX, kSplitBY);
-  sor_split_kernel<T, 0><<<grd, blk, 0, s>>>(a);
-  sor_split_kernel<T, 1><<<grd, blk, 0, s>>>(a);
-  return hipGetLastError();
-}
-
 // Natural <-> colour-split storage (nx even).
 __device__ __forceinline__ size_t split_entry(int idx, int nx, int ny, bool &black) {
   const int i = idx % nx, r = idx / nx;  // r = j + ny * k
@@ -714,11 +523,6 @@ hipError_t launch_unsplit(T *f, const T *red, const T *black, int nx, int ny, in
   return hipGetLastError();
 }
 
-template bool sor_split_supported<float>(int, int, int);
-template bool sor_split_supported<double>(int, int, int);
-template hipError_t launch_sor_split_iteration<float>(const SorSplitArgs<float> &, hipStream_t);
-template hipError_t launch_sor_split_iteration<double>(const SorSplitArgs<double> &,
-                                                       hipStream_t);
 template hipError_t launch_split<float>(const float *, float *, float *, int, int, int,
                                         hipStream_t);
 template hipError_t launch_split<double>(const double *, double *, double *, int, int, int,

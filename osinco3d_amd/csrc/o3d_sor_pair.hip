@@ -1,0 +1,588 @@
+// Red-black SOR, two iterations per launch (MI355X).
+//
+// The iterate and the rhs are in colour-split storage (o3d_sor.h): entry c of a
+// row's two halves is the pair of nodes (2c, 2c + 1).  A launch reads one
+// buffer and writes the other, so two iterations read the iterate and the rhs
+// once and write the iterate once; a launch per colour, updating it in place,
+// reads three of the four half arrays and writes one four times over.
+//
+// A block owns a tile of pairs x rows and a chunk of planes and computes the
+// four half sweeps (red, black, red, black) on the tile plus a halo that
+// loses one node per half sweep: 4 nodes in x and y, 4 planes below, 3 above.
+// It marches in z: step t runs red on plane t, black on t - 1, red on t - 2
+// and black on t - 3, each from the planes the previous half sweep has just
+// left, so a plane lives for 8 steps in registers and meets memory twice.  A
+// thread keeps its column of pairs on RY rows: z neighbours are its own
+// registers, the x neighbour beside the pair comes from the next lane by DPP,
+// and only the first and last row of each thread's RY pass through LDS (one
+// barrier per step).  Ghost nodes (periodic images, mirror images) load from
+// their image and evolve exactly as it does, so no boundary case is left in
+// the march.  Every half sweep is the point update of sor_kernel in its
+// operation order: the iterates are identical.
+//
+// The stop rule looks at dmax after every iteration, so the second iteration
+// of a pair is a guess that the first does not end the solve or change omega.
+// The next launch checks it; when it was wrong the source buffer still holds
+// the iterate before the pair, and that launch runs the first iteration (or
+// the pair with the right omegas) again.
+//
+// What bounds it: about 0.95 us per plane step however many blocks run (the
+// dependent chain of four point updates, LDS and barrier), and in large grids
+// the traffic of the halos, which neighbouring tiles find in their XCD's L2
+// only while they march side by side.  So tiles are handed to the XCDs in
+// contiguous runs (FP32 256^3: 90 us per launch in the plain order, 54 us so),
+// one block runs per CU (FP64 256^3: 105 us with one block of 384 threads per
+// CU, 131 us with two; 512 and 768 threads 128 and 125 us), and loads are
+// issued two planes ahead (three: no gain).  Per two iterations, launches of
+// one colour in place / this kernel: FP64 64^3 27.1 / 16.9 us, 128^3 36.7 /
+// 27.9, 256^3 186 / 108, 512x384x256 696 / 305; FP32 64^3 27.2 / 15.8, 256^3
+// 98 / 54, 384x256x128 93 / 40, 512x384x256 327 / 174 (the figures hold the
+// host's share of a batch of launches, about 3 us).
+#include <algorithm>
+#include <utility>
+
+#include "o3d_sor.h"
+
+namespace o3d {
+
+namespace {
+
+// Lanes (pairs) per row, rows per thread, threads per block and LDS asked for
+// beyond what the block uses (it sets how many blocks share a CU).
+template <typename T, int SHAPE>
+struct PairShape;
+template <>
+struct PairShape<double, 0> {
+  static constexpr int LX = 32, RY = 2, NT = 384, PAD = 40000;
+};
+template <>
+struct PairShape<float, 0> {
+  static constexpr int LX = 32, RY = 2, NT = 768, PAD = 0;
+};
+template <>
+struct PairShape<float, 1> {
+  static constexpr int LX = 64, RY = 4, NT = 512, PAD = 0;
+};
+
+constexpr int kPairRing = 8;  // planes t - 4 .. t + 2 and the one being loaded
+constexpr int kPairSlots = 64, kPairStride = 16;  // dmax words per iteration
+constexpr int kPairSets = 4;                      // launches in the dmax ring
+
+template <int K>
+struct PIC { static constexpr int value = K; };
+
+// Image of node q of an axis of n nodes for q in [-4, n + 4] (n >= 6);
+// positions further out belong to idle rows and lanes of a partial tile.
+__device__ __forceinline__ int pair_ghost(int q, int n, int periodic) {
+  if (q > n + 4) return n - 1;
+  if (periodic) return q < 0 ? q + n : (q >= n ? q - n : q);
+  return q < 0 ? -q : (q > n - 1 ? 2 * (n - 1) - q : q);
+}
+
+// xcd_tile for any number of blocks: block b runs on XCD b % 8, and each XCD
+// gets one contiguous run of tiles (the grids here are seldom a multiple of 8,
+// and the tiles' halos are half of what they load).
+__device__ __forceinline__ int pair_tile(int b, int nb) {
+  const int x = b & 7, q = nb >> 3, r = nb & 7;
+  return x * q + min(x, r) + (b >> 3);
+}
+
+// The value of the lane before (DIR = 0) or after (DIR = 1) this one.
+template <int DIR>
+__device__ __forceinline__ float lane_next(float v) {
+  constexpr int ctrl = DIR == 0 ? 0x138 : 0x130;  // wave_shr:1, wave_shl:1
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, true));
+}
+template <int DIR>
+__device__ __forceinline__ double lane_next(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  constexpr int ctrl = DIR == 0 ? 0x138 : 0x130;
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, ctrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), ctrl, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
+                                          (unsigned)lo));
+}
+
+// num / A.  FP64 divides as the reference does: the correction step of a
+// correctly rounded division from the reciprocal invA (quotient, exact
+// remainder by fma, corrected quotient), the last part of what the compiler
+// emits for num / A, whose refinement of 1 / A per node is left out; zero,
+// infinite and NaN numerators by div_fixup.  FP32 multiplies by 1 / A.
+__device__ __forceinline__ double pair_div(double num, double A, double invA) {
+  const double q = num * invA;
+  const double r = __builtin_fma(-q, A, num);
+  return __builtin_amdgcn_div_fixup(__builtin_fma(r, invA, q), A, num);
+}
+__device__ __forceinline__ float pair_div(float num, float, float invA) { return num * invA; }
+
+template <typename T>
+__device__ __forceinline__ T pload(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff) {
+  if constexpr (sizeof(T) == 8)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
+}
+
+template <typename T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pair_rsrc(const T *p, int n) {
+  // At most INT_MAX bytes (sor_buffer_fits, checked by the launcher).
+  return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0,
+                                           (int)((long long)n * (long long)sizeof(T)), 0x00020000);
+}
+
+// What one launch does: iterations it0 .. it0 + n - 1 from buffer src.
+struct PairStep {
+  bool done;       // the solve is over: the launch does nothing
+  int it0, n, src;
+  double d_prev, om_a, om_b;
+  // When done.
+  int reason, sweeps, result;
+  double dlast, omega;
+};
+
+// The reference's loop tail after iteration q with update d1 (the one before
+// it d0): true when the solve ends; om becomes omega of iteration q + 1.
+// Same rules and order as sor_decide_with of the single-iteration kernels.
+__device__ __forceinline__ bool pair_tail(int q, double d1, double d0, double eps,
+                                          double factor, int kmax, int idyn, int gs, double &om,
+                                          int &reason) {
+  reason = -1;
+  if (d1 < eps) reason = 0;
+  else if (fabs(d0 - d1) < eps / 1000.0) reason = 1;
+  // No eps or stagnation exit inside the Gauss-Seidel opening.
+  if (reason >= 0) return q > gs;
+  if (q > 1 && idyn == 1) {
+    if (d1 > d0) om = om * (2.0 - factor);
+    else if (d1 < 0.1 * d0) om = fmin(om * factor, 2.0);
+  }
+  if (q + 1 > kmax) { reason = 2; return true; }
+  return false;
+}
+
+// The next action from the previous launch's (P) and its two dmax values.
+template <typename T>
+__device__ __forceinline__ PairStep pair_decide(const SorSched &P, double da, double db,
+                                                const SorPairArgs<T> &a) {
+  PairStep s{};
+  s.src = P.src;
+  s.it0 = P.it0;
+  s.om_a = P.om_a;
+  s.d_prev = P.d_prev;
+  if (P.n > 0) {
+    double om = P.om_a;
+    int reason;
+    const bool stop = pair_tail(P.it0, da, P.it0 == 1 ? 1609.0 : P.d_prev, a.eps, a.factor,
+                                a.kmax, a.idyn, a.gs, om, reason);
+    if (stop && P.n == 2) {  // one iteration too many: the first alone
+      s.n = 1;
+      s.om_b = s.om_a;
+      return s;
+    }
+    if (!stop && P.n == 2 && om != P.om_b) {  // the pair with its own omegas
+      s.n = 2;
+      s.om_b = om;
+      return s;
+    }
+    int q = P.it0;
+    double d = da;
+    bool end = stop;
+    if (!stop && P.n == 2) {
+      ++q;
+      d = db;
+      end = pair_tail(q, db, da, a.eps, a.factor, a.kmax, a.idyn, a.gs, om, reason);
+    }
+    s.src = 1 - P.src;
+    if (end) {
+      s.done = true;
+      s.reason = reason;
+      s.sweeps = q;
+      s.result = s.src;
+      s.dlast = d;
+      s.omega = om;
+      return s;
+    }
+    s.it0 = q + 1;
+    s.om_a = om;
+    s.d_prev = d;
+  }
+  s.om_b = s.om_a;
+  s.n = s.it0 + 1 <= a.kmax ? 2 : 1;
+  return s;
+}
+
+template <typename T, int... K, typename F>
+__device__ __forceinline__ bool pair_group(std::integer_sequence<int, K...>, int m, int last,
+                                           F &&f) {
+  return ((m + K <= last && (f(m + K, PIC<K>{}), true)) && ...);
+}
+
+template <typename T, int SHAPE>
+__global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
+    sor_pair_kernel(const SorPairArgs<T> a) {
+  using Shape = PairShape<T, SHAPE>;
+  constexpr int LX = Shape::LX, RY = Shape::RY, NT = Shape::NT;
+  constexpr int NG = NT / LX, TY = NG * RY, NR = kPairRing;
+  static_assert(RY % 2 == 0 && TY % 2 == 0, "row parities are compile-time constants");
+  // First and last row of every thread's RY: old black, new red, new black,
+  // second red of the planes the next step reads; [0] the last rows, [1] the
+  // first ones.  One guard group on each side.
+  __shared__ T ex[2][4][2][NG + 2][LX];
+  __shared__ double scr[2][NT / O3D_WAVE];
+  const int tid = threadIdx.x;
+  const int lane = tid % LX, g = tid / LX;
+  SorState *st = a.st;
+  const int over = st->done;
+  const SorSched P = st->sched[a.launch & 1];
+  const unsigned long long *ds =
+      a.dslot + (size_t)((a.launch + kPairSets - 1) % kPairSets) * 2 * kPairSlots * kPairStride;
+  const size_t wl = (size_t)__lane_id() * kPairStride;
+  const unsigned long long dwa = ds[wl], dwb = ds[(size_t)kPairSlots * kPairStride + wl];
+
+  const int nx = a.nx, ny = a.ny, nz = a.nz, hx = nx / 2;
+  const int tile = pair_tile(blockIdx.x, gridDim.x);
+  const int tix = tile % a.ntx, rr = tile / a.ntx;
+  const int tiy = rr % a.nty, tiz = rr / a.nty;
+  const int c0 = tix * (LX - 4), y0 = tiy * (TY - 8), z0 = tiz * a.zc;
+  const int z1 = min(z0 + a.zc, nz);
+  const T ox = T(a.ox), oy = T(a.oy), oz = T(a.oz), A = T(a.A), invA = T(1.0 / a.A);
+
+  // Entries of the left and right node of this thread's pair, per row (they
+  // differ only for mirror images, whose two nodes lie in two pairs).
+  const int c = c0 - 2 + lane;
+  const int eL = pair_ghost(2 * c, nx, a.per[0]) >> 1;
+  const int eR = pair_ghost(2 * c + 1, nx, a.per[0]) >> 1;
+  const int jb = y0 - 4 + g * RY;
+  unsigned vL[RY], vR[RY];
+  bool own[RY];
+#pragma unroll
+  for (int r = 0; r < RY; ++r) {
+    const int row = hx * pair_ghost(jb + r, ny, a.per[1]);
+    vL[r] = (unsigned)(row + eL) * (unsigned)sizeof(T);
+    vR[r] = (unsigned)(row + eR) * (unsigned)sizeof(T);
+    const int lr = g * RY + r;
+    own[r] = lane >= 2 && lane < LX - 2 && c < hx && lr >= 4 && lr < TY - 4 && jb + r < ny;
+  }
+  const int n = nx * ny * nz;
+  const unsigned planeB = (unsigned)(hx * ny) * (unsigned)sizeof(T);
+  const unsigned halfB = planeB * (unsigned)nz;
+  // The source buffer as long as no pair was taken back; the first loads go
+  // out before the decision that may change it.
+  int src = a.launch & 1;
+  __amdgpu_buffer_rsrc_t rin = pair_rsrc(a.buf[src], n);
+  const __amdgpu_buffer_rsrc_t rrh = pair_rsrc(a.rhs, n);
+
+  // Ring slot of plane z0 - 4 + q is q & 7; z0 and the tile's first row are
+  // even, so the parity of row + plane is (r + q) & 1.
+  T R[NR][RY], B[NR][RY], fR[NR][RY], fB[NR][RY];
+#pragma unroll
+  for (int q = 0; q < NR; ++q)
+#pragma unroll
+    for (int r = 0; r < RY; ++r) R[q][r] = B[q][r] = fR[q][r] = fB[q][r] = T(0);
+  // Byte offset of plane z0 - 4 + q (at most nz + 4; the image as in
+  // pair_ghost, without branches).
+  const int zs = a.per[2] ? 1 : -1, zlo = a.per[2] ? nz : 0, zhi = a.per[2] ? -nz : 2 * (nz - 1);
+  auto zsoff = [&](int q) {
+    const int z = z0 - 4 + q, im = zs * z + (z < 0 ? zlo : zhi);
+    return planeB * (unsigned)(z < 0 || z >= nz ? im : z);
+  };
+  auto load_p = [&](int q, auto SL) {
+    constexpr int sl = decltype(SL)::value & 7;
+    const unsigned so = zsoff(q);
+#pragma unroll
+    for (int r = 0; r < RY; ++r) {
+      const bool odd = (r + sl) & 1;
+      R[sl][r] = pload<T>(rin, odd ? vR[r] : vL[r], so);
+      B[sl][r] = pload<T>(rin, odd ? vL[r] : vR[r], so + halfB);
+    }
+  };
+  auto load_f = [&](int q, auto SL) {
+    constexpr int sl = decltype(SL)::value & 7;
+    const unsigned so = zsoff(q);
+#pragma unroll
+    for (int r = 0; r < RY; ++r) {
+      const bool odd = (r + sl) & 1;
+      fR[sl][r] = pload<T>(rrh, odd ? vR[r] : vL[r], so);
+      fB[sl][r] = pload<T>(rrh, odd ? vL[r] : vR[r], so + halfB);
+    }
+  };
+  T dA[RY], dB[RY];
+#pragma unroll
+  for (int r = 0; r < RY; ++r) dA[r] = dB[r] = T(0);
+
+  // One half sweep of plane slot sl: X (this colour) from Y (the other), with
+  // the rows beside the thread's own from LDS; cnt: this plane counts for dmax.
+  auto half = [&](auto SL, auto COL, T(&X)[NR][RY], T(&Y)[NR][RY], const T(&F)[NR][RY], T lo,
+                  T hi, T w, T w1, bool cnt, T(&dm)[RY]) {
+    constexpr int sl = decltype(SL)::value & 7, sm = (sl + 7) & 7, sp = (sl + 1) & 7;
+    constexpr int col = decltype(COL)::value;
+    T d[RY];
+#pragma unroll
+    for (int r = 0; r < RY; ++r) {
+      // Node on the left of its pair: its other x neighbour is in the pair
+      // before; on the right: in the pair after.
+      const bool right = ((r + sl + col) & 1) != 0;
+      const T side = right ? lane_next<1>(Y[sl][r]) : lane_next<0>(Y[sl][r]);
+      const T ym = r == 0 ? lo : Y[sl][r == 0 ? 0 : r - 1];
+      const T yp = r == RY - 1 ? hi : Y[sl][r == RY - 1 ? r : r + 1];
+      const T num = -ox * (side + Y[sl][r]) - oy * (ym + yp) - oz * (Y[sm][r] + Y[sp][r]) +
+                    F[sl][r];
+      const T pn = pair_div(num, A, invA);
+      d[r] = pn - X[sl][r];
+      X[sl][r] = w1 * X[sl][r] + w * pn;
+    }
+    if (cnt) {
+#pragma unroll
+      for (int r = 0; r < RY; ++r) dm[r] = T(__builtin_fmax(T(__builtin_fabs(d[r])), dm[r]));
+    }
+  };
+  // First and last rows of the four planes the step after step m reads.
+  auto publish = [&](int b, auto K) {
+    constexpr int k = decltype(K)::value;
+    constexpr int s0 = (k + 2) & 7, s1 = (k + 1) & 7, s2 = k & 7, s3 = (k + 7) & 7;
+    ex[b][0][0][g + 1][lane] = B[s0][RY - 1];
+    ex[b][0][1][g + 1][lane] = B[s0][0];
+    ex[b][1][0][g + 1][lane] = R[s1][RY - 1];
+    ex[b][1][1][g + 1][lane] = R[s1][0];
+    ex[b][2][0][g + 1][lane] = B[s2][RY - 1];
+    ex[b][2][1][g + 1][lane] = B[s2][0];
+    ex[b][3][0][g + 1][lane] = R[s3][RY - 1];
+    ex[b][3][1][g + 1][lane] = R[s3][0];
+  };
+
+  // The guard groups feed rows outside the tile's valid region only; they
+  // hold zeros.
+  for (int q = tid; q < 2 * 4 * 2 * 2 * LX; q += NT) {
+    const int l = q % LX, e = q / LX;
+    ex[e & 1][(e >> 1) & 3][(e >> 3) & 1][(e >> 4) ? NG + 1 : 0][l] = T(0);
+  }
+  load_p(0, PIC<0>{});
+  load_p(1, PIC<1>{});
+  load_f(1, PIC<1>{});
+  load_p(2, PIC<2>{});
+
+  if (over) return;
+  PairStep s = pair_decide(P, wave_max(__longlong_as_double((long long)dwa)),
+                           wave_max(__longlong_as_double((long long)dwb)), a);
+  // Equal in every lane; in scalar registers, as the buffer descriptors and
+  // the branches of the march need them.
+  s.done = __builtin_amdgcn_readfirstlane((int)s.done) != 0;
+  s.n = __builtin_amdgcn_readfirstlane(s.n);
+  s.src = __builtin_amdgcn_readfirstlane(s.src);
+  if (blockIdx.x == 0) {
+    if (s.done) {
+      if (tid == 0) {
+        st->done = 1;
+        st->reason = s.reason;
+        st->exit_iter = s.reason == 2 ? a.kmax + 1 : s.sweeps;
+        st->sweeps = s.sweeps;
+        st->result = s.result;
+        st->dmax_final = s.dlast;
+        st->omega_final = s.omega;
+      }
+    } else {
+      if (tid == 0) {
+        st->sched[(a.launch + 1) & 1] = {s.it0, s.n, s.src, 0, s.d_prev, s.om_a, s.om_b};
+        st->sweeps = s.it0 + s.n - 1;
+      }
+      unsigned long long *nx_ds =
+          a.dslot + (size_t)((a.launch + 1) % kPairSets) * 2 * kPairSlots * kPairStride;
+      for (int q = tid; q < 2 * kPairSlots; q += NT) nx_ds[(size_t)q * kPairStride] = 0ull;
+    }
+  }
+  if (s.done) return;
+  if (s.src != src) {
+    src = s.src;
+    rin = pair_rsrc(a.buf[src], n);
+    load_p(0, PIC<0>{});
+    load_p(1, PIC<1>{});
+    load_p(2, PIC<2>{});
+  }
+  const __amdgpu_buffer_rsrc_t rout = pair_rsrc(a.buf[1 - src], n);
+  const double oma = s.it0 <= a.gs ? 1.0 : s.om_a, omb = s.it0 + 1 <= a.gs ? 1.0 : s.om_b;
+  const T wa = T(oma), wa1 = T(1.0 - oma), wb = T(omb), wb1 = T(1.0 - omb);
+  const bool two = s.n == 2;
+  publish(0, PIC<7>{});  // before step 0: its red reads plane slot 1's black
+  __syncthreads();
+
+  // Step m: t = z0 - 3 + m, slot of plane t is (m + 1) & 7.
+  const int last = z1 - z0 + 5;
+  auto step = [&](int m, auto K) {
+    constexpr int k = decltype(K)::value;
+    load_p(m + 3, PIC<k + 3>{});
+    load_f(m + 2, PIC<k + 2>{});
+    const int b = m & 1;
+    T lo[4], hi[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      lo[q] = ex[b][q][0][g][lane];
+      hi[q] = ex[b][q][1][g + 2][lane];
+    }
+    const int t = z0 - 3 + m;
+    half(PIC<k + 1>{}, PIC<0>{}, R, B, fR, lo[0], hi[0], wa, wa1, t >= z0 && t < z1, dA);
+    half(PIC<k>{}, PIC<1>{}, B, R, fB, lo[1], hi[1], wa, wa1, t - 1 >= z0 && t - 1 < z1, dA);
+    if (two) {
+      half(PIC<k + 7>{}, PIC<0>{}, R, B, fR, lo[2], hi[2], wb, wb1, t - 2 >= z0 && t - 2 < z1,
+           dB);
+      half(PIC<k + 6>{}, PIC<1>{}, B, R, fB, lo[3], hi[3], wb, wb1, t - 3 >= z0, dB);
+    }
+    publish(1 - b, K);
+    if (t - 3 >= z0) {
+      constexpr int sl = (k + 6) & 7;
+      const unsigned so = planeB * (unsigned)(t - 3);
+#pragma unroll
+      for (int r = 0; r < RY; ++r)
+        if (own[r]) {
+          if constexpr (sizeof(T) == 8) {
+            typedef unsigned u2 __attribute__((ext_vector_type(2)));
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, R[sl][r]), rout, vL[r],
+                                                  so, 0);
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, B[sl][r]), rout, vL[r],
+                                                  so + halfB, 0);
+          } else {
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, R[sl][r]), rout,
+                                                  vL[r], so, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, B[sl][r]), rout,
+                                                  vL[r], so + halfB, 0);
+          }
+        }
+    }
+    __syncthreads();
+  };
+  for (int m = 0; pair_group<T>(std::make_integer_sequence<int, 8>{}, m, last, step); m += 8) {
+  }
+
+  T ma = T(0), mb = T(0);
+#pragma unroll
+  for (int r = 0; r < RY; ++r)
+    if (own[r]) {
+      ma = dA[r] > ma ? dA[r] : ma;
+      mb = dB[r] > mb ? dB[r] : mb;
+    }
+  const double va = wave_max((double)ma), vb = wave_max((double)mb);
+  if (tid % O3D_WAVE == 0) {
+    scr[0][tid / O3D_WAVE] = va;
+    scr[1][tid / O3D_WAVE] = vb;
+  }
+  __syncthreads();
+  if (tid < 2) {
+    double v = scr[tid][0];
+#pragma unroll
+    for (int q = 1; q < NT / O3D_WAVE; ++q) v = fmax(v, scr[tid][q]);
+    if (v != 0.0)
+      atomicMax(&a.dslot[((size_t)(a.launch % kPairSets) * 2 * kPairSlots +
+                          (size_t)tid * kPairSlots + blockIdx.x % kPairSlots) * kPairStride],
+                (unsigned long long)__double_as_longlong(v));
+  }
+}
+
+__global__ void __launch_bounds__(256) sor_pair_init_kernel(SorState *st, double omega,
+                                                            unsigned long long *dslot,
+                                                            int words) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < words) dslot[i] = 0ull;
+  if (i == 0) {
+    st->omega_final = omega;
+    st->dmax_final = 0.0;
+    st->done = 0;
+    st->exit_iter = 0;
+    st->reason = -1;
+    st->sweeps = 0;
+    st->result = 0;
+    st->sched[0] = {1, 0, 0, 0, 1609.0, omega, omega};
+  }
+}
+
+// Concurrent blocks of the kernel on this device.
+template <typename T, int SHAPE>
+int pair_slots() {
+  static const int slots = [] {
+    int per_cu = 0, dev = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &per_cu, sor_pair_kernel<T, SHAPE>, PairShape<T, SHAPE>::NT,
+            PairShape<T, SHAPE>::PAD) != hipSuccess ||
+        hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+      (void)hipGetLastError();
+      return 256;
+    }
+    return std::max(1, per_cu * cus);
+  }();
+  return slots;
+}
+
+// Tiles of one shape: the even chunk of planes with the least
+// rounds * (planes + 6 of the pipeline + 3 of prologue).
+template <typename T, int SHAPE>
+void pair_tiling(SorPairArgs<T> &a) {
+  using Shape = PairShape<T, SHAPE>;
+  constexpr int OX = Shape::LX - 4, OY = Shape::NT / Shape::LX * Shape::RY - 8;
+  a.shape = SHAPE;
+  a.ntx = (a.nx / 2 + OX - 1) / OX;
+  a.nty = (a.ny + OY - 1) / OY;
+  const long long layer = (long long)a.ntx * a.nty;
+  const int slots = pair_slots<T, SHAPE>();
+  double best = 1e300;
+  for (int zc = 2; zc < a.nz + 2; zc += 2) {
+    const int ntz = (a.nz + zc - 1) / zc;
+    const long long rounds = (layer * ntz + slots - 1) / slots;
+    const double cost = (double)rounds * (zc + 9.0);
+    if (cost < best - 1e-9) {
+      best = cost;
+      a.zc = zc;
+      a.ntz = ntz;
+    }
+  }
+}
+
+template <typename T, int SHAPE>
+void pair_launch(const SorPairArgs<T> &a, hipStream_t s) {
+  using Shape = PairShape<T, SHAPE>;
+  sor_pair_kernel<T, SHAPE><<<a.ntx * a.nty * a.ntz, Shape::NT, Shape::PAD, s>>>(a);
+}
+
+}  // namespace
+
+size_t sor_pair_slot_words() { return (size_t)kPairSets * 2 * kPairSlots * kPairStride; }
+
+template <>
+void sor_pair_tiling<double>(SorPairArgs<double> &a) { pair_tiling<double, 0>(a); }
+// FP32: the narrow tile while both buffers and the rhs stay in the 256 MB of
+// the Infinity Cache, the wide one (longer rows, fewer x halos) beyond.  Per
+// launch, narrow / wide: 192^3 31.5 / 32.3 us, 256^3 53.8 / 64.4, 384x256x128
+// 39.8 / 49.5, then 288^3 96.9 / 87.1, 320^3 114 / 107, 512x384x256 219 / 174.
+template <>
+void sor_pair_tiling<float>(SorPairArgs<float> &a) {
+  const long long bytes = 12ll * a.nx * a.ny * a.nz;
+  if (bytes > (256ll << 20)) pair_tiling<float, 1>(a);
+  else pair_tiling<float, 0>(a);
+}
+
+template <typename T>
+hipError_t launch_sor_pair_init(const SorPairArgs<T> &a, double omega, hipStream_t s) {
+  const int words = (int)sor_pair_slot_words();
+  sor_pair_init_kernel<<<(words + 255) / 256, 256, 0, s>>>(a.st, omega, a.dslot, words);
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_sor_pair(const SorPairArgs<T> &a, hipStream_t s) {
+  if (a.nx % 2 != 0 || a.nx < 6 || a.ny < 6 || a.nz < 6 ||
+      a.zc % 2 != 0 || !sor_buffer_fits<T, T>(a.nx, a.ny, a.nz))
+    return hipErrorInvalidValue;
+  if constexpr (sizeof(T) == 4) {
+    if (a.shape == 1) pair_launch<T, 1>(a, s);
+    else pair_launch<T, 0>(a, s);
+  } else {
+    pair_launch<T, 0>(a, s);
+  }
+  return hipGetLastError();
+}
+
+template hipError_t launch_sor_pair_init<float>(const SorPairArgs<float> &, double, hipStream_t);
+template hipError_t launch_sor_pair_init<double>(const SorPairArgs<double> &, double,
+                                                 hipStream_t);
+template hipError_t launch_sor_pair<float>(const SorPairArgs<float> &, hipStream_t);
+template hipError_t launch_sor_pair<double>(const SorPairArgs<double> &, hipStream_t);
+
+}  // namespace o3d
