@@ -26,17 +26,20 @@
 // the iterate before the pair, and that launch runs the first iteration (or
 // the pair with the right omegas) again.
 //
-// What bounds it: about 0.95 us per plane step however many blocks run (the
-// dependent chain of four point updates, LDS and barrier), and in large grids
-// the traffic of the halos, which neighbouring tiles find in their XCD's L2
-// only while they march side by side.  So tiles are handed to the XCDs in
+// What bounds it: small grids by the plane step, 0.85 us (0.95 us with the
+// tests of the first steps as branches inside the march, which kept the
+// compiler from interleaving the half sweeps: 64^3 16.7 -> 15.2 us a launch);
+// large ones by memory, at 4.3 TB/s of the traffic that reaches the fabric (the
+// same kernel without its arithmetic takes as long), and there by the halos,
+// which neighbouring tiles find in their XCD's L2 only while they march side by
+// side.  So tiles are handed to the XCDs in
 // contiguous runs (FP32 256^3: 90 us per launch in the plain order, 54 us so),
 // one block runs per CU (FP64 256^3: 105 us with one block of 384 threads per
 // CU, 131 us with two; 512 and 768 threads 128 and 125 us), and loads are
 // issued two planes ahead (three: no gain).  Per two iterations, launches of
-// one colour in place / this kernel: FP64 64^3 27.1 / 16.9 us, 128^3 36.7 /
-// 27.9, 256^3 186 / 108, 512x384x256 696 / 305; FP32 64^3 27.2 / 15.8, 256^3
-// 98 / 54, 384x256x128 93 / 40, 512x384x256 327 / 174 (the figures hold the
+// one colour in place / this kernel: FP64 64^3 27.1 / 15.2 us, 128^3 36.7 /
+// 26.0, 256^3 186 / 107, 512x384x256 696 / 310; FP32 64^3 27.2 / 14.5, 256^3
+// 98 / 54, 384x256x128 93 / 38, 512x384x256 327 / 174 (the figures hold the
 // host's share of a batch of launches, about 3 us).
 #include <algorithm>
 #include <utility>
@@ -102,6 +105,19 @@ __device__ __forceinline__ double lane_next(double v) {
   const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), ctrl, 0xf, 0xf, true);
   return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
                                           (unsigned)lo));
+}
+
+// max(m, |d|), m for a NaN d, as one instruction (fmax would first
+// canonicalise its operands).
+__device__ __forceinline__ float max_abs(float m, float d) {
+  float r;
+  asm("v_max_f32 %0, %1, |%2|" : "=v"(r) : "v"(m), "v"(d));
+  return r;
+}
+__device__ __forceinline__ double max_abs(double m, double d) {
+  double r;
+  asm("v_max_f64 %0, %1, |%2|" : "=v"(r) : "v"(m), "v"(d));
+  return r;
 }
 
 // num / A.  FP64 divides as the reference does: the correction step of a
@@ -211,7 +227,7 @@ __device__ __forceinline__ PairStep pair_decide(const SorSched &P, double da, do
   return s;
 }
 
-template <typename T, int... K, typename F>
+template <int... K, typename F>
 __device__ __forceinline__ bool pair_group(std::integer_sequence<int, K...>, int m, int last,
                                            F &&f) {
   return ((m + K <= last && (f(m + K, PIC<K>{}), true)) && ...);
@@ -272,7 +288,7 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
   __amdgpu_buffer_rsrc_t rin = pair_rsrc(a.buf[src], n);
   const __amdgpu_buffer_rsrc_t rrh = pair_rsrc(a.rhs, n);
 
-  // Ring slot of plane z0 - 4 + q is q & 7; z0 and the tile's first row are
+  // Ring slot of plane z0 - 4 + q is q % 8; z0 and the tile's first row are
   // even, so the parity of row + plane is (r + q) & 1.
   T R[NR][RY], B[NR][RY], fR[NR][RY], fB[NR][RY];
 #pragma unroll
@@ -286,8 +302,8 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
     const int z = z0 - 4 + q, im = zs * z + (z < 0 ? zlo : zhi);
     return planeB * (unsigned)(z < 0 || z >= nz ? im : z);
   };
-  auto load_p = [&](int q, auto SL) {
-    constexpr int sl = decltype(SL)::value & 7;
+  auto load_p = [&](int q, auto SL) __attribute__((always_inline)) {
+    constexpr int sl = decltype(SL)::value % NR;
     const unsigned so = zsoff(q);
 #pragma unroll
     for (int r = 0; r < RY; ++r) {
@@ -296,8 +312,8 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
       B[sl][r] = pload<T>(rin, odd ? vL[r] : vR[r], so + halfB);
     }
   };
-  auto load_f = [&](int q, auto SL) {
-    constexpr int sl = decltype(SL)::value & 7;
+  auto load_f = [&](int q, auto SL) __attribute__((always_inline)) {
+    constexpr int sl = decltype(SL)::value % NR;
     const unsigned so = zsoff(q);
 #pragma unroll
     for (int r = 0; r < RY; ++r) {
@@ -311,10 +327,10 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
   for (int r = 0; r < RY; ++r) dA[r] = dB[r] = T(0);
 
   // One half sweep of plane slot sl: X (this colour) from Y (the other), with
-  // the rows beside the thread's own from LDS; cnt: this plane counts for dmax.
+  // the rows beside the thread's own from LDS; CNT: the plane counts for dmax.
   auto half = [&](auto SL, auto COL, T(&X)[NR][RY], T(&Y)[NR][RY], const T(&F)[NR][RY], T lo,
-                  T hi, T w, T w1, bool cnt, T(&dm)[RY]) {
-    constexpr int sl = decltype(SL)::value & 7, sm = (sl + 7) & 7, sp = (sl + 1) & 7;
+                  T hi, T w, T w1, auto CNT, T(&dm)[RY]) __attribute__((always_inline)) {
+    constexpr int sl = decltype(SL)::value % NR, sm = (sl + NR - 1) % NR, sp = (sl + 1) % NR;
     constexpr int col = decltype(COL)::value;
     T d[RY];
 #pragma unroll
@@ -331,15 +347,15 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
       d[r] = pn - X[sl][r];
       X[sl][r] = w1 * X[sl][r] + w * pn;
     }
-    if (cnt) {
+    if constexpr (decltype(CNT)::value) {
 #pragma unroll
-      for (int r = 0; r < RY; ++r) dm[r] = T(__builtin_fmax(T(__builtin_fabs(d[r])), dm[r]));
+      for (int r = 0; r < RY; ++r) dm[r] = max_abs(dm[r], d[r]);
     }
   };
   // First and last rows of the four planes the step after step m reads.
-  auto publish = [&](int b, auto K) {
+  auto publish = [&](int b, auto K) __attribute__((always_inline)) {
     constexpr int k = decltype(K)::value;
-    constexpr int s0 = (k + 2) & 7, s1 = (k + 1) & 7, s2 = k & 7, s3 = (k + 7) & 7;
+    constexpr int s0 = (k + 2) % NR, s1 = (k + 1) % NR, s2 = k % NR, s3 = (k + NR - 1) % NR;
     ex[b][0][0][g + 1][lane] = B[s0][RY - 1];
     ex[b][0][1][g + 1][lane] = B[s0][0];
     ex[b][1][0][g + 1][lane] = R[s1][RY - 1];
@@ -402,13 +418,18 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
   const double oma = s.it0 <= a.gs ? 1.0 : s.om_a, omb = s.it0 + 1 <= a.gs ? 1.0 : s.om_b;
   const T wa = T(oma), wa1 = T(1.0 - oma), wb = T(omb), wb1 = T(1.0 - omb);
   const bool two = s.n == 2;
-  publish(0, PIC<7>{});  // before step 0: its red reads plane slot 1's black
+  publish(0, PIC<NR - 1>{});  // before step 0: its red reads plane slot 1's black
   __syncthreads();
 
-  // Step m: t = z0 - 3 + m, slot of plane t is (m + 1) & 7.
+  // Step m: t = z0 - 3 + m, slot of plane t is (m + 1) % 8.
   const int last = z1 - z0 + 5;
-  auto step = [&](int m, auto K) {
+  // FIRST: steps 0 .. NR - 1, whose later half sweeps have not reached a plane
+  // with valid inputs yet: those do not count for dmax and are not stored.  From
+  // then on every half sweep updates nodes of the grid (the chunk's own or, at
+  // its end, the next one's, whose updates are the same there).
+  auto step = [&](int m, auto K, auto FIRST, auto TWO) __attribute__((always_inline)) {
     constexpr int k = decltype(K)::value;
+    constexpr bool first = decltype(FIRST)::value != 0, two = decltype(TWO)::value != 0;
     load_p(m + 3, PIC<k + 3>{});
     load_f(m + 2, PIC<k + 2>{});
     const int b = m & 1;
@@ -418,18 +439,19 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
       lo[q] = ex[b][q][0][g][lane];
       hi[q] = ex[b][q][1][g + 2][lane];
     }
-    const int t = z0 - 3 + m;
-    half(PIC<k + 1>{}, PIC<0>{}, R, B, fR, lo[0], hi[0], wa, wa1, t >= z0 && t < z1, dA);
-    half(PIC<k>{}, PIC<1>{}, B, R, fB, lo[1], hi[1], wa, wa1, t - 1 >= z0 && t - 1 < z1, dA);
-    if (two) {
-      half(PIC<k + 7>{}, PIC<0>{}, R, B, fR, lo[2], hi[2], wb, wb1, t - 2 >= z0 && t - 2 < z1,
-           dB);
-      half(PIC<k + 6>{}, PIC<1>{}, B, R, fB, lo[3], hi[3], wb, wb1, t - 3 >= z0, dB);
+    half(PIC<k + 1>{}, PIC<0>{}, R, B, fR, lo[0], hi[0], wa, wa1, PIC<1>{}, dA);
+    half(PIC<k>{}, PIC<1>{}, B, R, fB, lo[1], hi[1], wa, wa1,
+         PIC<!first || k >= 2>{}, dA);
+    if constexpr (two) {
+      half(PIC<k + NR - 1>{}, PIC<0>{}, R, B, fR, lo[2], hi[2], wb, wb1,
+           PIC<!first || k >= 4>{}, dB);
+      half(PIC<k + NR - 2>{}, PIC<1>{}, B, R, fB, lo[3], hi[3], wb, wb1,
+           PIC<!first || k >= 6>{}, dB);
     }
     publish(1 - b, K);
-    if (t - 3 >= z0) {
-      constexpr int sl = (k + 6) & 7;
-      const unsigned so = planeB * (unsigned)(t - 3);
+    if constexpr (!first || k >= 6) {
+      constexpr int sl = (k + NR - 2) % NR;
+      const unsigned so = planeB * (unsigned)(z0 - 6 + m);
 #pragma unroll
       for (int r = 0; r < RY; ++r)
         if (own[r]) {
@@ -449,8 +471,15 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
     }
     __syncthreads();
   };
-  for (int m = 0; pair_group<T>(std::make_integer_sequence<int, 8>{}, m, last, step); m += 8) {
-  }
+  auto march = [&](auto TWO) __attribute__((always_inline)) {
+    auto head = [&](int m, auto K) __attribute__((always_inline)) { step(m, K, PIC<1>{}, TWO); };
+    auto body = [&](int m, auto K) __attribute__((always_inline)) { step(m, K, PIC<0>{}, TWO); };
+    if (!pair_group(std::make_integer_sequence<int, NR>{}, 0, last, head)) return;
+    for (int m = NR; pair_group(std::make_integer_sequence<int, NR>{}, m, last, body); m += NR) {
+    }
+  };
+  if (two) march(PIC<1>{});
+  else march(PIC<0>{});
 
   T ma = T(0), mb = T(0);
 #pragma unroll
