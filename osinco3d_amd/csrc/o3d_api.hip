@@ -2202,40 +2202,6 @@ __global__ void lw_coarse_init_kernel(float *__restrict__ u0, const float *__res
   if (I < nc) u0[I] = s * (out[I] - in1[I]);
 }
 
-// q += trilinear interpolation of the coarse correction c (the multigrid
-// solution on the grid of F^3 block averages), one thread per pair of cells
-// (2t, 2t + 1) of a row (nx even), 16-byte accesses.
-__global__ void __launch_bounds__(256) mg_prolong_fine_kernel(double *__restrict__ q,
-                                                              const float *__restrict__ c,
-                                                              int nx, int ny, int nz, int F,
-                                                              int px, int py, int pz) {
-  const int t = blockIdx.x * 64 + threadIdx.x;
-  const int j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.z;
-  if (2 * t >= nx || j >= ny) return;
-  const int mx = nx / F, my = ny / F, mz = nz / F;
-  int y0, y1, z0, z1;
-  float wy, wz;
-  lw_axis(j, F, my, py, y0, y1, wy);
-  lw_axis(k, F, mz, pz, z0, z1, wz);
-  auto v = [&](int a, int b, int d) { return c[(size_t)a + (size_t)mx * (b + (size_t)my * d)]; };
-  float tv[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    int x0, x1;
-    float wx;
-    lw_axis(2 * t + h, F, mx, px, x0, x1, wx);
-    tv[h] = (1.f - wz) * ((1.f - wy) * ((1.f - wx) * v(x0, y0, z0) + wx * v(x1, y0, z0)) +
-                          wy * ((1.f - wx) * v(x0, y1, z0) + wx * v(x1, y1, z0))) +
-            wz * ((1.f - wy) * ((1.f - wx) * v(x0, y0, z1) + wx * v(x1, y0, z1)) +
-                  wy * ((1.f - wx) * v(x0, y1, z1) + wx * v(x1, y1, z1)));
-  }
-  double2 *o = reinterpret_cast<double2 *>(q + (size_t)nx * (j + (size_t)ny * k)) + t;
-  double2 w = *o;
-  w.x = w.x + (double)tv[0];
-  w.y = w.y + (double)tv[1];
-  *o = w;
-}
-
 __global__ void __launch_bounds__(256) lw_sumsq_kernel(const float *a, int n, double *part) {
   __shared__ double sc[4];
   double s = 0.0;
@@ -2500,10 +2466,7 @@ int solver_warm_guess(Solver &S, int *used, double *warm) {
     const int cyc = nn_coarse && S.p.coarse_cycles_learned > 0 ? S.p.coarse_cycles_learned
                                                                 : S.p.coarse_cycles;
     HIPCHK(mg_solve(S.mg, cyc, 1, 1, g_stream, !nn_coarse));
-    dim3 grid((S.p.nx / 2 + 63) / 64, (S.p.ny + 3) / 4, S.p.nz);
-    mg_prolong_fine_kernel<<<grid, dim3(64, 4), 0, g_stream>>>(q, S.mg.u[0], S.p.nx, S.p.ny,
-                                                               S.p.nz, F, per[0], per[1], per[2]);
-    HIPCHK(hipGetLastError());
+    HIPCHK(mg_prolong_add(q, S.mg.u[0], S.p.nx, S.p.ny, S.p.nz, per, g_stream));
   }
   CHK(lw_residual_l2_pair(S, S.P[S.cur], q, warm));
   if (warm[1] < warm[0]) {

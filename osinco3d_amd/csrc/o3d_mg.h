@@ -30,8 +30,8 @@ size_t mg_plan(MgHierarchy &H, const int m0[3], const double h[3], const int per
 void mg_bind(MgHierarchy &H, float *base);
 // `cycles` V(nu1, nu2) cycles on L u0 = f0 (f0 = H.f[0] filled by the
 // caller) from u0 = 0, or from the u0 = H.u[0] the caller wrote
-// (from_zero = false).
-hipError_t mg_solve(const MgHierarchy &H, int cycles, int nu1, int nu2, hipStream_t s,
+// (from_zero = false).  u and r of a level may trade places: read H.u[0] after.
+hipError_t mg_solve(MgHierarchy &H, int cycles, int nu1, int nu2, hipStream_t s,
                     bool from_zero = true);
 // The coarse-grid correction of a correction solve held in colour-split
 // storage (per row, the red nodes then the black ones, nx/2 entries each;
@@ -41,6 +41,9 @@ hipError_t mg_solve(const MgHierarchy &H, int cycles, int nu1, int nu2, hipStrea
 hipError_t mg_pool_split(const float *r, float *f0, int nx, int ny, int nz, hipStream_t s);
 hipError_t mg_prolong_split(float *e, const float *u0, int nx, int ny, int nz, const int per[3],
                             hipStream_t s);
+// q += the same interpolation, in natural order and FP64.
+hipError_t mg_prolong_add(double *q, const float *u0, int nx, int ny, int nz, const int per[3],
+                          hipStream_t s);
 // u0 = the trilinear interpolation of the level-1 field H.u[1] (a starting
 // iterate given on the next coarser level).  Needs two levels at least.
 hipError_t mg_seed_from_level1(const MgHierarchy &H, hipStream_t s);

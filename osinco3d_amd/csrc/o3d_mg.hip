@@ -11,6 +11,7 @@
 // colour being relaxed (or a pair of cells), and the levels of at most 16^3
 // cells run as one V-cycle in one block's LDS; the launch count dominates.
 #include <algorithm>
+#include <utility>
 
 #include "o3d_mg.h"
 
@@ -93,63 +94,269 @@ __device__ __forceinline__ float mg_relax_value(float fq, float sx, float sy, fl
   return (fq - (g.cx * sx + g.cy * sy + g.cz * sz)) * g.invd;
 }
 
-// Residual f - L u at cell (i, j, k).
-__device__ __forceinline__ float mg_res(const float *u, const float *f, const MgGrid &g, int i,
-                                        int j, int k) {
-  const int q = i + g.mx * (j + g.my * k);
-  return f[q] - (mg_lap_off(u, g, i, j, k) + g.diag * u[q]);
-}
-
-// The residual averaged over the 8 children of coarse cell (I, J, K).
+// The residual f - L u averaged over the 8 children of coarse cell (I, J, K),
+// the fine level's axes even: the children's own cells and the faces around
+// them are loaded once (20 loads of one or two cells, against 7 per child).
 __device__ __forceinline__ float mg_child_mean(const float *u, const float *f, const MgGrid &g,
                                                int I, int J, int K) {
+  const int i = 2 * I, j = 2 * J, k = 2 * K, pl = g.mx * g.my;
+  const int xm = mg_nb(i - 1, g.mx, g.px), xp = mg_nb(i + 2, g.mx, g.px);
+  const int ry[4] = {g.mx * mg_nb(j - 1, g.my, g.py), g.mx * j, g.mx * (j + 1),
+                     g.mx * mg_nb(j + 2, g.my, g.py)};
+  const int rz[4] = {pl * mg_nb(k - 1, g.mz, g.pz), pl * k, pl * (k + 1),
+                     pl * mg_nb(k + 2, g.mz, g.pz)};
+  auto pair = [&](const float *a, int y, int z) {
+    return *reinterpret_cast<const float2 *>(a + (i + ry[y] + rz[z]));
+  };
+  float2 c[4][4];  // [z][y], the rows that hold children or face them
+#pragma unroll
+  for (int z = 0; z < 4; ++z)
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+      if ((y == 1 || y == 2) || (z == 1 || z == 2)) c[z][y] = pair(u, y, z);
   float s = 0.f;
 #pragma unroll
-  for (int c = 0; c < 8; ++c)
-    s += mg_res(u, f, g, 2 * I + (c & 1), 2 * J + ((c >> 1) & 1), 2 * K + (c >> 2));
+  for (int n = 0; n < 4; ++n) {
+    const int y = 1 + (n & 1), z = 1 + (n >> 1);
+    const int row = ry[y] + rz[z];
+    const float2 v = c[z][y], ff = pair(f, y, z);
+    const float l = u[row + xm], r = u[row + xp];
+    const float2 ya = c[z][y - 1], yb = c[z][y + 1], za = c[z - 1][y], zb = c[z + 1][y];
+    s += ff.x - ((g.cx * (l + v.y) + g.cy * (ya.x + yb.x) + g.cz * (za.x + zb.x)) + g.diag * v.x);
+    s += ff.y - ((g.cx * (v.x + r) + g.cy * (ya.y + yb.y) + g.cz * (za.y + zb.y)) + g.diag * v.y);
+  }
   return 0.125f * s;
 }
 
-// Position of fine cell i on the grid coarser by 2: lower coarse cell and
-// the weight of the upper one (cell-centred; periodic wraps, others clamp).
-__device__ __forceinline__ void mg_axis(int i, int m, int per, int &c0, int &c1, float &w) {
-  const float X = 0.5f * (float)i - 0.25f;
-  int I0 = (int)floorf(X);
-  w = X - (float)I0;
-  int I1 = I0 + 1;
-  if (per) {
-    I0 = I0 < 0 ? I0 + m : I0;
-    I1 = I1 >= m ? I1 - m : I1;
-  } else {
-    if (I0 < 0) { I0 = 0; w = 0.f; }
-    if (I1 >= m) { I1 = m - 1; w = I0 == m - 1 ? 0.f : w; }
+// Trilinear interpolation of the coarse field uc (cx, cy, cz cells) at the 8
+// fine cells of coarse cell (I, J, K), v[2 * (2 * dz + dy) + dx].  Along an
+// axis a fine cell lies a quarter of a coarse cell from its own coarse cell's
+// centre: weight 1/4 of the neighbour on its side (periodic wraps, others
+// clamp).  Lines along x first, then y, then z; 27 loads for 8 cells.
+__device__ __forceinline__ void mg_interp_cell(const float *uc, int I, int J, int K, int cx,
+                                               int cy, int cz, int px, int py, int pz,
+                                               float v[8]) {
+  const int x[3] = {mg_nb(I - 1, cx, px), I, mg_nb(I + 1, cx, px)};
+  const int y[3] = {cx * mg_nb(J - 1, cy, py), cx * J, cx * mg_nb(J + 1, cy, py)};
+  const int pl = cx * cy;
+  const int z[3] = {pl * mg_nb(K - 1, cz, pz), pl * K, pl * mg_nb(K + 1, cz, pz)};
+  // Weight of the upper coarse cell for the lower and upper fine cell.
+  const float x0 = !px && I == 0 ? 0.f : 0.75f, x1 = !px && I == cx - 1 ? 0.f : 0.25f;
+  const float y0 = !py && J == 0 ? 0.f : 0.75f, y1 = !py && J == cy - 1 ? 0.f : 0.25f;
+  const float z0 = !pz && K == 0 ? 0.f : 0.75f, z1 = !pz && K == cz - 1 ? 0.f : 0.25f;
+  float p[3][4];  // per coarse plane, the 4 fine cells of (dy, dx)
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    float l[3], r[3];
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+      const float *q = uc + (y[b] + z[c]);
+      const float a0 = q[x[0]], a1 = q[x[1]], a2 = q[x[2]];
+      l[b] = (1.f - x0) * a0 + x0 * a1;
+      r[b] = (1.f - x1) * a1 + x1 * a2;
+    }
+    p[c][0] = (1.f - y0) * l[0] + y0 * l[1];
+    p[c][1] = (1.f - y0) * r[0] + y0 * r[1];
+    p[c][2] = (1.f - y1) * l[1] + y1 * l[2];
+    p[c][3] = (1.f - y1) * r[1] + y1 * r[2];
   }
-  c0 = I0;
-  c1 = I1;
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    v[n] = (1.f - z0) * p[0][n] + z0 * p[1][n];
+    v[4 + n] = (1.f - z1) * p[1][n] + z1 * p[2][n];
+  }
 }
 
-// Trilinear interpolation of the coarse field uc (cx, cy, cz cells) at the
-// fine cells (2I, j, k) and (2I + 1, j, k).
-__device__ __forceinline__ float2 mg_interp_pair(const float *uc, int I, int j, int k, int cx,
-                                                 int cy, int cz, int px, int py, int pz) {
-  int y0, y1, z0, z1;
-  float wy, wz;
-  mg_axis(j, cy, py, y0, y1, wy);
-  mg_axis(k, cz, pz, z0, z1, wz);
-  const int r00 = cx * (y0 + cy * z0), r10 = cx * (y1 + cy * z0);
-  const int r01 = cx * (y0 + cy * z1), r11 = cx * (y1 + cy * z1);
-  float v[2];
+// ------------------------------------------------------ fused level kernels
+// One whole red-black sweep of a level with everything around it in one
+// launch, for levels with every axis even.  A block stages a tile of 32 x 8 x
+// TZ cells with a halo of 2 in LDS, relaxes red on the tile and one cell
+// around it, then black on the tile, so neighbouring blocks recompute the halo
+// instead of meeting between the colours; the result goes to another array.
+//   ZERO      the level starts from u = 0 (nothing is read, and red is f / diag)
+//   PROLONG   u += the interpolated coarse correction before the sweep
+//   RESTRICT  (with ZERO) the averaged residual after the sweep goes to fc
+// Same updates in the same order as mg_smooth_kernel, mg_restrict_kernel and
+// mg_prolong_kernel, so the values are the same.  What bounds the levels is the
+// number of launches (3 to 4 us each below 128^3) and, at 128^3, the work per
+// cell of the tile and halo (a thread stages whole columns, so the index
+// arithmetic is once per column: with it per cell the kernel took twice as
+// long).  A V(1, 1) level was 8 launches and is 2: 128^3, from zero with
+// restriction 30 -> 10 us, with prolongation 23 -> 13 us; 64^3 12 -> 4.7 and
+// 10.5 -> 5.0 us; a plain sweep of 128^3 14.6 -> 10.6 us.
+constexpr int kSwX = 32, kSwY = 8, kSwNT = 512;
+
+template <int TZ, bool ZERO, bool PROLONG, bool RESTRICT>
+__global__ void __launch_bounds__(kSwNT) mg_sweep_kernel(float *__restrict__ uo,
+                                                         const float *__restrict__ u,
+                                                         const float *__restrict__ f,
+                                                         const float *__restrict__ uc,
+                                                         float *__restrict__ fc, MgGrid g,
+                                                         int ntx, int nty) {
+  static_assert(!RESTRICT || ZERO, "the residual's black halo needs red on a halo of 2");
+  constexpr int LX = kSwX + 4, LY = kSwY + 4, LZ = TZ + 4, LP = LX * LY;  // u, halo of 2
+  constexpr int HF = ZERO ? 2 : 1;                                        // f's halo
+  constexpr int FX = kSwX + 2 * HF, FY = kSwY + 2 * HF, FZ = TZ + 2 * HF, FP = FX * FY;
+  constexpr int CX = kSwX / 2 + 4, CY = kSwY / 2 + 4, CZ = TZ / 2 + 4;
+  static_assert(LP <= kSwNT && CX * CY <= kSwNT, "one column per thread");
+  __shared__ float su[LZ * LP];
+  __shared__ float sf[FZ * FP];
+  __shared__ float sc[PROLONG ? CZ * CY * CX : 1];
+  const int t = xcd_tile(blockIdx.x, gridDim.x);
+  const int bx = t % ntx, r = t / ntx, by = r % nty, bz = r / nty;
+  const int x0 = bx * kSwX, y0 = by * kSwY, z0 = bz * TZ;
+  const int tid = threadIdx.x;
+  const int plane = g.mx * g.my;
+  // Stored cell of cell q (periodic image; elsewhere any cell of the level,
+  // for positions that no cell of the tile reads).
+  auto img = [](int q, int m, int per) {
+    if (q < 0) q = per ? q + m : 0;
+    if (q >= m) q = per ? q - m : m - 1;
+    return min(max(q, 0), m - 1);
+  };
+  // A thread stages one column of each array; z is the same for the block.
+  if (tid < FP) {
+    const int lx = tid % FX, ly = tid / FX;
+    const float *fp = f + img(x0 - HF + lx, g.mx, g.px) + g.mx * img(y0 - HF + ly, g.my, g.py);
+    float v[FZ];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    int x0, x1;
-    float wx;
-    mg_axis(2 * I + h, cx, px, x0, x1, wx);
-    v[h] = (1.f - wz) * ((1.f - wy) * ((1.f - wx) * uc[r00 + x0] + wx * uc[r00 + x1]) +
-                         wy * ((1.f - wx) * uc[r10 + x0] + wx * uc[r10 + x1])) +
-           wz * ((1.f - wy) * ((1.f - wx) * uc[r01 + x0] + wx * uc[r01 + x1]) +
-                 wy * ((1.f - wx) * uc[r11 + x0] + wx * uc[r11 + x1]));
+    for (int lz = 0; lz < FZ; ++lz) v[lz] = fp[(size_t)plane * img(z0 - HF + lz, g.mz, g.pz)];
+#pragma unroll
+    for (int lz = 0; lz < FZ; ++lz) {
+      sf[tid + FP * lz] = v[lz];
+      // Red of the first sweep from zero; x0, y0, z0 and the halo are even.
+      if (ZERO) su[tid + FP * lz] = ((lx + ly + lz) & 1) == 0 ? v[lz] * g.invd : 0.f;
+    }
   }
-  return make_float2(v[0], v[1]);
+  if (!ZERO) {
+    const int lx = tid % LX, ly = tid / LX;
+    const int gi = x0 - 2 + lx, gj = y0 - 2 + ly;
+    const float *up = u + img(gi, g.mx, g.px) + g.mx * img(gj, g.my, g.py);
+    float v[LZ];
+    if (tid < LP) {
+#pragma unroll
+      for (int lz = 0; lz < LZ; ++lz) v[lz] = up[(size_t)plane * img(z0 - 2 + lz, g.mz, g.pz)];
+    }
+    if (PROLONG) {
+      if (tid < CX * CY) {
+        const int cx = g.mx >> 1, cy = g.my >> 1, cz = g.mz >> 1;
+        const float *cp = uc + img(x0 / 2 - 2 + tid % CX, cx, g.px) +
+                          cx * img(y0 / 2 - 2 + tid / CX, cy, g.py);
+#pragma unroll
+        for (int lz = 0; lz < CZ; ++lz)
+          sc[tid + CX * CY * lz] = cp[(size_t)(cx * cy) * img(z0 / 2 - 2 + lz, cz, g.pz)];
+      }
+      __syncthreads();
+    }
+    if (tid < LP) {
+      // Lower coarse cell (local) and weight of the upper one (mg_interp_cell).
+      const int X = (lx + 1) >> 1, Y = (ly + 1) >> 1;
+      float wx = (lx & 1) ? 0.25f : 0.75f, wy = (ly & 1) ? 0.25f : 0.75f;
+      if (!g.px && (gi <= 0 || gi >= g.mx - 1)) wx = 0.f;
+      if (!g.py && (gj <= 0 || gj >= g.my - 1)) wy = 0.f;
+      float c[CZ];
+      if (PROLONG) {
+#pragma unroll
+        for (int Z = 0; Z < CZ; ++Z) {
+          const float *a = sc + X + CX * (Y + CY * Z);
+          c[Z] = (1.f - wy) * ((1.f - wx) * a[0] + wx * a[1]) +
+                 wy * ((1.f - wx) * a[CX] + wx * a[CX + 1]);
+        }
+      }
+#pragma unroll
+      for (int lz = 0; lz < LZ; ++lz) {
+        float w = v[lz];
+        if (PROLONG) {
+          const int gk = z0 - 2 + lz, Z = (lz + 1) >> 1;
+          float wz = (lz & 1) ? 0.25f : 0.75f;
+          if (!g.pz && (gk <= 0 || gk >= g.mz - 1)) wz = 0.f;
+          w += (1.f - wz) * c[Z] + wz * c[Z + 1];
+        }
+        su[tid + LP * lz] = w;
+      }
+    }
+  }
+  __syncthreads();
+  // Offsets of the neighbours of a cell of su, the cell itself (the mirror)
+  // past an edge of an axis that does not wrap.
+  auto below = [](int q, int per, int d) { return !per && q == 0 ? 0 : -d; };
+  auto above = [](int q, int m, int per, int d) { return !per && q == m - 1 ? 0 : d; };
+  // A colour on the tile and one cell around it: a thread takes one pair of
+  // columns (17 pairs x 10 rows) on every third plane.
+  auto relax = [&](int colour) {
+    constexpr int HX = kSwX / 2 + 1, HY = kSwY + 2, HC = HX * HY, ZG = kSwNT / HC;
+    if (tid >= HC * ZG) return;
+    const int zg = tid / HC, q = tid - zg * HC;
+    const int ly = 1 + q / HX, lxp = 1 + 2 * (q % HX);
+    const int ym = below(y0 - 2 + ly, g.py, LX), yp = above(y0 - 2 + ly, g.my, g.py, LX);
+#pragma unroll
+    for (int n = 0; n < (TZ + 2 + ZG - 1) / ZG; ++n) {
+      const int lz = 1 + zg + n * ZG;
+      if (lz > TZ + 2) break;
+      const int lx = lxp + ((1 + ly + lz + colour) & 1);
+      const int i = x0 - 2 + lx, k = z0 - 2 + lz;
+      float *c = su + lx + LX * ly + LP * lz;
+      const float sx = c[below(i, g.px, 1)] + c[above(i, g.mx, g.px, 1)];
+      const float sy = c[ym] + c[yp];
+      const float sz = c[below(k, g.pz, LP)] + c[above(k, g.mz, g.pz, LP)];
+      *c = mg_relax_value(sf[lx - 2 + HF + FX * (ly - 2 + HF) + FP * (lz - 2 + HF)], sx, sy, sz,
+                          g);
+    }
+  };
+  if (!ZERO) {
+    relax(0);
+    __syncthreads();
+  }
+  if (RESTRICT) {
+    relax(1);
+    __syncthreads();
+    constexpr int NC = kSwX / 2 * (kSwY / 2) * (TZ / 2);
+    if (tid < NC) {
+      const int I = tid % (kSwX / 2), J = tid / (kSwX / 2) % (kSwY / 2),
+                K = tid / (kSwX / 2 * (kSwY / 2));
+      float s = 0.f;
+#pragma unroll
+      for (int n = 0; n < 8; ++n) {
+        const int lx = 2 + 2 * I + (n & 1), ly = 2 + 2 * J + ((n >> 1) & 1),
+                  lz = 2 + 2 * K + (n >> 2);
+        const int i = x0 - 2 + lx, j = y0 - 2 + ly, k = z0 - 2 + lz;
+        const float *c = su + lx + LX * ly + LP * lz;
+        // Even children have no upper edge, odd ones no lower edge.
+        const float sx = c[n & 1 ? -1 : below(i, g.px, 1)] + c[n & 1 ? above(i, g.mx, g.px, 1) : 1];
+        const float sy = c[n & 2 ? -LX : below(j, g.py, LX)] +
+                         c[n & 2 ? above(j, g.my, g.py, LX) : LX];
+        const float sz = c[n & 4 ? -LP : below(k, g.pz, LP)] +
+                         c[n & 4 ? above(k, g.mz, g.pz, LP) : LP];
+        s += sf[lx + FX * ly + FP * lz] -
+             ((g.cx * sx + g.cy * sy + g.cz * sz) + g.diag * *c);
+      }
+      const int ci = x0 / 2 + I, cj = y0 / 2 + J, ck = z0 / 2 + K;
+      if (2 * ci < g.mx && 2 * cj < g.my && 2 * ck < g.mz)
+        fc[ci + (g.mx >> 1) * (cj + (g.my >> 1) * ck)] = 0.125f * s;
+    }
+  }
+  // The tile's cells: a column of every second plane per thread, so the colour
+  // is the column's.
+  const int lx = 2 + tid % kSwX, ly = 2 + tid / kSwX % kSwY, zb = tid / (kSwX * kSwY);
+  const int i = x0 - 2 + lx, j = y0 - 2 + ly;
+  if (i >= g.mx || j >= g.my) return;
+  const int xm = below(i, g.px, 1), xp = above(i, g.mx, g.px, 1);
+  const int ym = below(j, g.py, LX), yp = above(j, g.my, g.py, LX);
+  const bool black = !RESTRICT && ((lx + ly + zb) & 1);
+  float *o = uo + i + (size_t)g.mx * j;
+#pragma unroll
+  for (int n = 0; n < TZ / 2; ++n) {
+    const int lz = 2 + zb + 2 * n, k = z0 - 2 + lz;
+    if (k >= g.mz) break;
+    const float *c = su + lx + LX * ly + LP * lz;
+    float v = *c;
+    if (black) {  // from the finished red
+      const float sz = c[below(k, g.pz, LP)] + c[above(k, g.mz, g.pz, LP)];
+      v = mg_relax_value(sf[lx - 2 + HF + FX * (ly - 2 + HF) + FP * (lz - 2 + HF)],
+                         c[xm] + c[xp], c[ym] + c[yp], sz, g);
+    }
+    o[(size_t)plane * k] = v;
+  }
 }
 
 // One colour of a red-black Gauss-Seidel sweep, one thread per cell of that
@@ -184,9 +391,8 @@ __global__ void __launch_bounds__(256) mg_smooth_any_kernel(float *__restrict__ 
 }
 
 // fc = the residual of the fine level averaged over the 8 children of each
-// coarse cell; uc = 0.
+// coarse cell.
 __global__ void __launch_bounds__(256) mg_restrict_kernel(float *__restrict__ fc,
-                                                          float *__restrict__ uc,
                                                           const float *__restrict__ u,
                                                           const float *__restrict__ f, MgGrid g) {
   const int cx = g.mx >> 1, cy = g.my >> 1, cz = g.mz >> 1;
@@ -195,25 +401,29 @@ __global__ void __launch_bounds__(256) mg_restrict_kernel(float *__restrict__ fc
   const int crow = idx / cx, I = idx - crow * cx;
   const int K = crow / cy, J = crow - K * cy;
   fc[idx] = mg_child_mean(u, f, g, I, J, K);
-  uc[idx] = 0.f;
 }
 
 // u += trilinear interpolation of the coarse correction uc, one thread per
-// pair of fine cells (2I, 2I + 1) of a row.
+// coarse cell.
 __global__ void __launch_bounds__(256) mg_prolong_kernel(float *__restrict__ u,
                                                          const float *__restrict__ uc, int mx,
                                                          int my, int mz, int px, int py, int pz) {
-  const int cx = mx >> 1;
+  const int cx = mx >> 1, cy = my >> 1, cz = mz >> 1;
   const int p = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (p >= cx * my * mz) return;
+  if (p >= cx * cy * cz) return;
   const int row = p / cx, I = p - row * cx;
-  const int k = row / my, j = row - k * my;
-  const float2 v = mg_interp_pair(uc, I, j, k, cx, my >> 1, mz >> 1, px, py, pz);
-  float2 *o = reinterpret_cast<float2 *>(u + (size_t)mx * row) + I;
-  float2 w = *o;
-  w.x += v.x;
-  w.y += v.y;
-  *o = w;
+  const int K = row / cy, J = row - K * cy;
+  float v[8];
+  mg_interp_cell(uc, I, J, K, cx, cy, cz, px, py, pz, v);
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    const size_t fr = (size_t)(2 * J + (n & 1)) + (size_t)my * (2 * K + (n >> 1));
+    float2 *o = reinterpret_cast<float2 *>(u + (size_t)mx * fr) + I;
+    float2 w = *o;
+    w.x += v[2 * n];
+    w.y += v[2 * n + 1];
+    *o = w;
+  }
 }
 
 // The coarsest level: `sweeps` red-black Gauss-Seidel sweeps from u = 0 by
@@ -256,6 +466,17 @@ struct MgSmall {
   int nu1, nu2, coarse_sweeps;
 };
 
+// p / n for the cell counts of the small levels (p < 2^16): exact, since
+// (p + 1/2) / n is at least 1 / (2 n) away from an integer, far more than the
+// rounding of the two float operations; an integer division by a run-time n
+// is some 20 instructions.
+struct SmallDiv {
+  int n;
+  float inv;
+  __device__ __forceinline__ explicit SmallDiv(int n_) : n(n_), inv(1.0f / (float)n_) {}
+  __device__ __forceinline__ int div(int p) const { return (int)(((float)p + 0.5f) * inv); }
+};
+
 __device__ __forceinline__ void lds_smooth(float *u, const float *f, const MgGrid &g,
                                            int sweeps) {
   if (g.mx & 1) {
@@ -271,23 +492,33 @@ __device__ __forceinline__ void lds_smooth(float *u, const float *f, const MgGri
       }
     return;
   }
-  const int hx = g.mx >> 1, nh = hx * g.my * g.mz;
-  int t[kMgSmallPer], jj[kMgSmallPer], kk[kMgSmallPer];
+  // Per cell pair of this thread: its offset and, for both of its cells, the
+  // neighbours' (the y and z neighbours lie in the rows beside).
+  const int hx = g.mx >> 1, nh = hx * g.my * g.mz, pl = g.mx * g.my;
+  const SmallDiv dx(hx), dy(g.my);
+  int base[kMgSmallPer], oxl[kMgSmallPer], oxr[kMgSmallPer], oym[kMgSmallPer], oyp[kMgSmallPer],
+      ozm[kMgSmallPer], ozp[kMgSmallPer];
 #pragma unroll
   for (int s = 0; s < kMgSmallPer; ++s) {
     const int p = threadIdx.x + s * kMgSmallThreads;
-    const int row = p / hx;
-    t[s] = p - row * hx;
-    kk[s] = row / g.my;
-    jj[s] = row - kk[s] * g.my;
+    const int row = dx.div(p), t = p - row * hx, k = dy.div(row), j = row - k * g.my;
+    base[s] = (2 * t + g.mx * row) * 2 + ((j + k) & 1);
+    oxl[s] = mg_nb(2 * t - 1, g.mx, g.px) - 2 * t;
+    oxr[s] = mg_nb(2 * t + 2, g.mx, g.px) - 2 * t;
+    oym[s] = g.mx * (mg_nb(j - 1, g.my, g.py) - j);
+    oyp[s] = g.mx * (mg_nb(j + 1, g.my, g.py) - j);
+    ozm[s] = pl * (mg_nb(k - 1, g.mz, g.pz) - k);
+    ozp[s] = pl * (mg_nb(k + 1, g.mz, g.pz) - k);
   }
   for (int sw = 0; sw < sweeps; ++sw)
     for (int colour = 0; colour < 2; ++colour) {
 #pragma unroll
       for (int s = 0; s < kMgSmallPer; ++s)
         if (threadIdx.x + s * kMgSmallThreads < nh) {
-          const int i = 2 * t[s] + ((jj[s] + kk[s] + colour) & 1);
-          mg_relax(u, f, g, i, jj[s], kk[s], i + g.mx * (jj[s] + g.my * kk[s]));
+          const int right = (base[s] + colour) & 1, l = base[s] >> 1, q = l + right;
+          const float sx = u[right ? l : l + oxl[s]] + u[right ? l + oxr[s] : l + 1];
+          u[q] = mg_relax_value(f[q], sx, u[q + oym[s]] + u[q + oyp[s]],
+                                u[q + ozm[s]] + u[q + ozp[s]], g);
         }
       __syncthreads();
     }
@@ -335,7 +566,7 @@ __device__ __forceinline__ void wave_smooth(float *u, const float *f, const MgGr
 
 __global__ void __launch_bounds__(kMgSmallThreads) mg_small_vcycle_kernel(
     float *__restrict__ u_out, const float *__restrict__ f_in, MgSmall S) {
-  __shared__ float su[kMgSmallCells], sf[kMgSmallCells];
+  __shared__ __align__(16) float su[kMgSmallCells], sf[kMgSmallCells];
   const int n0 = S.g[0].mx * S.g[0].my * S.g[0].mz;
   for (int q = threadIdx.x; q < n0; q += kMgSmallThreads) {
     sf[q] = f_in[q];
@@ -351,9 +582,10 @@ __global__ void __launch_bounds__(kMgSmallThreads) mg_small_vcycle_kernel(
     const float *f = sf + S.off[l];
     lds_smooth(u, f, g, S.nu1);
     const int nc = c.mx * c.my * c.mz;
+    const SmallDiv dx(c.mx), dy(c.my);
     for (int q = threadIdx.x; q < nc; q += kMgSmallThreads) {
-      const int crow = q / c.mx, I = q - crow * c.mx;
-      const int K = crow / c.my, J = crow - K * c.my;
+      const int crow = dx.div(q), I = q - crow * c.mx;
+      const int K = dy.div(crow), J = crow - K * c.my;
       sf[S.off[l + 1] + q] = mg_child_mean(u, f, g, I, J, K);
       su[S.off[l + 1] + q] = 0.f;
     }
@@ -376,13 +608,19 @@ __global__ void __launch_bounds__(kMgSmallThreads) mg_small_vcycle_kernel(
     const MgGrid &g = S.g[l], &c = S.g[l + 1];
     float *u = su + S.off[l];
     const float *uc = su + S.off[l + 1];
-    const int hx = g.mx >> 1, np = hx * g.my * g.mz;
+    const int np = c.mx * c.my * c.mz;
+    const SmallDiv dx(c.mx), dy(c.my);
     for (int q = threadIdx.x; q < np; q += kMgSmallThreads) {
-      const int row = q / hx, I = q - row * hx;
-      const int k = row / g.my, j = row - k * g.my;
-      const float2 v = mg_interp_pair(uc, I, j, k, c.mx, c.my, c.mz, g.px, g.py, g.pz);
-      u[g.mx * row + 2 * I] += v.x;
-      u[g.mx * row + 2 * I + 1] += v.y;
+      const int row = dx.div(q), I = q - row * c.mx;
+      const int K = dy.div(row), J = row - K * c.my;
+      float v[8];
+      mg_interp_cell(uc, I, J, K, c.mx, c.my, c.mz, g.px, g.py, g.pz, v);
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        float *o = u + 2 * I + g.mx * (2 * J + (n & 1) + g.my * (2 * K + (n >> 1)));
+        o[0] += v[2 * n];
+        o[1] += v[2 * n + 1];
+      }
     }
     __syncthreads();
     lds_smooth(u, sf + S.off[l], g, S.nu2);
@@ -428,9 +666,41 @@ bool small_from(const MgHierarchy &H, int l) {
   }
   return tot <= (size_t)kMgSmallCells;
 }
-hipError_t vcycle(const MgHierarchy &H, int l, int nu1, int nu2, hipStream_t s) {
+// One sweep of level l from H.u[l] into H.r[l], which then trade places.  Tiles
+// of 8 planes, or of 4 while 8 would leave CUs without a block.
+template <bool ZERO, bool PROLONG, bool RESTRICT>
+hipError_t sweep(MgHierarchy &H, int l, hipStream_t s) {
+  const MgGrid g = grid_of(H, l);
+  const int ntx = (g.mx + kSwX - 1) / kSwX, nty = (g.my + kSwY - 1) / kSwY;
+  const float *uc = PROLONG ? H.u[l + 1] : nullptr;
+  float *fc = RESTRICT ? H.f[l + 1] : nullptr;
+  if ((long long)ntx * nty * ((g.mz + 7) / 8) >= 512)
+    mg_sweep_kernel<8, ZERO, PROLONG, RESTRICT><<<ntx * nty * ((g.mz + 7) / 8), kSwNT, 0, s>>>(
+        H.r[l], H.u[l], H.f[l], uc, fc, g, ntx, nty);
+  else
+    mg_sweep_kernel<4, ZERO, PROLONG, RESTRICT><<<ntx * nty * ((g.mz + 3) / 4), kSwNT, 0, s>>>(
+        H.r[l], H.u[l], H.f[l], uc, fc, g, ntx, nty);
+  std::swap(H.u[l], H.r[l]);
+  return hipGetLastError();
+}
+
+__global__ void mg_zero_kernel(float *u, int n) {
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx < n) u[idx] = 0.f;
+}
+
+hipError_t clear_level(const MgHierarchy &H, int l, hipStream_t s) {
+  const int n = H.m[l][0] * H.m[l][1] * H.m[l][2];
+  mg_zero_kernel<<<blocks_for(n), 256, 0, s>>>(H.u[l], n);
+  return hipGetLastError();
+}
+
+// A V(nu1, nu2) cycle from level l down; zero: u starts from 0 (its array need
+// not be cleared).
+hipError_t vcycle(MgHierarchy &H, int l, int nu1, int nu2, bool zero, hipStream_t s) {
   const MgGrid g = grid_of(H, l);
   const int n = g.mx * g.my * g.mz;
+  hipError_t e = hipSuccess;
   if (l > 0 && H.levels - l >= 2 && small_from(H, l)) {
     MgSmall S;
     S.levels = H.levels - l;
@@ -453,17 +723,38 @@ hipError_t vcycle(const MgHierarchy &H, int l, int nu1, int nu2, hipStream_t s) 
       mg_coarsest_kernel<<<1, threads, 0, s>>>(H.u[l], H.f[l], g, n <= 64 ? 30 : 60);
       return hipGetLastError();
     }
+    if (zero && (e = clear_level(H, l, s)) != hipSuccess) return e;
     return smooth(H, l, 60, s);
   }
-  hipError_t e = smooth(H, l, nu1, s);
-  if (e != hipSuccess) return e;
-  mg_restrict_kernel<<<blocks_for(n / 8), 256, 0, s>>>(H.f[l + 1], H.u[l + 1], H.u[l], H.f[l], g);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = vcycle(H, l + 1, nu1, nu2, s)) != hipSuccess) return e;
-  mg_prolong_kernel<<<blocks_for(n / 2), 256, 0, s>>>(H.u[l], H.u[l + 1], g.mx, g.my, g.mz, g.px,
-                                                      g.py, g.pz);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  return smooth(H, l, nu2, s);
+  // Every axis of a level above the last is even.
+  int pre = nu1;
+  bool restricted = false;
+  if (zero && pre == 1) {
+    if ((e = sweep<true, false, true>(H, l, s)) != hipSuccess) return e;
+    restricted = true;
+    pre = 0;
+  } else if (zero && pre > 1) {
+    if ((e = sweep<true, false, false>(H, l, s)) != hipSuccess) return e;
+    --pre;
+  } else if (zero) {
+    if ((e = clear_level(H, l, s)) != hipSuccess) return e;
+  }
+  for (; pre > 0; --pre)
+    if ((e = sweep<false, false, false>(H, l, s)) != hipSuccess) return e;
+  if (!restricted) {
+    mg_restrict_kernel<<<blocks_for(n / 8), 256, 0, s>>>(H.f[l + 1], H.u[l], H.f[l], g);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  if ((e = vcycle(H, l + 1, nu1, nu2, true, s)) != hipSuccess) return e;
+  if (nu2 < 1) {
+    mg_prolong_kernel<<<blocks_for(n / 8), 256, 0, s>>>(H.u[l], H.u[l + 1], g.mx, g.my, g.mz,
+                                                        g.px, g.py, g.pz);
+    return hipGetLastError();
+  }
+  if ((e = sweep<false, true, false>(H, l, s)) != hipSuccess) return e;
+  for (int q = 1; q < nu2; ++q)
+    if ((e = sweep<false, false, false>(H, l, s)) != hipSuccess) return e;
+  return hipSuccess;
 }
 
 // Per-block sums of f (at most kMgMeanBlocks blocks), then f -= their total / n:
@@ -473,6 +764,8 @@ __global__ void __launch_bounds__(256) mg_sum_kernel(const float *__restrict__ f
                                                      double *__restrict__ part) {
   __shared__ double sc[4];
   double s = 0.0;
+  // Eight loads in flight, added in order.
+#pragma unroll 8
   for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) s += (double)f[i];
   s = block_sum<4>(s, sc);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
@@ -486,11 +779,6 @@ __global__ void __launch_bounds__(256) mg_center_kernel(float *__restrict__ f, i
   s = block_sum<4>(s, sc);
   const float m = (float)(s / n);
   for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) f[i] -= m;
-}
-
-__global__ void mg_zero_kernel(float *u, int n) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx < n) u[idx] = 0.f;
 }
 
 __global__ void __launch_bounds__(256) mg_pool_split_kernel(const float *__restrict__ r,
@@ -511,43 +799,41 @@ __global__ void __launch_bounds__(256) mg_pool_split_kernel(const float *__restr
   f0[idx] = 0.125f * t;
 }
 
-// The trilinear interpolation of the level-0 solution onto the fine grid,
-// stored colour-split (the first FP32 correction solve's starting iterate):
-// one thread per pair of cells (2c, 2c + 1) of a row, which are one red and
-// one black cell, so both halves of the split array are written coalesced;
-// 2D block (64 x 4) over (c, j), blockIdx.z = k: no 64-bit index division.
-__global__ void __launch_bounds__(256) mg_prolong_split_kernel(float *__restrict__ e,
-                                                               const float *__restrict__ u0,
-                                                               int nx, int ny, int nz, int px,
-                                                               int py, int pz) {
-  const int hx = nx / 2;
-  const int c = blockIdx.x * 64 + threadIdx.x;
-  const int j = blockIdx.y * 4 + threadIdx.y, k = blockIdx.z;
-  if (c >= hx || j >= ny) return;
-  const size_t half = (size_t)nx * ny * nz / 2;
-  const size_t o = (size_t)hx * (j + (size_t)ny * k) + c;
-  const int q = (j + k) & 1;
-  const int cx = nx / 2, cy = ny / 2, cz = nz / 2;
-  int y0, y1, z0, z1;
-  float wy, wz;
-  mg_axis(j, cy, py, y0, y1, wy);
-  mg_axis(k, cz, pz, z0, z1, wz);
-  auto cv = [&](int a, int b, int d) {
-    return u0[(size_t)a + (size_t)cx * (b + (size_t)cy * d)];
-  };
-  auto at = [&](int i) {
-    int x0, x1;
-    float wx;
-    mg_axis(i, cx, px, x0, x1, wx);
-    return (1.f - wz) * ((1.f - wy) * ((1.f - wx) * cv(x0, y0, z0) + wx * cv(x1, y0, z0)) +
-                         wy * ((1.f - wx) * cv(x0, y1, z0) + wx * cv(x1, y1, z0))) +
-           wz * ((1.f - wy) * ((1.f - wx) * cv(x0, y0, z1) + wx * cv(x1, y0, z1)) +
-                 wy * ((1.f - wx) * cv(x0, y1, z1) + wx * cv(x1, y1, z1)));
-  };
-  const float va = at(2 * c), vb = at(2 * c + 1);
-  // Red cell: i = 2c + q; black: i = 2c + 1 - q (entry c of its colour's row).
-  e[o] = q ? vb : va;
-  e[half + o] = q ? va : vb;
+// The trilinear interpolation of the level-0 solution onto the fine grid, one
+// thread per coarse cell, 64 x 4 of them per block and blockIdx.z = the plane.
+// SPLIT: stored colour-split (the first FP32 correction solve's starting
+// iterate; a pair of cells (2c, 2c + 1) of a row is one red and one black cell,
+// both entry c); else added to the FP64 field q.  A thread per pair of fine
+// cells was bound by its arithmetic (97 % VALU busy): 512x384x256 split 94 us.
+template <bool SPLIT>
+__global__ void __launch_bounds__(256) mg_prolong_top_kernel(float *__restrict__ e,
+                                                             double *__restrict__ q,
+                                                             const float *__restrict__ u0,
+                                                             int nx, int ny, int nz, int px,
+                                                             int py, int pz) {
+  const int cx = nx / 2, cy = ny / 2;
+  const int I = blockIdx.x * 64 + threadIdx.x;
+  const int J = blockIdx.y * 4 + threadIdx.y, K = blockIdx.z;
+  if (I >= cx || J >= cy) return;
+  float v[8];
+  mg_interp_cell(u0, I, J, K, cx, cy, nz / 2, px, py, pz, v);
+  const size_t half = (size_t)cx * ny * nz;
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    const size_t row = (size_t)(2 * J + (n & 1)) + (size_t)ny * (2 * K + (n >> 1));
+    if (SPLIT) {
+      // Red cell: i = 2 I + (j + k) % 2.
+      const bool odd = ((n & 1) + (n >> 1)) & 1;
+      e[cx * row + I] = odd ? v[2 * n + 1] : v[2 * n];
+      e[half + cx * row + I] = odd ? v[2 * n] : v[2 * n + 1];
+    } else {
+      double2 *o = reinterpret_cast<double2 *>(q + (size_t)nx * row) + I;
+      double2 w = *o;
+      w.x = w.x + (double)v[2 * n];
+      w.y = w.y + (double)v[2 * n + 1];
+      *o = w;
+    }
+  }
 }
 
 }  // namespace
@@ -562,9 +848,18 @@ hipError_t mg_pool_split(const float *r, float *f0, int nx, int ny, int nz, hipS
 hipError_t mg_prolong_split(float *e, const float *u0, int nx, int ny, int nz, const int per[3],
                             hipStream_t s) {
   if (nx % 2 || ny % 2 || nz % 2) return hipErrorInvalidValue;
-  dim3 grid((nx / 2 + 63) / 64, (ny + 3) / 4, nz);
-  mg_prolong_split_kernel<<<grid, dim3(64, 4), 0, s>>>(e, u0, nx, ny, nz, per[0], per[1],
-                                                       per[2]);
+  const dim3 grid((nx / 2 + 63) / 64, (ny / 2 + 3) / 4, nz / 2);
+  mg_prolong_top_kernel<true><<<grid, dim3(64, 4), 0, s>>>(e, nullptr, u0, nx, ny, nz, per[0],
+                                                           per[1], per[2]);
+  return hipGetLastError();
+}
+
+hipError_t mg_prolong_add(double *q, const float *u0, int nx, int ny, int nz, const int per[3],
+                          hipStream_t s) {
+  if (nx % 2 || ny % 2 || nz % 2) return hipErrorInvalidValue;
+  const dim3 grid((nx / 2 + 63) / 64, (ny / 2 + 3) / 4, nz / 2);
+  mg_prolong_top_kernel<false><<<grid, dim3(64, 4), 0, s>>>(nullptr, q, u0, nx, ny, nz, per[0],
+                                                            per[1], per[2]);
   return hipGetLastError();
 }
 
@@ -573,12 +868,12 @@ hipError_t mg_seed_from_level1(const MgHierarchy &H, hipStream_t s) {
   const MgGrid g = grid_of(H, 0);
   const int n0 = g.mx * g.my * g.mz;
   mg_zero_kernel<<<(n0 + 255) / 256, 256, 0, s>>>(H.u[0], n0);
-  mg_prolong_kernel<<<blocks_for(n0 / 2), 256, 0, s>>>(H.u[0], H.u[1], g.mx, g.my, g.mz, g.px,
+  mg_prolong_kernel<<<blocks_for(n0 / 8), 256, 0, s>>>(H.u[0], H.u[1], g.mx, g.my, g.mz, g.px,
                                                        g.py, g.pz);
   return hipGetLastError();
 }
 
-hipError_t mg_solve(const MgHierarchy &H, int cycles, int nu1, int nu2, hipStream_t s,
+hipError_t mg_solve(MgHierarchy &H, int cycles, int nu1, int nu2, hipStream_t s,
                     bool from_zero) {
   if (H.levels < 1) return hipErrorInvalidValue;
   if ((long long)H.m[0][0] * H.m[0][1] * H.m[0][2] >= (1LL << 31)) return hipErrorInvalidValue;
@@ -594,9 +889,10 @@ hipError_t mg_solve(const MgHierarchy &H, int cycles, int nu1, int nu2, hipStrea
     mg_sum_kernel<<<nb, 256, 0, s>>>(H.f[0], n0, part);
     mg_center_kernel<<<nb, 256, 0, s>>>(H.f[0], n0, part, nb);
   }
-  if (from_zero) mg_zero_kernel<<<(n0 + 255) / 256, 256, 0, s>>>(H.u[0], n0);
   hipError_t e = hipGetLastError();
-  for (int c = 0; c < cycles && e == hipSuccess; ++c) e = vcycle(H, 0, nu1, nu2, s);
+  if (cycles < 1 && from_zero) e = clear_level(H, 0, s);
+  for (int c = 0; c < cycles && e == hipSuccess; ++c)
+    e = vcycle(H, 0, nu1, nu2, from_zero && c == 0, s);
   return e;
 }
 
