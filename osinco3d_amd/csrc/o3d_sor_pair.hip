@@ -35,11 +35,13 @@
 // side.  So tiles are handed to the XCDs in
 // contiguous runs (FP32 256^3: 90 us per launch in the plain order, 54 us so),
 // one block runs per CU (FP64 256^3: 105 us with one block of 384 threads per
-// CU, 131 us with two; 512 and 768 threads 128 and 125 us), and loads are
-// issued two planes ahead (three: no gain).  Per two iterations, launches of
+// CU, 131 us with two), loads are issued two planes ahead (three: no gain), and
+// every second launch marches from the other end, towards what the last one
+// left in the Infinity Cache (FP32 512x384x256 173 -> 156 us, FP64 320^3 199 ->
+// 188).  Per two iterations, launches of
 // one colour in place / this kernel: FP64 64^3 27.1 / 15.2 us, 128^3 36.7 /
-// 26.0, 256^3 186 / 107, 512x384x256 696 / 310; FP32 64^3 27.2 / 14.5, 256^3
-// 98 / 54, 384x256x128 93 / 38, 512x384x256 327 / 174 (the figures hold the
+// 24.2, 256^3 186 / 106, 512x384x256 696 / 306; FP32 64^3 27.2 / 14.5, 256^3
+// 98 / 54, 384x256x128 93 / 38, 512x384x256 327 / 156 (the figures hold the
 // host's share of a batch of launches, about 3 us).
 #include <algorithm>
 #include <utility>
@@ -57,6 +59,10 @@ struct PairShape;
 template <>
 struct PairShape<double, 0> {
   static constexpr int LX = 32, RY = 2, NT = 384, PAD = 40000;
+};
+template <>
+struct PairShape<double, 1> {
+  static constexpr int LX = 32, RY = 2, NT = 512, PAD = 20000;
 };
 template <>
 struct PairShape<float, 0> {
@@ -233,7 +239,9 @@ __device__ __forceinline__ bool pair_group(std::integer_sequence<int, K...>, int
   return ((m + K <= last && (f(m + K, PIC<K>{}), true)) && ...);
 }
 
-template <typename T, int SHAPE>
+// FLIP: the march runs through the planes backwards in an even number of them
+// (virtual plane v is plane nz - 1 - v, of the other parity).
+template <typename T, int SHAPE, int FLIP>
 __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
     sor_pair_kernel(const SorPairArgs<T> a) {
   using Shape = PairShape<T, SHAPE>;
@@ -258,7 +266,10 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
   const int nx = a.nx, ny = a.ny, nz = a.nz, hx = nx / 2;
   const int tile = pair_tile(blockIdx.x, gridDim.x);
   const int tix = tile % a.ntx, rr = tile / a.ntx;
-  const int tiy = rr % a.nty, tiz = rr / a.nty;
+  // Every second launch marches the other way: what the last one touched last
+  // (and the Infinity Cache still holds) is read first.
+  const bool rev = a.launch & 1;
+  const int tiy = rr % a.nty, tiz = rev ? a.ntz - 1 - rr / a.nty : rr / a.nty;
   const int c0 = tix * (LX - 4), y0 = tiy * (TY - 8), z0 = tiz * a.zc;
   const int z1 = min(z0 + a.zc, nz);
   const T ox = T(a.ox), oy = T(a.oy), oz = T(a.oz), A = T(a.A), invA = T(1.0 / a.A);
@@ -300,14 +311,15 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
   const int zs = a.per[2] ? 1 : -1, zlo = a.per[2] ? nz : 0, zhi = a.per[2] ? -nz : 2 * (nz - 1);
   auto zsoff = [&](int q) {
     const int z = z0 - 4 + q, im = zs * z + (z < 0 ? zlo : zhi);
-    return planeB * (unsigned)(z < 0 || z >= nz ? im : z);
+    const int v = z < 0 || z >= nz ? im : z;
+    return planeB * (unsigned)(rev ? nz - 1 - v : v);
   };
   auto load_p = [&](int q, auto SL) __attribute__((always_inline)) {
     constexpr int sl = decltype(SL)::value % NR;
     const unsigned so = zsoff(q);
 #pragma unroll
     for (int r = 0; r < RY; ++r) {
-      const bool odd = (r + sl) & 1;
+      const bool odd = (r + sl + FLIP) & 1;
       R[sl][r] = pload<T>(rin, odd ? vR[r] : vL[r], so);
       B[sl][r] = pload<T>(rin, odd ? vL[r] : vR[r], so + halfB);
     }
@@ -317,7 +329,7 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
     const unsigned so = zsoff(q);
 #pragma unroll
     for (int r = 0; r < RY; ++r) {
-      const bool odd = (r + sl) & 1;
+      const bool odd = (r + sl + FLIP) & 1;
       fR[sl][r] = pload<T>(rrh, odd ? vR[r] : vL[r], so);
       fB[sl][r] = pload<T>(rrh, odd ? vL[r] : vR[r], so + halfB);
     }
@@ -337,7 +349,7 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
     for (int r = 0; r < RY; ++r) {
       // Node on the left of its pair: its other x neighbour is in the pair
       // before; on the right: in the pair after.
-      const bool right = ((r + sl + col) & 1) != 0;
+      const bool right = ((r + sl + col + FLIP) & 1) != 0;
       const T side = right ? lane_next<1>(Y[sl][r]) : lane_next<0>(Y[sl][r]);
       const T ym = r == 0 ? lo : Y[sl][r == 0 ? 0 : r - 1];
       const T yp = r == RY - 1 ? hi : Y[sl][r == RY - 1 ? r : r + 1];
@@ -451,7 +463,7 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
     publish(1 - b, K);
     if constexpr (!first || k >= 6) {
       constexpr int sl = (k + NR - 2) % NR;
-      const unsigned so = planeB * (unsigned)(z0 - 6 + m);
+      const unsigned so = planeB * (unsigned)(rev ? nz - 1 - (z0 - 6 + m) : z0 - 6 + m);
 #pragma unroll
       for (int r = 0; r < RY; ++r)
         if (own[r]) {
@@ -528,7 +540,7 @@ int pair_slots() {
   static const int slots = [] {
     int per_cu = 0, dev = 0, cus = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, sor_pair_kernel<T, SHAPE>, PairShape<T, SHAPE>::NT,
+            &per_cu, sor_pair_kernel<T, SHAPE, 0>, PairShape<T, SHAPE>::NT,
             PairShape<T, SHAPE>::PAD) != hipSuccess ||
         hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
@@ -541,9 +553,10 @@ int pair_slots() {
 }
 
 // Tiles of one shape: the even chunk of planes with the least
-// rounds * (planes + 6 of the pipeline + 3 of prologue).
+// rounds * (planes + 6 of the pipeline + 3 of prologue), the plane steps of the
+// launch, which it returns.
 template <typename T, int SHAPE>
-void pair_tiling(SorPairArgs<T> &a) {
+double pair_tiling(SorPairArgs<T> &a) {
   using Shape = PairShape<T, SHAPE>;
   constexpr int OX = Shape::LX - 4, OY = Shape::NT / Shape::LX * Shape::RY - 8;
   a.shape = SHAPE;
@@ -562,29 +575,49 @@ void pair_tiling(SorPairArgs<T> &a) {
       a.ntz = ntz;
     }
   }
+  return best;
 }
 
 template <typename T, int SHAPE>
 void pair_launch(const SorPairArgs<T> &a, hipStream_t s) {
   using Shape = PairShape<T, SHAPE>;
-  sor_pair_kernel<T, SHAPE><<<a.ntx * a.nty * a.ntz, Shape::NT, Shape::PAD, s>>>(a);
+  const int blocks = a.ntx * a.nty * a.ntz;
+  if ((a.launch & 1) && a.nz % 2 == 0)
+    sor_pair_kernel<T, SHAPE, 1><<<blocks, Shape::NT, Shape::PAD, s>>>(a);
+  else
+    sor_pair_kernel<T, SHAPE, 0><<<blocks, Shape::NT, Shape::PAD, s>>>(a);
 }
 
 }  // namespace
 
 size_t sor_pair_slot_words() { return (size_t)kPairSets * 2 * kPairSlots * kPairStride; }
 
+// Both buffers and the rhs stay in the 256 MB of the Infinity Cache.
+template <typename T>
+bool pair_cached(const SorPairArgs<T> &a) {
+  return 3ll * (long long)sizeof(T) * a.nx * a.ny * a.nz <= (256ll << 20);
+}
+
+// FP64: 8 waves own 24 of 32 rows, 6 waves 16 of 24, for a plane step of 0.90 and
+// 0.86 us, so 8 waves take fewer steps in most grids; beyond the cache the smaller
+// tile's halos are found in L2 more often.  Per launch, 6 / 8 waves: 64^3 15.4 /
+// 16.1 us, 128^3 26.0 / 24.2, 192^3 49.5 / 39.9, 208^3 59 / 49, then 256^3 106 /
+// 114, 320^3 188 / 198, 512x384x256 306 / 378.
 template <>
-void sor_pair_tiling<double>(SorPairArgs<double> &a) { pair_tiling<double, 0>(a); }
-// FP32: the narrow tile while both buffers and the rhs stay in the 256 MB of
-// the Infinity Cache, the wide one (longer rows, fewer x halos) beyond.  Per
+void sor_pair_tiling<double>(SorPairArgs<double> &a) {
+  const double six = 0.86 * pair_tiling<double, 0>(a);
+  if (!pair_cached(a)) return;
+  SorPairArgs<double> b = a;
+  if (0.90 * pair_tiling<double, 1>(b) < six) a = b;
+}
+// FP32: the narrow tile in the cache, the wide one (longer rows, fewer x halos)
+// beyond.  Per
 // launch, narrow / wide: 192^3 31.5 / 32.3 us, 256^3 53.8 / 64.4, 384x256x128
 // 39.8 / 49.5, then 288^3 96.9 / 87.1, 320^3 114 / 107, 512x384x256 219 / 174.
 template <>
 void sor_pair_tiling<float>(SorPairArgs<float> &a) {
-  const long long bytes = 12ll * a.nx * a.ny * a.nz;
-  if (bytes > (256ll << 20)) pair_tiling<float, 1>(a);
-  else pair_tiling<float, 0>(a);
+  if (pair_cached(a)) pair_tiling<float, 0>(a);
+  else pair_tiling<float, 1>(a);
 }
 
 template <typename T>
@@ -599,12 +632,8 @@ hipError_t launch_sor_pair(const SorPairArgs<T> &a, hipStream_t s) {
   if (a.nx % 2 != 0 || a.nx < 6 || a.ny < 6 || a.nz < 6 ||
       a.zc % 2 != 0 || !sor_buffer_fits<T, T>(a.nx, a.ny, a.nz))
     return hipErrorInvalidValue;
-  if constexpr (sizeof(T) == 4) {
-    if (a.shape == 1) pair_launch<T, 1>(a, s);
-    else pair_launch<T, 0>(a, s);
-  } else {
-    pair_launch<T, 0>(a, s);
-  }
+  if (a.shape == 1) pair_launch<T, 1>(a, s);
+  else pair_launch<T, 0>(a, s);
   return hipGetLastError();
 }
 
