@@ -426,6 +426,44 @@ __global__ void __launch_bounds__(256) mg_prolong_kernel(float *__restrict__ u,
   }
 }
 
+// An odd axis that wraps puts two cells of one colour beside each other, so a
+// colour relaxed in place would depend on which wave of the block comes first.
+// There all cells of a colour are read before any is written (with one barrier
+// more); elsewhere the cells of a colour do not meet.
+__device__ __forceinline__ bool mg_colours_meet(const MgGrid &g) {
+  return ((g.mx & g.px) | (g.my & g.py) | (g.mz & g.pz)) & 1;
+}
+
+// One colour of a level of at most kMgCoarsestCells cells in LDS, a cell per
+// thread at a time, by a block of at least 64 threads (1024 above 64 cells).
+__device__ __forceinline__ void lds_relax_any(float *u, const float *f, const MgGrid &g,
+                                              int colour, bool meet) {
+  const int n = g.mx * g.my * g.mz;
+  constexpr int kPer = kMgCoarsestCells / 1024;
+  float v[kPer];
+#pragma unroll
+  for (int s = 0; s < kPer; ++s) {
+    const int q = threadIdx.x + s * blockDim.x;
+    if (q < n) {
+      const int row = q / g.mx, i = q - row * g.mx;
+      const int k = row / g.my, j = row - k * g.my;
+      v[s] = u[q];
+      if (((i + j + k) & 1) == colour) {
+        v[s] = (f[q] - mg_lap_off(u, g, i, j, k)) * g.invd;
+        if (!meet) u[q] = v[s];
+      }
+    }
+  }
+  __syncthreads();
+  if (!meet) return;
+#pragma unroll
+  for (int s = 0; s < kPer; ++s) {
+    const int q = threadIdx.x + s * blockDim.x;
+    if (q < n) u[q] = v[s];
+  }
+  __syncthreads();
+}
+
 // The coarsest level: `sweeps` red-black Gauss-Seidel sweeps from u = 0 by
 // one block, the level staged in LDS.
 __global__ void __launch_bounds__(1024) mg_coarsest_kernel(float *__restrict__ u,
@@ -438,15 +476,9 @@ __global__ void __launch_bounds__(1024) mg_coarsest_kernel(float *__restrict__ u
     sf[q] = f[q];
   }
   __syncthreads();
+  const bool meet = mg_colours_meet(g);
   for (int s = 0; s < sweeps; ++s)
-    for (int colour = 0; colour < 2; ++colour) {
-      for (int q = threadIdx.x; q < n; q += blockDim.x) {
-        const int row = q / g.mx, i = q - row * g.mx;
-        const int k = row / g.my, j = row - k * g.my;
-        if (((i + j + k) & 1) == colour) mg_relax(su, sf, g, i, j, k, q);
-      }
-      __syncthreads();
-    }
+    for (int colour = 0; colour < 2; ++colour) lds_relax_any(su, sf, g, colour, meet);
   for (int q = threadIdx.x; q < n; q += blockDim.x) u[q] = su[q];
 }
 
@@ -479,17 +511,10 @@ struct SmallDiv {
 
 __device__ __forceinline__ void lds_smooth(float *u, const float *f, const MgGrid &g,
                                            int sweeps) {
+  const bool meet = mg_colours_meet(g);
   if (g.mx & 1) {
-    const int n = g.mx * g.my * g.mz;
     for (int s = 0; s < sweeps; ++s)
-      for (int colour = 0; colour < 2; ++colour) {
-        for (int q = threadIdx.x; q < n; q += kMgSmallThreads) {
-          const int row = q / g.mx, i = q - row * g.mx;
-          const int k = row / g.my, j = row - k * g.my;
-          if (((i + j + k) & 1) == colour) mg_relax(u, f, g, i, j, k, q);
-        }
-        __syncthreads();
-      }
+      for (int colour = 0; colour < 2; ++colour) lds_relax_any(u, f, g, colour, meet);
     return;
   }
   // Per cell pair of this thread: its offset and, for both of its cells, the
@@ -512,14 +537,22 @@ __device__ __forceinline__ void lds_smooth(float *u, const float *f, const MgGri
   }
   for (int sw = 0; sw < sweeps; ++sw)
     for (int colour = 0; colour < 2; ++colour) {
+      float v[kMgSmallPer];
 #pragma unroll
       for (int s = 0; s < kMgSmallPer; ++s)
         if (threadIdx.x + s * kMgSmallThreads < nh) {
           const int right = (base[s] + colour) & 1, l = base[s] >> 1, q = l + right;
           const float sx = u[right ? l : l + oxl[s]] + u[right ? l + oxr[s] : l + 1];
-          u[q] = mg_relax_value(f[q], sx, u[q + oym[s]] + u[q + oyp[s]],
+          v[s] = mg_relax_value(f[q], sx, u[q + oym[s]] + u[q + oyp[s]],
                                 u[q + ozm[s]] + u[q + ozp[s]], g);
+          if (!meet) u[q] = v[s];
         }
+      __syncthreads();
+      if (!meet) continue;
+#pragma unroll
+      for (int s = 0; s < kMgSmallPer; ++s)
+        if (threadIdx.x + s * kMgSmallThreads < nh)
+          u[(base[s] >> 1) + ((base[s] + colour) & 1)] = v[s];
       __syncthreads();
     }
 }
