@@ -729,7 +729,7 @@ extern "C" int o3d_nu_t(double *nu_t, const double *ux, const double *uy, const 
     CHK(s.scratch(n, &f1[c]));
   }
   const double *f2[3] = {nullptr, nullptr, nullptr};
-  const Tiling tl = make_tiling(nx, ny, nz);
+  const Tiling tl = predict_tiling<double>(nx, ny, nz, true);
   FieldPartial *part, *fin;
   CHK(s.scratch(tl.blocks(), &part));
   CHK(s.scratch(1, &fin));
@@ -793,7 +793,7 @@ extern "C" int o3d_predict_velocity(double *ux_pred, double *uy_pred, double *uz
   double *f1[3];
   const double *f2[3], *f3[3];
   for (int c = 0; c < 3; ++c) { f1[c] = F[c]; f2[c] = F[c] + n; f3[c] = F[c] + 2 * n; }
-  const Tiling tl = make_tiling(nx, ny, nz);
+  const Tiling tl = predict_tiling<double>(nx, ny, nz, les);
   FieldPartial *part;
   CHK(s.scratch(tl.blocks(), &part));
   const double h[3] = {dx, dy, dz};

@@ -103,6 +103,17 @@ def test_nu_t(orc, bc):
     assert st[0] == ref[0] and st[1] == ref[1] and np.array_equal(st[3:], ref[3:])
 
 
+def test_nu_t_statistics_cover_every_chunk(orc):
+    # Several z chunks of the kernel's own tiling: its block records are
+    # allocated and reduced for that tiling.
+    ux, uy, uz = rand_fields((64, 16, 64), 3, seed=10)
+    d = (0.2, 0.21, 0.19)
+    out = np.empty_like(ux)
+    st = capi.nu_t(out, ux, uy, uz, d, 0.17, 0.2, BCS[0])
+    ref = orc.function_stats(orc.nu_t(ux, uy, uz, d, 0.17, 0.2, BCS[0]))
+    assert st[0] == ref[0] and st[1] == ref[1] and np.array_equal(st[3:], ref[3:])
+
+
 @pytest.mark.parametrize("bc", BCS)
 @pytest.mark.parametrize("itscheme", [1, 2, 3])
 @pytest.mark.parametrize("iles", [0, 1])
