@@ -49,7 +49,7 @@ Tiling make_tiling_slots(int nx, int ny, int nz, int slots) {
   if (slots <= 0) return make_tiling(nx, ny, nz);
   double best = 1e30;
   int best_ntz = 1;
-  for (int ntz = 1; ntz <= std::max(1, nz / 8); ++ntz) {
+  for (int ntz = 1; ntz <= std::max(1, nz / 2); ++ntz) {
     const int zc = (nz + ntz - 1) / ntz;
     const int n_t = (nz + zc - 1) / zc;
     const int rounds = (layer * n_t + slots - 1) / slots;
