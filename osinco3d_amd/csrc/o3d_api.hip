@@ -326,6 +326,7 @@ struct SorRun {
     HIPCHK(launch_sor_pair_init<T>(pa, omega, g_stream));
     expect = std::min(std::max(1, expect), pa.kmax);
     int batch = (expect + 1) / 2 + 1 + ((expect & 1) && expect < pa.kmax ? 1 : 0);
+    if (pa.whole) batch = 1;
     pa.launch = 0;
     bool first = true;
     while (true) {
@@ -345,7 +346,8 @@ struct SorRun {
       HIPCHK(hipStreamSynchronize(g_stream));
       // Timed are launches that ran two iterations each: a batch the solve
       // did not end in, or the Gauss-Seidel opening.
-      const int timed = !hst->done ? batch - 1
+      const int timed = pa.whole     ? 0
+                        : !hst->done ? batch - 1
                                    : (mid_set && hst->sweeps >= pa.gs ? pa.gs / 2 - 1 : 0);
       if (timed > 0) {
         float ms = 0.f;
@@ -358,7 +360,7 @@ struct SorRun {
       // At most two launches per iteration (a pair and its first sweep again).
       if (pa.launch > 2 * pa.kmax + 16) return fail("SOR state did not close after kmax");
       first = false;
-      batch = 8;
+      batch = pa.whole ? 1 : 8;
     }
     *sweeps_out = hst->sweeps;
     return 0;
@@ -815,7 +817,7 @@ extern "C" int o3d_predict_velocity(double *ux_pred, double *uy_pred, double *uz
 // start iterate) and b1 and the split rhs.
 template <typename T>
 SorPairArgs<T> pair_args(const SorArgs<T, T> &a, T *b0, T *b1, const T *rhs,
-                         unsigned long long *dslot) {
+                         unsigned long long *dslot, bool whole = true) {
   SorPairArgs<T> pa{};
   pa.buf[0] = b0;
   pa.buf[1] = b1;
@@ -825,12 +827,15 @@ SorPairArgs<T> pair_args(const SorArgs<T, T> &a, T *b0, T *b1, const T *rhs,
   pa.nx = a.nx; pa.ny = a.ny; pa.nz = a.nz;
   for (int q = 0; q < 3; ++q) pa.per[q] = a.per[q];
   pa.ox = a.ox; pa.oy = a.oy; pa.oz = a.oz; pa.A = a.A;
+  pa.invA = 1.0 / a.A;
   pa.eps = a.eps;
+  pa.eps_stag = a.eps / 1000.0;
   pa.factor = a.factor;
   pa.kmax = a.kmax;
   pa.idyn = a.idyn;
   pa.gs = a.gs;
-  sor_pair_tiling<T>(pa);
+  pa.whole = whole && sor_whole<T>(pa);
+  if (!pa.whole) sor_pair_tiling<T>(pa);
   return pa;
 }
 
@@ -2913,7 +2918,7 @@ extern "C" int o3d_solver_sor_period(void *handle, int iterations, double *us) {
   const int launches = std::max(2, (iterations + 1) / 2);
   sor_args_common<float, float>(S, r.a, S.R, S.st, 2 * launches);
   r.a.eps = 0.0;  // never converged, never stagnant: every launch sweeps
-  r.pa = pair_args<float>(r.a, S.E[0], S.E[1], S.R, S.dslot);
+  r.pa = pair_args<float>(r.a, S.E[0], S.E[1], S.R, S.dslot, false);
   HIPCHK(launch_sor_pair_init<float>(r.pa, S.omega, g_stream));
   hipEvent_t e0 = S.ev[0], e1 = S.ev[1];
   for (; r.pa.launch < launches; ++r.pa.launch) {

@@ -84,10 +84,29 @@ __device__ __forceinline__ double wave_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, O3D_WAVE);
   return v;
 }
+// Lanes of a DPP pattern's source, a lane itself where the pattern has none.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_lane(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const int l = (int)(unsigned)b, h = (int)(unsigned)(b >> 32);
+  const int lo = __builtin_amdgcn_update_dpp(l, l, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(h, h, CTRL, ROWS, 0xf, false);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
+                                          (unsigned)lo));
+}
+// By DPP (all lanes active): six steps through the LDS cross-lane path cost
+// 0.3 us, which every launch of the SOR kernels spends three times.
 __device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, O3D_WAVE));
-  return v;
+  v = fmax(v, dpp_lane<0x111, 0xf>(v));  // row_shr:1, 2, 4, 8
+  v = fmax(v, dpp_lane<0x112, 0xf>(v));
+  v = fmax(v, dpp_lane<0x114, 0xf>(v));
+  v = fmax(v, dpp_lane<0x118, 0xf>(v));
+  v = fmax(v, dpp_lane<0x142, 0xa>(v));  // row_bcast:15, row_bcast:31
+  v = fmax(v, dpp_lane<0x143, 0xc>(v));
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, 63);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), 63);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 __device__ __forceinline__ double wave_min(double v) {
 #pragma unroll

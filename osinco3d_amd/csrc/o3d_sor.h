@@ -116,8 +116,9 @@ struct SorPairArgs {
   unsigned long long *dslot;  // sor_pair_slot_words() words: dmax of the last launches
   int nx, ny, nz, per[3];
   int shape, ntx, nty, ntz, zc;
-  double ox, oy, oz, A;
-  double eps, factor;
+  bool whole;  // sor_whole
+  double ox, oy, oz, A, invA;      // invA = 1 / A
+  double eps, eps_stag, factor;    // eps_stag = eps / 1000, the stagnation rule's
   int kmax, idyn, gs;
   int launch;
 };
@@ -127,6 +128,10 @@ bool sor_split_supported(int nx) { return nx % (sizeof(T) == 8 ? 2 : 8) == 0; }
 size_t sor_pair_slot_words();
 template <typename T>
 void sor_pair_tiling(SorPairArgs<T> &a);
+// True, with the shape set, where the grid fits one block: a launch then runs all
+// iterations of the solve (at most 512; the next launch goes on).
+template <typename T>
+bool sor_whole(SorPairArgs<T> &a);
 template <typename T>
 hipError_t launch_sor_pair_init(const SorPairArgs<T> &a, double omega, hipStream_t s);
 template <typename T>

@@ -66,7 +66,7 @@ struct PairShape<double, 1> {
 };
 template <>
 struct PairShape<float, 0> {
-  static constexpr int LX = 32, RY = 2, NT = 768, PAD = 0;
+  static constexpr int LX = 32, RY = 2, NT = 768, PAD = 30000;
 };
 template <>
 struct PairShape<float, 1> {
@@ -147,6 +147,17 @@ __device__ __forceinline__ T pload(__amdgpu_buffer_rsrc_t r, unsigned voff, unsi
 }
 
 template <typename T>
+__device__ __forceinline__ void pstore(T v, __amdgpu_buffer_rsrc_t r, unsigned voff,
+                                       unsigned soff) {
+  if constexpr (sizeof(T) == 8) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, voff, soff, 0);
+  } else {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, voff, soff, 0);
+  }
+}
+
+template <typename T>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t pair_rsrc(const T *p, int n) {
   // At most INT_MAX bytes (sor_buffer_fits, checked by the launcher).
   return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0,
@@ -166,19 +177,19 @@ struct PairStep {
 // The reference's loop tail after iteration q with update d1 (the one before
 // it d0): true when the solve ends; om becomes omega of iteration q + 1.
 // Same rules and order as sor_decide_with of the single-iteration kernels.
-__device__ __forceinline__ bool pair_tail(int q, double d1, double d0, double eps,
-                                          double factor, int kmax, int idyn, int gs, double &om,
-                                          int &reason) {
+template <typename T>
+__device__ __forceinline__ bool pair_tail(int q, double d1, double d0, const SorPairArgs<T> &a,
+                                          double &om, int &reason) {
   reason = -1;
-  if (d1 < eps) reason = 0;
-  else if (fabs(d0 - d1) < eps / 1000.0) reason = 1;
+  if (d1 < a.eps) reason = 0;
+  else if (fabs(d0 - d1) < a.eps_stag) reason = 1;
   // No eps or stagnation exit inside the Gauss-Seidel opening.
-  if (reason >= 0) return q > gs;
-  if (q > 1 && idyn == 1) {
-    if (d1 > d0) om = om * (2.0 - factor);
-    else if (d1 < 0.1 * d0) om = fmin(om * factor, 2.0);
+  if (reason >= 0) return q > a.gs;
+  if (q > 1 && a.idyn == 1) {
+    if (d1 > d0) om = om * (2.0 - a.factor);
+    else if (d1 < 0.1 * d0) om = fmin(om * a.factor, 2.0);
   }
-  if (q + 1 > kmax) { reason = 2; return true; }
+  if (q + 1 > a.kmax) { reason = 2; return true; }
   return false;
 }
 
@@ -194,8 +205,7 @@ __device__ __forceinline__ PairStep pair_decide(const SorSched &P, double da, do
   if (P.n > 0) {
     double om = P.om_a;
     int reason;
-    const bool stop = pair_tail(P.it0, da, P.it0 == 1 ? 1609.0 : P.d_prev, a.eps, a.factor,
-                                a.kmax, a.idyn, a.gs, om, reason);
+    const bool stop = pair_tail(P.it0, da, P.it0 == 1 ? 1609.0 : P.d_prev, a, om, reason);
     if (stop && P.n == 2) {  // one iteration too many: the first alone
       s.n = 1;
       s.om_b = s.om_a;
@@ -212,7 +222,7 @@ __device__ __forceinline__ PairStep pair_decide(const SorSched &P, double da, do
     if (!stop && P.n == 2) {
       ++q;
       d = db;
-      end = pair_tail(q, db, da, a.eps, a.factor, a.kmax, a.idyn, a.gs, om, reason);
+      end = pair_tail(q, db, da, a, om, reason);
     }
     s.src = 1 - P.src;
     if (end) {
@@ -272,7 +282,7 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
   const int tiy = rr % a.nty, tiz = rev ? a.ntz - 1 - rr / a.nty : rr / a.nty;
   const int c0 = tix * (LX - 4), y0 = tiy * (TY - 8), z0 = tiz * a.zc;
   const int z1 = min(z0 + a.zc, nz);
-  const T ox = T(a.ox), oy = T(a.oy), oz = T(a.oz), A = T(a.A), invA = T(1.0 / a.A);
+  const T ox = T(a.ox), oy = T(a.oy), oz = T(a.oz), A = T(a.A), invA = T(a.invA);
 
   // Entries of the left and right node of this thread's pair, per row (they
   // differ only for mirror images, whose two nodes lie in two pairs).
@@ -467,18 +477,8 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
 #pragma unroll
       for (int r = 0; r < RY; ++r)
         if (own[r]) {
-          if constexpr (sizeof(T) == 8) {
-            typedef unsigned u2 __attribute__((ext_vector_type(2)));
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, R[sl][r]), rout, vL[r],
-                                                  so, 0);
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, B[sl][r]), rout, vL[r],
-                                                  so + halfB, 0);
-          } else {
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, R[sl][r]), rout,
-                                                  vL[r], so, 0);
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, B[sl][r]), rout,
-                                                  vL[r], so + halfB, 0);
-          }
+          pstore(R[sl][r], rout, vL[r], so);
+          pstore(B[sl][r], rout, vL[r], so + halfB);
         }
     }
     __syncthreads();
@@ -514,6 +514,124 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
       atomicMax(&a.dslot[((size_t)(a.launch % kPairSets) * 2 * kPairSlots +
                           (size_t)tid * kPairSlots + blockIdx.x % kPairSlots) * kPairStride],
                 (unsigned long long)__double_as_longlong(v));
+  }
+}
+
+// ------------------------------------------------------------- small grids
+// Whole iterations of a grid that fits one block's LDS, as many as the solve
+// takes (at most kBlockIters per launch, the state carried on in `sched`).  A
+// launch of the march costs 11 us however small its grid; here an iteration is two
+// barriers and the stop rule's block maximum.  A thread keeps PER pairs in
+// registers and, of each, the LDS places of its neighbours (16 bits each); every
+// half sweep reads the other colour from LDS, which bounds it together with the
+// FP64 unit of the one CU.
+// Same updates in the same order as sor_pair_kernel, and its stop rule after every
+// iteration.
+constexpr int kBlockNT = 1024, kBlockIters = 512;
+
+template <typename T, int PER>
+__global__ void __launch_bounds__(kBlockNT) sor_block_kernel(const SorPairArgs<T> a) {
+  constexpr int NP = PER * kBlockNT;
+  __shared__ T ex[2][NP];  // black, red
+  __shared__ double scr[2][kBlockNT / O3D_WAVE];
+  SorState *st = a.st;
+  if (st->done) return;
+  const SorSched P = st->sched[a.launch & 1];
+  const int src = P.src;
+  const int tid = threadIdx.x;
+  const int nx = a.nx, ny = a.ny, nz = a.nz, hx = nx / 2, np = hx * ny * nz;
+  const T ox = T(a.ox), oy = T(a.oy), oz = T(a.oz), A = T(a.A), invA = T(a.invA);
+  const T *in = a.buf[src];
+  T R[PER], B[PER], fR[PER], fB[PER];
+  // Entries of the other colour: y - 1 | y + 1, z - 1 | z + 1, the x neighbour
+  // outside the pair of the red | of the black node.
+  unsigned oy2[PER], oz2[PER], os2[PER];
+#pragma unroll
+  for (int m = 0; m < PER; ++m) {
+    const int p = tid + m * kBlockNT;
+    R[m] = B[m] = fR[m] = fB[m] = T(0);
+    oy2[m] = oz2[m] = os2[m] = 0;
+    if (p >= np) continue;
+    R[m] = in[p];
+    B[m] = in[np + p];
+    fR[m] = a.rhs[p];
+    fB[m] = a.rhs[np + p];
+    const int row = p / hx, c = p - row * hx, k = row / ny, j = row - k * ny;
+    const int yb = c + hx * ny * k, zb = c + hx * j;
+    oy2[m] = (unsigned)(yb + hx * pair_ghost(j - 1, ny, a.per[1])) |
+             (unsigned)(yb + hx * pair_ghost(j + 1, ny, a.per[1])) << 16;
+    oz2[m] = (unsigned)(zb + hx * ny * pair_ghost(k - 1, nz, a.per[2])) |
+             (unsigned)(zb + hx * ny * pair_ghost(k + 1, nz, a.per[2])) << 16;
+    const unsigned l = (unsigned)(hx * row + (pair_ghost(2 * c - 1, nx, a.per[0]) >> 1));
+    const unsigned r = (unsigned)(hx * row + (pair_ghost(2 * c + 2, nx, a.per[0]) >> 1));
+    os2[m] = (j + k) & 1 ? r | l << 16 : l | r << 16;
+    ex[0][p] = B[m];
+  }
+  __syncthreads();
+  T dm = T(0);
+  // One colour, X, from the other one, Y (e: its LDS copy).
+  auto half = [&](auto COL, T(&X)[PER], const T(&Y)[PER], const T(&F)[PER], T w, T w1)
+      __attribute__((always_inline)) {
+    constexpr int col = decltype(COL)::value;
+    const T *e = ex[col];
+    T *o = ex[1 - col];
+#pragma unroll
+    for (int m = 0; m < PER; ++m) {
+      const int p = tid + m * kBlockNT;
+      // Keeps the unpacked places out of registers of their own across iterations.
+      asm("" : "+v"(oy2[m]), "+v"(oz2[m]), "+v"(os2[m]));
+      const T side = e[col ? os2[m] >> 16 : os2[m] & 0xffffu];
+      const T num = -ox * (side + Y[m]) - oy * (e[oy2[m] & 0xffffu] + e[oy2[m] >> 16]) -
+                    oz * (e[oz2[m] & 0xffffu] + e[oz2[m] >> 16]) + F[m];
+      const T pn = pair_div(num, A, invA);
+      const T d = pn - X[m];
+      X[m] = w1 * X[m] + w * pn;
+      if (p < np) {
+        dm = max_abs(dm, d);
+        o[p] = X[m];
+      }
+    }
+    __syncthreads();
+  };
+  int it = P.it0, reason = -1;
+  double om = P.om_a, dprev = P.d_prev;
+  bool end = false;
+  for (int q = 0; q < kBlockIters; ++q) {
+    const double w = it <= a.gs ? 1.0 : om;
+    dm = T(0);
+    half(PIC<0>{}, R, B, fR, T(w), T(1.0 - w));
+    // The maximum of the last iteration's other buffer has been read.
+    half(PIC<1>{}, B, R, fB, T(w), T(1.0 - w));
+    const double v = wave_max((double)dm);
+    if (tid % O3D_WAVE == 0) scr[q & 1][tid / O3D_WAVE] = v;
+    __syncthreads();
+    const double d = wave_max(scr[q & 1][tid % (kBlockNT / O3D_WAVE)]);
+    end = pair_tail(it, d, it == 1 ? 1609.0 : dprev, a, om, reason);
+    dprev = d;
+    ++it;
+    if (end) break;
+  }
+  T *out = a.buf[1 - src];
+#pragma unroll
+  for (int m = 0; m < PER; ++m) {
+    const int p = tid + m * kBlockNT;
+    if (p < np) {
+      out[p] = R[m];
+      out[np + p] = B[m];
+    }
+  }
+  if (tid == 0) {
+    st->sweeps = it - 1;
+    if (end) {
+      st->done = 1;
+      st->reason = reason;
+      st->exit_iter = reason == 2 ? a.kmax + 1 : it - 1;
+      st->result = 1 - src;
+      st->dmax_final = dprev;
+      st->omega_final = om;
+    } else {
+      st->sched[(a.launch + 1) & 1] = {it, 0, 1 - src, 0, dprev, om, om};
+    }
   }
 }
 
@@ -620,6 +738,27 @@ void sor_pair_tiling<float>(SorPairArgs<float> &a) {
   else pair_tiling<float, 1>(a);
 }
 
+// Grids of sor_block_kernel, whose launch runs the whole solve: pairs per thread, 0
+// for larger grids.  Per iteration, march / block: FP64 8^3 5.5 / 0.67 us, 16^3
+// 5.6 / 1.55, 20x20x16 5.6 / 2.5; 8 pairs of doubles spill (24^3 5.6 / 5.3, without
+// the launches' gaps).  FP32 16^3 5.4 / 0.45, 24x20x20 5.6 / 0.88, 24^3 5.9 / 2.1.
+constexpr int kBlockShape = 8;
+template <typename T>
+static int block_per(const SorPairArgs<T> &a) {
+  const long long pairs = (long long)(a.nx / 2) * a.ny * a.nz;
+  for (int per = 2; per <= 32 / (int)sizeof(T); per *= 2)
+    if (pairs <= (long long)per * kBlockNT) return per;
+  return 0;
+}
+template <typename T>
+bool sor_whole(SorPairArgs<T> &a) {
+  if (!block_per(a)) return false;
+  a.shape = kBlockShape;
+  a.ntx = a.nty = a.ntz = 1;
+  a.zc = 2;
+  return true;
+}
+
 template <typename T>
 hipError_t launch_sor_pair_init(const SorPairArgs<T> &a, double omega, hipStream_t s) {
   const int words = (int)sor_pair_slot_words();
@@ -632,11 +771,21 @@ hipError_t launch_sor_pair(const SorPairArgs<T> &a, hipStream_t s) {
   if (a.nx % 2 != 0 || a.nx < 6 || a.ny < 6 || a.nz < 6 ||
       a.zc % 2 != 0 || !sor_buffer_fits<T, T>(a.nx, a.ny, a.nz))
     return hipErrorInvalidValue;
-  if (a.shape == 1) pair_launch<T, 1>(a, s);
+  if (a.shape == kBlockShape) {
+    const int per = block_per(a);
+    if (per == 2) sor_block_kernel<T, 2><<<1, kBlockNT, 0, s>>>(a);
+    else if (per == 4) sor_block_kernel<T, 4><<<1, kBlockNT, 0, s>>>(a);
+    else if (per == 0) return hipErrorInvalidValue;
+    if constexpr (sizeof(T) == 4) {
+      if (per == 8) sor_block_kernel<T, 8><<<1, kBlockNT, 0, s>>>(a);
+    }
+  } else if (a.shape == 1) pair_launch<T, 1>(a, s);
   else pair_launch<T, 0>(a, s);
   return hipGetLastError();
 }
 
+template bool sor_whole<float>(SorPairArgs<float> &);
+template bool sor_whole<double>(SorPairArgs<double> &);
 template hipError_t launch_sor_pair_init<float>(const SorPairArgs<float> &, double, hipStream_t);
 template hipError_t launch_sor_pair_init<double>(const SorPairArgs<double> &, double,
                                                  hipStream_t);

@@ -46,3 +46,34 @@ def test_pair_f32_equals_single(solver, shape):
         b = capi.poisson_f32(pb, rhs, d, 1.7, 1e-30, kmax, 0, solver, variant=2)
         assert a == b, kmax
         assert np.array_equal(pa, pb), kmax
+
+
+# Grids of one block, up to its largest of every number of pairs per thread.
+@pytest.mark.parametrize("solver,shape", [("0000", (16, 16, 16)), ("111111", (17, 16, 16)),
+                                          ("0011", (16, 13, 38)), ("0000", (16, 16, 32))])
+def test_block_f64_equals_oracle(orc, solver, shape):
+    rhs, p0 = rand_fields(shape, 2, seed=63)
+    rhs -= rhs.mean()
+    d = (0.3, 0.35, 0.4)
+    for omega, eps, kmax, idyn in ((1.6, 1e-4, 300, 0), (1.6, 1e-2, 300, 1), (1.6, 1e-30, 1, 0),
+                                   (1.6, 1e-30, 8, 1),
+                                   # More iterations than one launch runs.
+                                   (1.0, 1e-30, 701, 0)):
+        pg, po = p0.copy(), p0.copy()
+        got = capi.poisson(pg, rhs, d, omega, eps, kmax, idyn, solver)
+        it, dm, rs, om, _ = orc.sor(po, rhs, d, solver, omega, eps, kmax, idyn, red_black=True)
+        assert got == (it, dm, rs, om), (omega, eps, kmax)
+        assert np.array_equal(pg, po), (omega, eps, kmax)
+
+
+@pytest.mark.parametrize("solver,shape", [("0000", (6, 6, 8)), ("0011", (16, 11, 24)),
+                                          ("111111", (9, 29, 24)), ("0000", (16, 16, 64))])
+def test_block_f32_equals_single(solver, shape):
+    rhs, p0 = [a.astype(np.float32) for a in rand_fields(shape, 2, seed=64)]
+    d = (0.3, 0.35, 0.4)
+    for kmax in (5, 600):
+        pa, pb = p0.copy(), p0.copy()
+        a = capi.poisson_f32(pa, rhs, d, 1.0, 1e-30, kmax, 0, solver, variant=0)
+        b = capi.poisson_f32(pb, rhs, d, 1.0, 1e-30, kmax, 0, solver, variant=2)
+        assert a == b, kmax
+        assert np.array_equal(pa, pb), kmax
