@@ -687,13 +687,16 @@ namespace {
 // Shared by o3d_nu_t and o3d_predict_velocity: the fused predict kernel with
 // the reference's slot semantics.
 int predict_common(double *up[3], const double *u[3], double *f1[3], const double *f2[3],
-                   const double *f3[3], double *nut, int nh, bool les, double re, double adu,
+                   const double *f3[3], double *const s1[3], double *const s2[3], double *nut, int nh, bool les, double re, double adu,
                    double bdu, double cdu, double cs, double delta, const double h[3], int nx,
                    int ny, int nz, const int *bc, FieldPartial *nut_part) {
   PredictArgs<double> a;
   for (int c = 0; c < 3; ++c) {
     a.u[c] = u[c]; a.up[c] = up[c]; a.f1[c] = f1[c]; a.f2[c] = f2[c]; a.f3[c] = f3[c];
+    if (s1) a.s1[c] = s1[c];
+    if (s2) a.s2[c] = s2[c];
   }
+  a.shift = s2 ? 2 : (s1 ? 1 : 0);
   a.nut = nut;
   a.nut_part = nut_part;
   a.nx = nx; a.ny = ny; a.nz = nz;
@@ -736,7 +739,7 @@ extern "C" int o3d_nu_t(double *nu_t, const double *ux, const double *uy, const 
   CHK(s.scratch(tl.blocks(), &part));
   CHK(s.scratch(1, &fin));
   const double h[3] = {dx, dy, dz};
-  CHK(predict_common(up, u, f1, f2, f2, nut, 1, true, 1.0, 0.0, 0.0, 0.0, cs, delta, h, nx, ny,
+  CHK(predict_common(up, u, f1, f2, f2, nullptr, nullptr, nut, 1, true, 1.0, 0.0, 0.0, 0.0, cs, delta, h, nx, ny,
                      nz, bc, part));
   FieldPartial r;
   CHK(finalize_to_host(part, tl.blocks(), 1, 0, fin, &r));
@@ -799,17 +802,17 @@ extern "C" int o3d_predict_velocity(double *ux_pred, double *uy_pred, double *uz
   FieldPartial *part;
   CHK(s.scratch(tl.blocks(), &part));
   const double h[3] = {dx, dy, dz};
-  CHK(predict_common(up, u, f1, f2, f3, les ? nut : nullptr, ci + 1, les, re, adt[ci], bdt[ci],
-                     cdt[ci], cs, delta, h, nx, ny, nz, bc, part));
-  // History shift by copy, src/integration.f90:176-188.
-  for (int c = 0; c < 3; ++c) {
-    if (itscheme == 2) {
-      HIPCHK(launch_copy<double>(F[c] + n, F[c], (int)n, g_stream));
-    } else if (itscheme == 3) {
-      HIPCHK(launch_copy<double>(F[c] + 2 * n, F[c] + n, (int)n, g_stream));
-      HIPCHK(launch_copy<double>(F[c] + n, F[c], (int)n, g_stream));
-    }
-  }
+  // History shift (src/integration.f90:176-188) by the kernel itself: it holds the
+  // values, and a copy pass per slot reads them again.  At the first step of scheme 3
+  // it does not read the slot that moves on.
+  double *s1[3], *s2[3];
+  for (int c = 0; c < 3; ++c) { s1[c] = F[c] + n; s2[c] = F[c] + 2 * n; }
+  const bool move2 = itscheme == 3 && ci == 0;
+  for (int c = 0; move2 && c < 3; ++c)
+    HIPCHK(launch_copy<double>(s2[c], s1[c], (int)n, g_stream));
+  CHK(predict_common(up, u, f1, f2, f3, itscheme == 2 || itscheme == 3 ? s1 : nullptr,
+                     itscheme == 3 && !move2 ? s2 : nullptr, les ? nut : nullptr, ci + 1, les, re,
+                     adt[ci], bdt[ci], cdt[ci], cs, delta, h, nx, ny, nz, bc, part));
   return s.finish();
 }
 
@@ -1568,10 +1571,11 @@ extern "C" int o3d_transeq(double *phi, const double *ux, const double *uy, cons
   CHK(s.scratch(3 * a.tl.blocks(), &a.part));
   double *sums;
   CHK(s.scratch(3, &sums));
+  // History shift (src/integration.f90:453-460), as in o3d_predict_velocity.
+  if (itscheme == 3 && ci == 0) HIPCHK(launch_copy<double>(F + 2 * n, F + n, (int)n, g_stream));
+  a.s1 = itscheme >= 2 ? F + n : nullptr;
+  a.s2 = itscheme == 3 && ci > 0 ? F + 2 * n : nullptr;
   HIPCHK(launch_transeq<double>(a, sums, g_stream));
-  // History shift by copy, as the reference (src/integration.f90:453-460).
-  if (itscheme == 3) HIPCHK(launch_copy<double>(F + 2 * n, F + n, (int)n, g_stream));
-  if (itscheme >= 2) HIPCHK(launch_copy<double>(F + n, F, (int)n, g_stream));
   return s.finish();
 }
 

@@ -46,6 +46,10 @@ struct PredictArgs {
   const T *f3[3];  // n-2 (read when nh == 3)
   T *nut;          // nu_t out (may be null)
   FieldPartial *nut_part;  // per-block nu_t statistics (LES)
+  // In-place history shift: s1 <- the new F (shift >= 1), s2 <- the value read
+  // from f2 (shift == 2, nh >= 2).  They may be the arrays f2 and f3.
+  int shift = 0;
+  T *s1[3] = {}, *s2[3] = {};
   int nx, ny, nz, bc[3];
   Tiling tl;
   T d1[3][3], d2[3][3];
@@ -118,6 +122,7 @@ struct TranseqArgs {
   const T *f2, *f3;  // F of the two previous steps (read when nh >= 2 / 3)
   double *part;      // 3 sums per block
   int nh, les;
+  T *s1, *s2;        // in-place history shift: F and f2's value (may be null)
   T adu, bdu, cdu, alpha0, sc;
   int nx, ny, nz, bc[3];
   Tiling tl;

@@ -398,6 +398,9 @@ __global__ void __launch_bounds__(kTX *kTY) predict_kernel(const PredictArgs<T> 
         if (NH >= 3) un = un + A.cdu * h3[c];
         A.f1[c][idx] = F;
         A.up[c][idx] = un;
+        // The history shift of the callers that keep it in place.
+        if (A.shift >= 1) A.s1[c][idx] = F;
+        if (NH >= 2 && A.shift >= 2) A.s2[c][idx] = h2[c];
       }
     }
     {
@@ -927,7 +930,8 @@ __global__ void __launch_bounds__(kTX *kTY) transeq_kernel(const TranseqArgs<T> 
       const T alpha = A.les ? A.alpha0 + A.nu_t[idx] / A.sc : A.alpha0;
       const T F = alpha * (lx + ly + lz) - (ux * gx + uy * gy + uz * gz) + sr;
       T pn = q[3] + A.adu * F;
-      if (A.nh >= 2) pn = pn + A.bdu * A.f2[idx];
+      const T h2 = A.nh >= 2 ? A.f2[idx] : T(0);
+      if (A.nh >= 2) pn = pn + A.bdu * h2;
       if (A.nh >= 3) pn = pn + A.cdu * A.f3[idx];
       A.f1[idx] = F;
       A.phi_new[idx] = pn;
@@ -1012,6 +1016,8 @@ __global__ void __launch_bounds__(kTX *kTY) diag_kernel(const DiagArgs<T> A) {
   for (int s = 0; s < 7; ++s) {
     bool fz;
     const int kk = ghost_index(P.z0 - 3 + s, nz, A.bc[2], fz);
+      if (A.s2) A.s2[idx] = h2;
+      if (A.s1) A.s1[idx] = F;
     q[0][s] = load_ghost(A.u[0], col + plane * kk, own_neg[0]);
     q[1][s] = load_ghost(A.u[1], col + plane * kk, own_neg[1]);
     q[2][s] = load_ghost(A.u[2], col + plane * kk, fz);

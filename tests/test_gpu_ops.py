@@ -499,3 +499,26 @@ def test_measurement_entry_points():
             s2.sor_period(1)
         finally:
             s2.close()
+
+
+@pytest.mark.parametrize("itscheme,itime", [(1, 1), (2, 1), (2, 3), (3, 1), (3, 2), (3, 4)])
+def test_history_shift_in_place(itscheme, itime):
+    # The shift of the history slots, written by the kernels that form the new
+    # term: slot 1 = the new term, slot 2 = the old slot 1, as the copies did.
+    sh = (9, 11, 70)
+    u = rand_fields(sh, 3, seed=15)
+    phi, src = rand_fields(sh, 2, seed=16)
+    d = (0.11, 0.13, 0.17)
+    coef = [0.01, 0.02, 0.03]
+    rng = np.random.default_rng(17)
+    old = rng.standard_normal((4, 3) + sh)
+    F = [old[c].copy() for c in range(3)]
+    capi.predict_velocity([np.empty(sh) for _ in range(3)], u, F, 100.0, coef, coef, coef, itime,
+                          itscheme, d, 0, 0.17, 0.2, None, BCS[0])
+    fp = old[3].copy()
+    capi.transeq(np.clip(phi, 0.0, 1.0), u, src, fp, 100.0, 0.7, coef, coef, coef, itime, itscheme,
+                 d, 0, None, BCS[0])
+    for f, o in zip(F + [fp], old):
+        assert not np.array_equal(f[0], o[0])
+        assert np.array_equal(f[1], f[0] if itscheme >= 2 else o[1])
+        assert np.array_equal(f[2], o[1] if itscheme == 3 else o[2])
