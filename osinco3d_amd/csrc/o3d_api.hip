@@ -668,7 +668,7 @@ extern "C" int o3d_divergence(double *divf, const double *fx, const double *fy, 
   a.nx = nx; a.ny = ny; a.nz = nz;
   for (int q = 0; q < 3; ++q) a.bc[q] = bc[q];
   a.odd = odd != 0;
-  a.tl = make_tiling(nx, ny, nz);
+  a.tl = div_tiling<double>(nx, ny, nz);
   const double h[3] = {dx, dy, dz};
   fill_coef<double>(a.d1, h, false);
   a.divisor = divisor;
@@ -687,7 +687,8 @@ namespace {
 // Shared by o3d_nu_t and o3d_predict_velocity: the fused predict kernel with
 // the reference's slot semantics.
 int predict_common(double *up[3], const double *u[3], double *f1[3], const double *f2[3],
-                   const double *f3[3], double *const s1[3], double *const s2[3], double *nut, int nh, bool les, double re, double adu,
+                   const double *f3[3], double *const s1[3], double *const s2[3],
+                   double *nut, int nh, bool les, double re, double adu,
                    double bdu, double cdu, double cs, double delta, const double h[3], int nx,
                    int ny, int nz, const int *bc, FieldPartial *nut_part) {
   PredictArgs<double> a;
@@ -739,8 +740,8 @@ extern "C" int o3d_nu_t(double *nu_t, const double *ux, const double *uy, const 
   CHK(s.scratch(tl.blocks(), &part));
   CHK(s.scratch(1, &fin));
   const double h[3] = {dx, dy, dz};
-  CHK(predict_common(up, u, f1, f2, f2, nullptr, nullptr, nut, 1, true, 1.0, 0.0, 0.0, 0.0, cs, delta, h, nx, ny,
-                     nz, bc, part));
+  CHK(predict_common(up, u, f1, f2, f2, nullptr, nullptr, nut, 1, true, 1.0, 0.0, 0.0, 0.0, cs,
+                     delta, h, nx, ny, nz, bc, part));
   FieldPartial r;
   CHK(finalize_to_host(part, tl.blocks(), 1, 0, fin, &r));
   CHK(s.finish());
@@ -1513,7 +1514,7 @@ int diag_dev(int mode, double *out0, double *out1, double *out2, const double *u
   a.mode = mode;
   a.nx = nx; a.ny = ny; a.nz = nz;
   for (int q = 0; q < 3; ++q) a.bc[q] = bc[q];
-  a.tl = make_tiling(nx, ny, nz);
+  a.tl = diag_tiling<double>(mode, nx, ny, nz);
   const double h[3] = {dx, dy, dz};
   fill_coef<double>(a.d1, h, false);
   HIPCHK(launch_diag<double>(a, g_stream));

@@ -33,6 +33,8 @@ Tiling make_tiling_slots(int nx, int ny, int nz, int slots);
 template <typename T>
 Tiling div_tiling(int nx, int ny, int nz);
 template <typename T>
+Tiling diag_tiling(int mode, int nx, int ny, int nz);
+template <typename T>
 Tiling predict_tiling(int nx, int ny, int nz, bool les);
 template <typename T, typename TP>
 Tiling correct_tiling(int nx, int ny, int nz);
@@ -44,12 +46,12 @@ struct PredictArgs {
   T *f1[3];        // new history slot (written)
   const T *f2[3];  // n-1 (read when nh >= 2)
   const T *f3[3];  // n-2 (read when nh == 3)
-  T *nut;          // nu_t out (may be null)
-  FieldPartial *nut_part;  // per-block nu_t statistics (LES)
   // In-place history shift: s1 <- the new F (shift >= 1), s2 <- the value read
   // from f2 (shift == 2, nh >= 2).  They may be the arrays f2 and f3.
   int shift = 0;
   T *s1[3] = {}, *s2[3] = {};
+  T *nut;          // nu_t out (may be null)
+  FieldPartial *nut_part;  // per-block nu_t statistics (LES)
   int nx, ny, nz, bc[3];
   Tiling tl;
   T d1[3][3], d2[3][3];
@@ -120,9 +122,9 @@ struct TranseqArgs {
   const T *nu_t;     // read when les
   T *f1;             // F of this step
   const T *f2, *f3;  // F of the two previous steps (read when nh >= 2 / 3)
+  T *s1, *s2;        // in-place history shift: F and f2's value (may be null)
   double *part;      // 3 sums per block
   int nh, les;
-  T *s1, *s2;        // in-place history shift: F and f2's value (may be null)
   T adu, bdu, cdu, alpha0, sc;
   int nx, ny, nz, bc[3];
   Tiling tl;

@@ -731,20 +731,57 @@ hipError_t launch_correct(const CorrectArgs<T, TP> &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// --------------------------------------------------------------- statistics
-// src/utils.f90:243-375: per block, the 16 sums behind E_k, eps, eps2,
-// enstrophy and the mean squares (FP64 accumulation).
-// Slot order: 0 e_k, 1 eps, 2 eps2, 3 dzeta, 4..6 u^2 v^2 w^2, 7..15 (du_c/dx_a)^2.
+// The value at a 32-bit byte offset from a base that is the same in every lane (an
+// address in scalar registers and one vector register, no 64-bit vector adds).
 template <typename T>
-__global__ void __launch_bounds__(kTX *kTY) stats_kernel(const StatsArgs<T> A) {
-  __shared__ T pl[3][kTY + 6][kTX + 6];
-  __shared__ ReduceScratch sc;
+__device__ __forceinline__ T load_at(const T *__restrict__ base, unsigned bytes) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes);
+}
+// v with its sign bit flipped where m is the sign bit, unchanged where m is 0.
+__device__ __forceinline__ float flip_sign(float v, unsigned m) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) ^ m);
+}
+__device__ __forceinline__ double flip_sign(double v, unsigned m) {
+  return __builtin_bit_cast(double, __builtin_bit_cast(unsigned long long, v) ^
+                                        ((unsigned long long)m << 32));
+}
+
+template <typename T, int K>
+struct March {
+  static constexpr int NR = 8;
+  // Ring slot of plane k + s at step K.
+  static constexpr int slot(int s) { return (K + s + 3 + NR) % NR; }
+};
+
+template <int... K, typename F>
+__device__ __forceinline__ bool march_group(std::integer_sequence<int, K...>, int k, int end,
+                                            F &&f) {
+  return ((k + K < end && (f(k + K, std::integral_constant<int, K>{}), true)) && ...);
+}
+
+// The z march of the kernels that need the nine first derivatives of (u, v, w) and
+// no other stencil input: body(k, ij, q, L, g, r, cc) once per owned node, with
+// ij its index in plane k, q(c, s) = component c at plane k + s of the node's column (signs applied), L =
+// plane k in LDS (the node at [r][cc]) and g[c][a] = du_c / dx_a with the wall
+// zeros.
+// The column is a ring of 8 planes in registers and the loop runs through its 8
+// positions unrolled, so nothing moves from register to register; the next column
+// value and the halo of the next plane are loaded a step before they are used.
+// Plane k + 1 is staged in the other LDS buffer while k is worked on: one barrier
+// per plane.  256^3 FP64, against loads used in their own step and two barriers:
+// statistics 418 -> 300 us (197 registers, one block per CU: LDS reads and
+// arithmetic 40 % each, little of it overlapped), curl 255 -> 227 us (3.6 TB/s), Q
+// 255 -> 183 us (held to 128 registers; 212 us without).  predict_kernel is faster
+// in its own form, with two planes in flight (256^3 FP64 333 us, 356 us so).
+template <typename T, typename Args, typename Body>
+__device__ __forceinline__ void velocity_march(const Args &A, T (&pl)[2][3][kTY + 6][kTX + 6],
+                                               Body &&body) {
+  constexpr int NR = 8;
   const int nx = A.nx, ny = A.ny, nz = A.nz;
   const TilePos P = tile_pos(A.tl, nx, ny, nz, A.bc);
-  const int plane = nx * ny;
+  const size_t plane = (size_t)nx * ny;
   const int col = P.gi + nx * P.gj;
   const int tx = P.tx, ty = P.ty;
-  const bool own_neg[2] = {P.fi, P.fj};
   int hx_col = -1, hx_g = 0;
   bool hx_f = false;
   if (tx < 3) { hx_col = tx; hx_g = ghost_safe(P.x0 + tx - 3, nx, A.bc[0], hx_f); }
@@ -753,102 +790,151 @@ __global__ void __launch_bounds__(kTX *kTY) stats_kernel(const StatsArgs<T> A) {
   bool hy_f = false;
   if (ty < 3) { hy_row = ty; hy_g = ghost_safe(P.y0 + ty - 3, ny, A.bc[1], hy_f); }
   else if (ty >= kTY - 3) { hy_row = ty + 6; hy_g = ghost_safe(P.y0 + ty + 3, ny, A.bc[1], hy_f); }
-  const int hx_idx = hx_g + nx * P.gj;
-  const int hy_idx = P.gi + nx * hy_g;
+  // Byte offsets in a plane (below 2^32: a plane is at most a sixth of 2^31 nodes);
+  // lanes without a halo cell load their own column.
+  const unsigned es = sizeof(T), co = (unsigned)col * es;
+  const unsigned xo = hx_col >= 0 ? (unsigned)(hx_g + nx * P.gj) * es : co;
+  const unsigned yo = hy_row >= 0 ? (unsigned)(P.gi + nx * hy_g) * es : co;
+  // u_c is odd along axis c.
+  auto sign = [](bool neg) { return neg ? 0x80000000u : 0u; };
+  const unsigned sq[2] = {sign(P.fi), sign(P.fj)};
+  const unsigned sx0 = sign(hx_col >= 0 && hx_f), sy1 = sign(hy_row >= 0 && hy_f);
   const bool edge_x = A.bc[0] == FREE_SLIP && (P.i == 0 || P.i == nx - 1);
   const bool edge_y = A.bc[1] == FREE_SLIP && (P.j == 0 || P.j == ny - 1);
   const bool xdir = A.bc[0] == DIRICHLET && (P.x0 == 0 || P.x0 + kTX + 2 >= nx);
-  double acc[16];
-#pragma unroll
-  for (int m = 0; m < 16; ++m) acc[m] = 0.0;
-  T q[3][7];
-#pragma unroll
-  for (int s = 0; s < 6; ++s) {
+
+  T q[3][NR], hx[3], hy[3];
+  // Plane kp (-3 .. nz + 3) of the column into ring slot sl, raw; its sign for w.
+  auto load_z = [&](int kp, int sl) __attribute__((always_inline)) {
     bool fz;
-    const int kk = ghost_index(P.z0 - 3 + s, nz, A.bc[2], fz);
-    q[0][s] = load_ghost(A.u[0], col + plane * kk, own_neg[0]);
-    q[1][s] = load_ghost(A.u[1], col + plane * kk, own_neg[1]);
-    q[2][s] = load_ghost(A.u[2], col + plane * kk, fz);
-  }
-  for (int k = P.z0; k < P.z1; ++k) {
-    {
-      bool fz;
-      const int kk = ghost_index(k + 3, nz, A.bc[2], fz);
-      q[0][6] = load_ghost(A.u[0], col + plane * kk, own_neg[0]);
-      q[1][6] = load_ghost(A.u[1], col + plane * kk, own_neg[1]);
-      q[2][6] = load_ghost(A.u[2], col + plane * kk, fz);
-    }
-    const int pk = plane * k;
-    T hx[3], hy[3];
-    if (hx_col >= 0) {
-      hx[0] = load_ghost(A.u[0], hx_idx + pk, hx_f);
-      hx[1] = load_ghost(A.u[1], hx_idx + pk, own_neg[1]);
-      hx[2] = A.u[2][hx_idx + pk];
-    }
-    if (hy_row >= 0) {
-      hy[0] = load_ghost(A.u[0], hy_idx + pk, own_neg[0]);
-      hy[1] = load_ghost(A.u[1], hy_idx + pk, hy_f);
-      hy[2] = A.u[2][hy_idx + pk];
-    }
+    const size_t o = plane * ghost_index(kp, nz, A.bc[2], fz);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) q[c][sl] = load_at(A.u[c] + o, co);
+    return sign(fz);
+  };
+  auto sign_z = [&](int sl, unsigned sz) __attribute__((always_inline)) {
+    q[0][sl] = flip_sign(q[0][sl], sq[0]);
+    q[1][sl] = flip_sign(q[1][sl], sq[1]);
+    q[2][sl] = flip_sign(q[2][sl], sz);
+  };
+  auto load_halo = [&](int kp) __attribute__((always_inline)) {
+    const size_t o = plane * min(kp, nz - 1);  // planes after the last are not used
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      pl[c][ty + 3][tx + 3] = q[c][3];
-      if (hx_col >= 0) pl[c][ty + 3][hx_col] = hx[c];
-      if (hy_row >= 0) pl[c][hy_row][tx + 3] = hy[c];
+      hx[c] = load_at(A.u[c] + o, xo);
+      hy[c] = load_at(A.u[c] + o, yo);
+    }
+  };
+  // Ring slot sl and the halo as a plane of LDS buffer b.
+  auto stage = [&](int b, int sl) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) pl[b][c][ty + 3][tx + 3] = q[c][sl];
+    if (hx_col >= 0) {
+      pl[b][0][ty + 3][hx_col] = flip_sign(hx[0], sx0);
+      pl[b][1][ty + 3][hx_col] = flip_sign(hx[1], sq[1]);
+      pl[b][2][ty + 3][hx_col] = hx[2];
+    }
+    if (hy_row >= 0) {
+      pl[b][0][hy_row][tx + 3] = flip_sign(hy[0], sq[0]);
+      pl[b][1][hy_row][tx + 3] = flip_sign(hy[1], sy1);
+      pl[b][2][hy_row][tx + 3] = hy[2];
     }
     __syncthreads();
     if (xdir) {
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
-        xdir_fill<T>(&pl[c][ty + 3][0], tx + 3, P.x0, nx);
-        if (hx_col >= 0) xdir_fill<T>(&pl[c][ty + 3][0], hx_col, P.x0, nx);
+        xdir_fill<T>(&pl[b][c][ty + 3][0], tx + 3, P.x0, nx);
+        if (hx_col >= 0) xdir_fill<T>(&pl[b][c][ty + 3][0], hx_col, P.x0, nx);
       }
       __syncthreads();
     }
+  };
+  load_halo(P.z0);
+#pragma unroll
+  for (int s = -3; s <= 3; ++s) sign_z(March<T, 0>::slot(s), load_z(P.z0 + s, March<T, 0>::slot(s)));
+  stage(0, March<T, 0>::slot(0));
+  auto step = [&](int k, auto KK) __attribute__((always_inline)) {
+    constexpr int K = decltype(KK)::value;
+    using M = March<T, K>;
+    const unsigned sz = load_z(k + 4, M::slot(4));
+    load_halo(k + 1);
     if (P.valid) {
-      const int r = ty + 3, cc = tx + 3;
-      double g[3][3], l[3][3];
+      const int r = ty + 3, cc = tx + 3, ij = P.i + nx * P.j;
+      const T(&L)[3][kTY + 6][kTX + 6] = pl[K & 1];
+      T g[3][3];
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
-        g[c][0] = d1<T>(pl[c][r][cc - 3], pl[c][r][cc - 2], pl[c][r][cc - 1], pl[c][r][cc + 1],
-                        pl[c][r][cc + 2], pl[c][r][cc + 3], A.d1[0]);
-        g[c][1] = d1<T>(pl[c][r - 3][cc], pl[c][r - 2][cc], pl[c][r - 1][cc], pl[c][r + 1][cc],
-                        pl[c][r + 2][cc], pl[c][r + 3][cc], A.d1[1]);
-        g[c][2] = d1<T>(q[c][0], q[c][1], q[c][2], q[c][4], q[c][5], q[c][6], A.d1[2]);
-        l[c][0] = d2<T>(pl[c][r][cc - 2], pl[c][r][cc - 1], pl[c][r][cc], pl[c][r][cc + 1],
-                        pl[c][r][cc + 2], A.d2[0]);
-        l[c][1] = d2<T>(pl[c][r - 2][cc], pl[c][r - 1][cc], pl[c][r][cc], pl[c][r + 1][cc],
-                        pl[c][r + 2][cc], A.d2[1]);
-        l[c][2] = d2<T>(q[c][1], q[c][2], q[c][3], q[c][4], q[c][5], A.d2[2]);
+        g[c][0] = d1<T>(L[c][r][cc - 3], L[c][r][cc - 2], L[c][r][cc - 1], L[c][r][cc + 1],
+                        L[c][r][cc + 2], L[c][r][cc + 3], A.d1[0]);
+        g[c][1] = d1<T>(L[c][r - 3][cc], L[c][r - 2][cc], L[c][r - 1][cc], L[c][r + 1][cc],
+                        L[c][r + 2][cc], L[c][r + 3][cc], A.d1[1]);
+        g[c][2] = d1<T>(q[c][M::slot(-3)], q[c][M::slot(-2)], q[c][M::slot(-1)],
+                        q[c][M::slot(1)], q[c][M::slot(2)], q[c][M::slot(3)], A.d1[2]);
       }
-      if (edge_x) { g[1][0] = 0.0; g[2][0] = 0.0; }
-      if (edge_y) { g[0][1] = 0.0; g[2][1] = 0.0; }
-      if (A.bc[2] == FREE_SLIP && (k == 0 || k == nz - 1)) { g[0][2] = 0.0; g[1][2] = 0.0; }
-      const double ux = q[0][3], uy = q[1][3], uz = q[2][3];
-      const double xnu = A.xnu;
-      acc[0] += 0.5 * (ux * ux + uy * uy + uz * uz);
-      const double a2 = 2.0 * g[0][0], b2 = 2.0 * g[1][1], c2 = 2.0 * g[2][2];
-      const double s12 = g[0][1] + g[1][0], s13 = g[0][2] + g[2][0], s23 = g[1][2] + g[2][1];
-      acc[1] += 0.5 * xnu * (a2 * a2 + b2 * b2 + c2 * c2 + 2.0 * (s12 * s12) +
-                             2.0 * (s13 * s13) + 2.0 * (s23 * s23));
-      acc[2] += (-xnu) * (ux * (l[0][0] + l[0][1] + l[0][2]) + uy * (l[1][0] + l[1][1] + l[1][2]) +
-                          uz * (l[2][0] + l[2][1] + l[2][2]));
-      const double w1 = g[2][1] - g[1][2], w2 = g[0][2] - g[2][0], w3 = g[1][0] - g[0][1];
-      acc[3] += 0.5 * (w1 * w1 + w2 * w2 + w3 * w3);
-      acc[4] += ux * ux;
-      acc[5] += uy * uy;
-      acc[6] += uz * uz;
-#pragma unroll
-      for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int a = 0; a < 3; ++a) acc[7 + 3 * c + a] += g[c][a] * g[c][a];
+      if (edge_x) { g[1][0] = T(0); g[2][0] = T(0); }
+      if (edge_y) { g[0][1] = T(0); g[2][1] = T(0); }
+      if (A.bc[2] == FREE_SLIP && (k == 0 || k == nz - 1)) { g[0][2] = T(0); g[1][2] = T(0); }
+      body(k, ij, [&](int c, auto S) __attribute__((always_inline)) {
+        return q[c][M::slot(decltype(S)::value)];
+      }, L, g, r, cc);
     }
-    __syncthreads();
+    sign_z(M::slot(4), sz);
+    stage(1 - (K & 1), M::slot(1));
+  };
+  for (int k = P.z0; march_group(std::make_integer_sequence<int, NR>{}, k, P.z1, step); k += NR) {
+  }
+}
+// Plane offsets for q(c, .) of velocity_march.
+template <int S>
+using Pl = std::integral_constant<int, S>;
+
+// --------------------------------------------------------------- statistics
+// src/utils.f90:243-375: per block, the 16 sums behind E_k, eps, eps2,
+// enstrophy and the mean squares (FP64 accumulation).
+// Slot order: 0 e_k, 1 eps, 2 eps2, 3 dzeta, 4..6 u^2 v^2 w^2, 7..15 (du_c/dx_a)^2.
+template <typename T>
+__global__ void __launch_bounds__(kTX *kTY) stats_kernel(const StatsArgs<T> A) {
+  __shared__ T pl[2][3][kTY + 6][kTX + 6];
+  __shared__ ReduceScratch sc;
+  double acc[16];
+#pragma unroll
+  for (int m = 0; m < 16; ++m) acc[m] = 0.0;
+  velocity_march<T>(A, pl, [&](int, int, auto &&q, const T(&L)[3][kTY + 6][kTX + 6],
+                            const T(&gt)[3][3], int r, int cc) __attribute__((always_inline)) {
+    double g[3][3];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int s = 0; s < 6; ++s) q[c][s] = q[c][s + 1];
-  }
+      for (int a = 0; a < 3; ++a) g[c][a] = gt[c][a];
+    const double u[3] = {q(0, Pl<0>{}), q(1, Pl<0>{}), q(2, Pl<0>{})};
+    const double xnu = A.xnu;
+    acc[0] += 0.5 * (u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+    const double a2 = 2.0 * g[0][0], b2 = 2.0 * g[1][1], c2 = 2.0 * g[2][2];
+    const double s12 = g[0][1] + g[1][0], s13 = g[0][2] + g[2][0], s23 = g[1][2] + g[2][1];
+    acc[1] += 0.5 * xnu * (a2 * a2 + b2 * b2 + c2 * c2 + 2.0 * (s12 * s12) +
+                           2.0 * (s13 * s13) + 2.0 * (s23 * s23));
+    double ul[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const T z = q(c, Pl<0>{});
+      const double lx = d2<T>(L[c][r][cc - 2], L[c][r][cc - 1], z, L[c][r][cc + 1],
+                              L[c][r][cc + 2], A.d2[0]);
+      const double ly = d2<T>(L[c][r - 2][cc], L[c][r - 1][cc], z, L[c][r + 1][cc],
+                              L[c][r + 2][cc], A.d2[1]);
+      const double lz = d2<T>(q(c, Pl<-2>{}), q(c, Pl<-1>{}), z, q(c, Pl<1>{}), q(c, Pl<2>{}),
+                              A.d2[2]);
+      ul[c] = u[c] * (lx + ly + lz);
+    }
+    acc[2] += (-xnu) * (ul[0] + ul[1] + ul[2]);
+    const double w1 = g[2][1] - g[1][2], w2 = g[0][2] - g[2][0], w3 = g[1][0] - g[0][1];
+    acc[3] += 0.5 * (w1 * w1 + w2 * w2 + w3 * w3);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) acc[4 + c] += u[c] * u[c];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) acc[7 + 3 * c + a] += g[c][a] * g[c][a];
+  });
 #pragma unroll
   for (int m = 0; m < 16; ++m) {
     const double v = block_sum<kNW>(acc[m], sc.v);
@@ -934,6 +1020,8 @@ __global__ void __launch_bounds__(kTX *kTY) transeq_kernel(const TranseqArgs<T> 
       if (A.nh >= 2) pn = pn + A.bdu * h2;
       if (A.nh >= 3) pn = pn + A.cdu * A.f3[idx];
       A.f1[idx] = F;
+      if (A.s2) A.s2[idx] = h2;
+      if (A.s1) A.s1[idx] = F;
       A.phi_new[idx] = pn;
       const T c = fmax(T(0), fmin(T(1), pn));
       s_old += (double)pn;
@@ -977,7 +1065,7 @@ __global__ void __launch_bounds__(256) transeq_clip_kernel(T *phi, const T *phi_
 template <typename T>
 hipError_t launch_transeq(const TranseqArgs<T> &a, double *sums, hipStream_t s) {
   transeq_kernel<T><<<dim3(a.tl.blocks()), dim3(kTX * kTY), 0, s>>>(a);
-  finalize_sums_kernel<<<1, 1024, 0, s>>>(a.part, a.tl.blocks(), 3, sums);
+  finalize_sums_kernel<<<3, 1024, 0, s>>>(a.part, a.tl.blocks(), 3, sums);
   const int n = a.nx * a.ny * a.nz;
   transeq_clip_kernel<T><<<(n + 255) / 256, 256, 0, s>>>(a.phi_out, a.phi_new, sums, n);
   return hipGetLastError();
@@ -990,101 +1078,35 @@ hipError_t launch_transeq(const TranseqArgs<T> &a, double *sums, hipStream_t s) 
 // variant choice (u_c odd along axis c: derxi/deryi/derzi on the diagonal,
 // the p variants with their wall zeros across), as in the predict kernel, and
 // each output keeps the reference's operation order.
+template <typename T, int MODE>
+__global__ void __launch_bounds__(kTX *kTY, 4) diag_kernel(const DiagArgs<T> A) {
+  __shared__ T pl[2][3][kTY + 6][kTX + 6];
+  velocity_march<T>(A, pl, [&](int k, int ij, auto &&, const T(&)[3][kTY + 6][kTX + 6],
+                            const T(&g)[3][3], int, int) __attribute__((always_inline)) {
+    const int idx = ij + A.nx * A.ny * k;
+    if (MODE == 0) {
+      A.out[0][idx] = g[2][1] - g[1][2];  // duz/dy - duy/dz
+      A.out[1][idx] = g[0][2] - g[2][0];  // dux/dz - duz/dx
+      A.out[2][idx] = g[1][0] - g[0][1];  // duy/dx - dux/dy
+    } else {
+      A.out[0][idx] = -(T(0.5) * (g[0][0] * g[0][0] + g[1][1] * g[1][1] + g[2][2] * g[2][2])) -
+                      g[0][1] * g[1][0] - g[0][2] * g[2][0] - g[1][2] * g[2][1];
+    }
+  });
+}
+
 template <typename T>
-__global__ void __launch_bounds__(kTX *kTY) diag_kernel(const DiagArgs<T> A) {
-  __shared__ T pl[3][kTY + 6][kTX + 6];
-  const int nx = A.nx, ny = A.ny, nz = A.nz;
-  const TilePos P = tile_pos(A.tl, nx, ny, nz, A.bc);
-  const int plane = nx * ny;
-  const int col = P.gi + nx * P.gj;
-  const int tx = P.tx, ty = P.ty;
-  const bool own_neg[2] = {P.fi, P.fj};
-  int hx_col = -1, hx_g = 0;
-  bool hx_f = false;
-  if (tx < 3) { hx_col = tx; hx_g = ghost_safe(P.x0 + tx - 3, nx, A.bc[0], hx_f); }
-  else if (tx >= kTX - 3) { hx_col = tx + 6; hx_g = ghost_safe(P.x0 + tx + 3, nx, A.bc[0], hx_f); }
-  int hy_row = -1, hy_g = 0;
-  bool hy_f = false;
-  if (ty < 3) { hy_row = ty; hy_g = ghost_safe(P.y0 + ty - 3, ny, A.bc[1], hy_f); }
-  else if (ty >= kTY - 3) { hy_row = ty + 6; hy_g = ghost_safe(P.y0 + ty + 3, ny, A.bc[1], hy_f); }
-  const int hx_idx = hx_g + nx * P.gj;
-  const int hy_idx = P.gi + nx * hy_g;
-  const bool edge_x = A.bc[0] == FREE_SLIP && (P.i == 0 || P.i == nx - 1);
-  const bool edge_y = A.bc[1] == FREE_SLIP && (P.j == 0 || P.j == ny - 1);
-  T q[3][8];
-#pragma unroll
-  for (int s = 0; s < 7; ++s) {
-    bool fz;
-    const int kk = ghost_index(P.z0 - 3 + s, nz, A.bc[2], fz);
-      if (A.s2) A.s2[idx] = h2;
-      if (A.s1) A.s1[idx] = F;
-    q[0][s] = load_ghost(A.u[0], col + plane * kk, own_neg[0]);
-    q[1][s] = load_ghost(A.u[1], col + plane * kk, own_neg[1]);
-    q[2][s] = load_ghost(A.u[2], col + plane * kk, fz);
-  }
-  for (int k = P.z0; k < P.z1; ++k) {
-    {
-      // k + 4 <= nz + 3 stays a valid mirror / wrap index for nz >= 6.
-      bool fz;
-      const int kk = ghost_index(k + 4, nz, A.bc[2], fz);
-      q[0][7] = load_ghost(A.u[0], col + plane * kk, own_neg[0]);
-      q[1][7] = load_ghost(A.u[1], col + plane * kk, own_neg[1]);
-      q[2][7] = load_ghost(A.u[2], col + plane * kk, fz);
-    }
-    const int pk = plane * k;
-    T hx[3], hy[3];
-    if (hx_col >= 0) {
-      hx[0] = load_ghost(A.u[0], hx_idx + pk, hx_f);
-      hx[1] = load_ghost(A.u[1], hx_idx + pk, own_neg[1]);
-      hx[2] = A.u[2][hx_idx + pk];
-    }
-    if (hy_row >= 0) {
-      hy[0] = load_ghost(A.u[0], hy_idx + pk, own_neg[0]);
-      hy[1] = load_ghost(A.u[1], hy_idx + pk, hy_f);
-      hy[2] = A.u[2][hy_idx + pk];
-    }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      pl[c][ty + 3][tx + 3] = q[c][3];
-      if (hx_col >= 0) pl[c][ty + 3][hx_col] = hx[c];
-      if (hy_row >= 0) pl[c][hy_row][tx + 3] = hy[c];
-    }
-    __syncthreads();
-    if (P.valid) {
-      const int idx = P.i + nx * P.j + pk;
-      const int r = ty + 3, cc = tx + 3;
-      T g[3][3];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        g[c][0] = d1<T>(pl[c][r][cc - 3], pl[c][r][cc - 2], pl[c][r][cc - 1], pl[c][r][cc + 1],
-                        pl[c][r][cc + 2], pl[c][r][cc + 3], A.d1[0]);
-        g[c][1] = d1<T>(pl[c][r - 3][cc], pl[c][r - 2][cc], pl[c][r - 1][cc], pl[c][r + 1][cc],
-                        pl[c][r + 2][cc], pl[c][r + 3][cc], A.d1[1]);
-        g[c][2] = d1<T>(q[c][0], q[c][1], q[c][2], q[c][4], q[c][5], q[c][6], A.d1[2]);
-      }
-      if (edge_x) { g[1][0] = T(0); g[2][0] = T(0); }
-      if (edge_y) { g[0][1] = T(0); g[2][1] = T(0); }
-      if (A.bc[2] == FREE_SLIP && (k == 0 || k == nz - 1)) { g[0][2] = T(0); g[1][2] = T(0); }
-      if (A.mode == 0) {
-        A.out[0][idx] = g[2][1] - g[1][2];  // duz/dy - duy/dz
-        A.out[1][idx] = g[0][2] - g[2][0];  // dux/dz - duz/dx
-        A.out[2][idx] = g[1][0] - g[0][1];  // duy/dx - dux/dy
-      } else {
-        A.out[0][idx] = -(T(0.5) * (g[0][0] * g[0][0] + g[1][1] * g[1][1] + g[2][2] * g[2][2])) -
-                        g[0][1] * g[1][0] - g[0][2] * g[2][0] - g[1][2] * g[2][1];
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int s = 0; s < 7; ++s) q[c][s] = q[c][s + 1];
-  }
+Tiling diag_tiling(int mode, int nx, int ny, int nz) {
+  static const int slots[2] = {stencil_slots((const void *)diag_kernel<T, 0>),
+                               stencil_slots((const void *)diag_kernel<T, 1>)};
+  return make_tiling_slots(nx, ny, nz, slots[mode ? 1 : 0]);
 }
 
 template <typename T>
 hipError_t launch_diag(const DiagArgs<T> &a, hipStream_t s) {
-  diag_kernel<T><<<dim3(a.tl.blocks()), dim3(kTX * kTY), 0, s>>>(a);
+  const dim3 blk(kTX * kTY), grd(a.tl.blocks());
+  if (a.mode == 0) diag_kernel<T, 0><<<grd, blk, 0, s>>>(a);
+  else diag_kernel<T, 1><<<grd, blk, 0, s>>>(a);
   return hipGetLastError();
 }
 
@@ -1177,17 +1199,17 @@ hipError_t launch_finalize_sets(const FinalizeSet *sets, int n, hipStream_t s) {
 __global__ void __launch_bounds__(1024) finalize_sums_kernel(const double *part, int nparts,
                                                              int width, double *out) {
   __shared__ double sv[16];
-  for (int m = 0; m < width; ++m) {
-    double s = 0.0;
-    for (int b = threadIdx.x; b < nparts; b += blockDim.x) s += part[(size_t)b * width + m];
-    s = block_sum<16>(s, sv);
-    if (threadIdx.x == 0) out[m] = s;
-  }
+  // A block per sum: one block after the other took 23 us for 16 sums of 1024.
+  const int m = blockIdx.x;
+  double s = 0.0;
+  for (int b = threadIdx.x; b < nparts; b += blockDim.x) s += part[(size_t)b * width + m];
+  s = block_sum<16>(s, sv);
+  if (threadIdx.x == 0) out[m] = s;
 }
 
 hipError_t launch_finalize_sums(const double *part, int nparts, int width, double *out,
                                 hipStream_t s) {
-  finalize_sums_kernel<<<1, 1024, 0, s>>>(part, nparts, width, out);
+  finalize_sums_kernel<<<width, 1024, 0, s>>>(part, nparts, width, out);
   return hipGetLastError();
 }
 
@@ -1200,6 +1222,7 @@ template hipError_t launch_predict<double>(const PredictArgs<double> &, int, boo
 template hipError_t launch_predict<float>(const PredictArgs<float> &, int, bool, hipStream_t);
 template Tiling predict_tiling<double>(int, int, int, bool);
 template Tiling predict_tiling<float>(int, int, int, bool);
+template Tiling diag_tiling<double>(int, int, int, int);
 template Tiling div_tiling<double>(int, int, int);
 template Tiling div_tiling<float>(int, int, int);
 template Tiling correct_tiling<double, double>(int, int, int);
