@@ -41,6 +41,10 @@ int o3d_init(int device);
 int o3d_set_stream(void *stream);
 const char *o3d_last_error(void);
 int o3d_sync(void);
+/* Give back the device buffers the library keeps between calls for scratch and
+ * staging (at most 1 GiB idle; a failed allocation of its own gives them back
+ * too). */
+int o3d_release_scratch(void);
 /* Library version string. */
 const char *o3d_version(void);
 /* Measurement: a hand-written streaming triad c = a + s b over three device

@@ -12,6 +12,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <mutex>
 #include <type_traits>
 #include <string>
 #include <vector>
@@ -146,14 +147,110 @@ int reg_touch(const void *p, size_t bytes, bool write) {
   return 0;
 }
 
-// Staging of host arrays through device buffers for one call.
+// Device buffers of finished calls, kept for the next one: allocating and freeing
+// the 134 MB field of o3d_transeq at 256^3 took as long as its kernels (380 us a
+// call, now and then 3.7 ms).  At most kLimit bytes are idle (the oldest go first);
+// o3d_release_scratch or a failed allocation gives all of them back.  A block is in
+// the pool only while nothing on the GPU uses it: Staged puts it there after its
+// stream has been waited for.
+class ScratchPool {
+ public:
+  static ScratchPool &get() {
+    static ScratchPool *pool = new ScratchPool;  // outlives the HIP runtime's teardown
+    return *pool;
+  }
+  // A block of at least `bytes` (its true size in *size), or null.
+  void *take(size_t bytes, size_t *size) {
+    bytes = (std::max<size_t>(bytes, 1) + 4095) / 4096 * 4096;
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    {
+      std::lock_guard<std::mutex> lock(m_);
+      size_t best = idle_.size();
+      for (size_t q = 0; q < idle_.size(); ++q)
+        if (idle_[q].dev == dev && idle_[q].bytes >= bytes && idle_[q].bytes <= 2 * bytes &&
+            (best == idle_.size() || idle_[q].bytes < idle_[best].bytes))
+          best = q;
+      if (best < idle_.size()) {
+        void *p = idle_[best].p;
+        *size = idle_[best].bytes;
+        held_ -= *size;
+        idle_.erase(idle_.begin() + best);
+        return p;
+      }
+    }
+    *size = bytes;
+    return allocate(bytes);
+  }
+  void give(void *p, size_t bytes) {
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    std::vector<void *> out;
+    {
+      std::lock_guard<std::mutex> lock(m_);
+      if (bytes > kLimit) {
+        out.push_back(p);
+      } else {
+        while (held_ + bytes > kLimit) {
+          out.push_back(idle_.front().p);
+          held_ -= idle_.front().bytes;
+          idle_.erase(idle_.begin());
+        }
+        idle_.push_back({p, bytes, dev});
+        held_ += bytes;
+      }
+    }
+    for (void *q : out) (void)hipFree(q);
+  }
+  void release() {
+    std::vector<Block> out;
+    {
+      std::lock_guard<std::mutex> lock(m_);
+      out.swap(idle_);
+      held_ = 0;
+    }
+    for (const Block &b : out) (void)hipFree(b.p);
+  }
+  // hipMalloc, once more without the idle blocks when it fails; null then.
+  void *allocate(size_t bytes) {
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    release();
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+
+ private:
+  static constexpr size_t kLimit = (size_t)1 << 30;
+  struct Block { void *p; size_t bytes; int dev; };
+  std::mutex m_;
+  std::vector<Block> idle_;  // oldest first
+  size_t held_ = 0;
+};
+
+// Staging of host arrays through device buffers for one call, and its scratch.
 struct Staged {
   struct Out { void *dev; void *host; size_t bytes; };
-  std::vector<void *> allocs;
+  struct Alloc { void *p; size_t bytes; };
+  std::vector<Alloc> allocs;
   std::vector<Out> outs;
   std::vector<RegEntry *> written;
+  bool idle = false;  // finish() has waited for the stream and nothing came after
   ~Staged() {
-    for (void *p : allocs) (void)hipFree(p);
+    for (const Alloc &a : allocs) {
+      if (idle) ScratchPool::get().give(a.p, a.bytes);
+      else (void)hipFree(a.p);
+    }
+  }
+  int device(size_t bytes, void **d) {
+    size_t size = 0;
+    *d = ScratchPool::get().take(bytes, &size);
+    if (!*d) return fail("out of device memory (%zu bytes)", bytes);
+    allocs.push_back({*d, size});
+    idle = false;
+    return 0;
   }
   template <typename T>
   int in(const T *p, size_t n, const T **dev) {
@@ -172,8 +269,7 @@ struct Staged {
     }
     CHK(reg_touch(p, bytes, false));
     void *d = nullptr;
-    HIPCHK(hipMalloc(&d, bytes));
-    allocs.push_back(d);
+    CHK(device(bytes, &d));
     HIPCHK(hipMemcpyAsync(d, p, bytes, hipMemcpyHostToDevice, g_stream));
     g_h2d += (double)bytes;
     *dev = (const T *)d;
@@ -199,8 +295,7 @@ struct Staged {
     }
     CHK(reg_touch(p, bytes, true));
     void *d = nullptr;
-    HIPCHK(hipMalloc(&d, bytes));
-    allocs.push_back(d);
+    CHK(device(bytes, &d));
     if (copy_in) {
       HIPCHK(hipMemcpyAsync(d, p, bytes, hipMemcpyHostToDevice, g_stream));
       g_h2d += (double)bytes;
@@ -212,8 +307,7 @@ struct Staged {
   template <typename T>
   int scratch(size_t n, T **dev) {
     void *d = nullptr;
-    HIPCHK(hipMalloc(&d, n * sizeof(T)));
-    allocs.push_back(d);
+    CHK(device(n * sizeof(T), &d));
     *dev = (T *)d;
     return 0;
   }
@@ -229,7 +323,61 @@ struct Staged {
         e->host_valid = true;
       }
     HIPCHK(hipStreamSynchronize(g_stream));
+    idle = true;
     return 0;
+  }
+};
+
+// What a solve reads back through (pinned) and times with.  One set is kept between
+// calls (making it took about 100 us); a call that finds it taken makes its own.
+struct HostState {
+  SorState *hst = nullptr;
+  double *hfin = nullptr;  // 4 values
+  std::vector<hipEvent_t> ev;
+  ~HostState() {
+    for (hipEvent_t e : ev) (void)hipEventDestroy(e);
+    if (hst) (void)hipHostFree(hst);
+    if (hfin) (void)hipHostFree(hfin);
+  }
+  int open() {
+    if (!hst) HIPCHK(hipHostMalloc((void **)&hst, sizeof(SorState)));
+    if (!hfin) HIPCHK(hipHostMalloc((void **)&hfin, 4 * sizeof(double)));
+    while (ev.size() < 2) {
+      hipEvent_t e;
+      HIPCHK(hipEventCreate(&e));
+      ev.push_back(e);
+    }
+    return 0;
+  }
+};
+std::mutex g_host_mutex;
+HostState *g_host_spare = nullptr;
+int g_host_dev = 0;  // the device its events belong to
+struct HostLease {
+  HostState *h = nullptr;
+  bool idle = false;  // the caller has waited for all that uses it
+  ~HostLease() {
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    {
+      std::lock_guard<std::mutex> lock(g_host_mutex);
+      if (idle && !g_host_spare) {
+        g_host_spare = h;
+        g_host_dev = dev;
+        h = nullptr;
+      }
+    }
+    delete h;
+  }
+  int open() {
+    int dev = 0;
+    HIPCHK(hipGetDevice(&dev));
+    {
+      std::lock_guard<std::mutex> lock(g_host_mutex);
+      if (g_host_spare && g_host_dev == dev) std::swap(h, g_host_spare);
+    }
+    if (!h) h = new HostState;
+    return h->open();
   }
 };
 
@@ -447,6 +595,11 @@ extern "C" int o3d_set_stream(void *stream) {
 
 extern "C" const char *o3d_last_error(void) { return g_err.c_str(); }
 
+extern "C" int o3d_release_scratch(void) {
+  ScratchPool::get().release();
+  return 0;
+}
+
 extern "C" int o3d_sync(void) {
   HIPCHK(hipStreamSynchronize(g_stream));
   return 0;
@@ -470,8 +623,8 @@ extern "C" int o3d_register(const void *host, size_t bytes, int mirror) {
   for (const RegEntry &e : g_reg)
     if (!(e.host + e.bytes <= lo || lo + bytes <= e.host))
       return fail("o3d_register: %p overlaps a registered array", host);
-  void *d = nullptr;
-  HIPCHK(hipMalloc(&d, bytes));
+  void *d = ScratchPool::get().allocate(bytes);
+  if (!d) return fail("o3d_register: out of device memory (%zu bytes)", bytes);
   g_reg.push_back({(char *)host, bytes, d, false, true, mirror != 0});
   return 0;
 }
@@ -861,10 +1014,10 @@ int poisson_dev(T *pp, const T *rhs, double dx, double dy, double dz, int nx, in
   const int n = nx * ny * nz;
   SorRun<T, T> r;
   CHK(s.scratch(1, &r.st));
-  HIPCHK(hipHostMalloc((void **)&r.hst, sizeof(SorState)));
-  std::vector<hipEvent_t> ev(2);
-  for (auto &e : ev) HIPCHK(hipEventCreate(&e));
-  r.events = &ev;
+  HostLease lease;
+  CHK(lease.open());
+  r.hst = lease.h->hst;
+  r.events = &lease.h->ev;
   T *other;
   CHK(s.scratch(n, &other));
   r.buf[0] = pp;
@@ -913,9 +1066,8 @@ int poisson_dev(T *pp, const T *rhs, double dx, double dy, double dz, int nx, in
     if (exit_iter) *exit_iter = r.hst->exit_iter;
     if (dmax) *dmax = r.hst->dmax_final;
     if (reason) *reason = r.hst->reason;
+    lease.idle = true;
   }
-  for (auto &e : ev) (void)hipEventDestroy(e);
-  (void)hipHostFree(r.hst);
   return rc;
 }
 }  // namespace
@@ -1187,15 +1339,11 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
   CHK(s.scratch(1, &run.st));
   unsigned long long *dslot;
   CHK(s.scratch(sor_pair_slot_words(), &dslot));
-  HIPCHK(hipHostMalloc((void **)&run.hst, sizeof(SorState)));
-  double *hfin = nullptr;
-  if (hipHostMalloc((void **)&hfin, 4 * sizeof(double)) != hipSuccess) {
-    (void)hipHostFree(run.hst);
-    return fail("multigrid: pinned allocation failed");
-  }
-  std::vector<hipEvent_t> ev(2);
-  for (auto &e : ev) (void)hipEventCreate(&e);
-  run.events = &ev;
+  HostLease lease;
+  CHK(lease.open());
+  run.hst = lease.h->hst;
+  double *hfin = lease.h->hfin;
+  run.events = &lease.h->ev;
   SorArgs<float, float> &a = run.a;
   a.rhs = nullptr;
   a.st = run.st;
@@ -1254,10 +1402,8 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
     }
     ++done;
   }
-  for (auto &e : ev) (void)hipEventDestroy(e);
-  (void)hipHostFree(run.hst);
-  (void)hipHostFree(hfin);
   if (rc != 0) return rc;
+  lease.idle = true;
   if (cycles) *cycles = done;
   if (resmax) *resmax = rmax;
   if (reason) *reason = why;
@@ -1346,7 +1492,10 @@ extern "C" int o3d_correct_velocity(double *ux, double *uy, double *uz, const do
   CHK(s.scratch(3, &fin));
   HIPCHK(launch_correct<double, double>(a, g_stream));
   FieldPartial r[3];
-  for (int c = 0; c < 3; ++c) CHK(finalize_to_host(a.part, a.tl.blocks(), 3, c, fin + c, &r[c]));
+  FinalizeSet sets[3];
+  for (int c = 0; c < 3; ++c) sets[c] = {a.part, a.tl.blocks(), 3, c, fin + c};
+  HIPCHK(launch_finalize_sets(sets, 3, g_stream));
+  HIPCHK(hipMemcpyAsync(r, fin, sizeof(r), hipMemcpyDeviceToHost, g_stream));
   CHK(s.finish());
   int diverged = 0;
   for (int c = 0; c < 3; ++c) {
@@ -1674,16 +1823,16 @@ struct Solver {
   size_t esz() const { return mixed ? 4 : 8; }
   template <typename T>
   int alloc(T **p_, size_t count) {
-    void *d = nullptr;
-    HIPCHK(hipMalloc(&d, count * sizeof(T)));
+    void *d = ScratchPool::get().allocate(count * sizeof(T));
+    if (!d) return fail("out of device memory (%zu bytes)", count * sizeof(T));
     HIPCHK(hipMemset(d, 0, count * sizeof(T)));
     allocs.push_back(d);
     *p_ = (T *)d;
     return 0;
   }
   int allocv(void **p_, size_t bytes) {
-    void *d = nullptr;
-    HIPCHK(hipMalloc(&d, bytes));
+    void *d = ScratchPool::get().allocate(bytes);
+    if (!d) return fail("out of device memory (%zu bytes)", bytes);
     HIPCHK(hipMemset(d, 0, bytes));
     allocs.push_back(d);
     *p_ = d;
