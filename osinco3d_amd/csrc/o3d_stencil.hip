@@ -134,44 +134,101 @@ __device__ __forceinline__ T d2(T m2, T m1, T z, T p1, T p2, const T *c) {
 // drop-ins).  which = axis*6 + (order-1)*3 + variant, variant 0 = _00,
 // 1 = p_11 (even), 2 = i_11 (odd); 18/19 = the 2D stubs derz_2dsim and
 // derzz_2dsim (src/derivation.f90:481-495, 934-948).
-template <typename T, int AXIS, int ORDER>
-__global__ void __launch_bounds__(256) der_kernel(T *__restrict__ df, const T *__restrict__ f,
-                                                  int nx, int ny, int nz, int variant, T ca,
-                                                  T cb, T cc) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  const int N = nx * ny * nz;
-  if (idx >= N) return;
-  const int i = idx % nx, j = (idx / nx) % ny, k = idx / (nx * ny);
-  const int n = AXIS == 0 ? nx : (AXIS == 1 ? ny : nz);
-  const int p = AXIS == 0 ? i : (AXIS == 1 ? j : k);
-  const int stride = AXIS == 0 ? 1 : (AXIS == 1 ? nx : nx * ny);
-  const int base = idx - p * stride;
+// What bounds it is memory; one node per thread spent its time on the index
+// divisions and ghost tests of every node instead.
+//
+// Along y and z a thread takes kDerRun nodes of its line: it loads the line once (22
+// independent loads in flight for 16 results; the positions, and with them the ghost
+// tests, are the same in the whole block).  Lines are numbered without gaps: along z
+// the nodes of a plane, along y (i, k).  185^3 FP64, first / second derivative: along
+// y 52 / 40 us and along z 56 / 47 us, now 21 / 20 us along either (4.9 TB/s).
+constexpr int kDerRun = 16;
+template <typename T, int ORDER>
+__global__ void __launch_bounds__(256) der_line_kernel(T *__restrict__ df,
+                                                       const T *__restrict__ f, int lines,
+                                                       int per, int jump, int n, int stride,
+                                                       int variant, T ca, T cb, T cc) {
+  constexpr int R = kDerRun, H = ORDER == 1 ? 3 : 2;
+  const int l = blockIdx.x * blockDim.x + threadIdx.x;
+  if (l >= lines) return;
+  const int base = l / per * jump + l % per;
+  const int p0 = blockIdx.y * R;
   const int bc = variant == 0 ? PERIODIC : FREE_SLIP;
-  const bool odd = variant == 2;
-  auto F = [&](int s) -> T {
-    if (variant == 3) {  // x-Dirichlet: extrapolated ends
-      const int q = p + s;
-      if (q < 0)
-        return xdir_extrap<T>(-q, f[base], f[base + stride], f[base + 2 * stride],
-                              f[base + 3 * stride]);
-      if (q > n - 1) {
-        const int e = base + (n - 1) * stride;
-        return xdir_extrap<T>(q - (n - 1), f[e], f[e - stride], f[e - 2 * stride],
-                              f[e - 3 * stride]);
-      }
-      return f[base + q * stride];
+  T v[R + 2 * H];
+#pragma unroll
+  for (int s = 0; s < R + 2 * H; ++s) {
+    const int q = p0 - H + s;
+    v[s] = T(0);
+    if (q < n + H) {
+      bool fl;
+      const T w = f[base + ghost_index(q, n, bc, fl) * stride];
+      v[s] = (fl && variant == 2) ? -w : w;
     }
-    bool fl;
-    const int q = ghost_index(p + s, n, bc, fl);
-    const T v = f[base + q * stride];
-    return (fl && odd) ? -v : v;
-  };
+  }
   const T c[3] = {ca, cb, cc};
-  if (ORDER == 1) {
-    if (variant == 1 && (p == 0 || p == n - 1)) { df[idx] = T(0); return; }
-    df[idx] = d1<T>(F(-3), F(-2), F(-1), F(1), F(2), F(3), c);
-  } else {
-    df[idx] = d2<T>(F(-2), F(-1), f[idx], F(1), F(2), c);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int p = p0 + r;
+    if (p >= n) break;
+    T d;
+    if constexpr (ORDER == 1) {
+      d = d1<T>(v[r], v[r + 1], v[r + 2], v[r + 4], v[r + 5], v[r + 6], c);
+      if (variant == 1 && (p == 0 || p == n - 1)) d = T(0);
+    } else {
+      d = d2<T>(v[r], v[r + 1], v[r + 2], v[r + 3], v[r + 4], c);
+    }
+    df[base + p * stride] = d;
+  }
+}
+
+// Along x a thread takes one x position on kDerRows rows: the neighbours' offsets and
+// signs are worked out once.  185^3 FP64: 43 -> 40 us (input from HBM) and 31 -> 23 us
+// (in the Infinity Cache).
+constexpr int kDerRows = 4;
+template <typename T, int ORDER, bool XDIR>
+__global__ void __launch_bounds__(256) der_row_kernel(T *__restrict__ df,
+                                                      const T *__restrict__ f, int nx, int rows,
+                                                      int variant, T ca, T cb, T cc) {
+  constexpr int R = kDerRows, H = ORDER == 1 ? 3 : 2;
+  const int l = blockIdx.x * blockDim.x + threadIdx.x;
+  const int g = l / nx, i = l - g * nx;
+  if (g * R >= rows) return;
+  const int bc = variant == 0 ? PERIODIC : FREE_SLIP;
+  int off[2 * H + 1];
+  bool neg[2 * H + 1];
+#pragma unroll
+  for (int s = -H; s <= H; ++s) {
+    bool fl = false;
+    off[s + H] = XDIR ? i + s : ghost_index(i + s, nx, bc, fl);
+    neg[s + H] = fl && variant == 2;
+  }
+  const T c[3] = {ca, cb, cc};
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int row = g * R + r;
+    if (row >= rows) break;
+    const T *fr = f + row * nx;
+    T v[2 * H + 1];
+#pragma unroll
+    for (int s = 0; s <= 2 * H; ++s) {
+      const int q = off[s];
+      if (XDIR && q < 0) {  // x-Dirichlet: extrapolated ends
+        v[s] = xdir_extrap<T>(-q, fr[0], fr[1], fr[2], fr[3]);
+      } else if (XDIR && q > nx - 1) {
+        v[s] = xdir_extrap<T>(q - (nx - 1), fr[nx - 1], fr[nx - 2], fr[nx - 3], fr[nx - 4]);
+      } else {
+        const T w = fr[q];
+        v[s] = neg[s] ? -w : w;
+      }
+    }
+    T d;
+    if constexpr (ORDER == 1) {
+      d = d1<T>(v[0], v[1], v[2], v[4], v[5], v[6], c);
+      if (variant == 1 && (i == 0 || i == nx - 1)) d = T(0);
+    } else {
+      d = d2<T>(v[0], v[1], v[2], v[3], v[4], c);
+    }
+    df[row * nx + i] = d;
   }
 }
 
@@ -198,11 +255,27 @@ hipError_t launch_der(int which, T *df, const T *f, int nx, int ny, int nz, doub
   double a, b, c;
   if (order == 1) { D1Coef k = d1coef(h); a = k.a; b = k.b; c = k.c; }
   else { D2Coef k = d2coef(h); a = k.a; b = k.b; c = k.c; }
-#define O3D_DER(AX, OR)                                                                   \
-  der_kernel<T, AX, OR><<<grd, blk, 0, s>>>(df, f, nx, ny, nz, variant, T(a), T(b), T(c))
-  if (axis == 0) { if (order == 1) O3D_DER(0, 1); else O3D_DER(0, 2); }
-  else if (axis == 1) { if (order == 1) O3D_DER(1, 1); else O3D_DER(1, 2); }
-  else { if (order == 1) O3D_DER(2, 1); else O3D_DER(2, 2); }
+  const auto blocks = [](long long n) { return (unsigned)((n + 255) / 256); };
+#define O3D_DER(KERNEL, GRID, ...) \
+  KERNEL<<<GRID, blk, 0, s>>>(df, f, __VA_ARGS__, variant, T(a), T(b), T(c))
+  if (axis == 0) {
+    const int rows = ny * nz;
+    const dim3 grid(blocks((long long)nx * ((rows + kDerRows - 1) / kDerRows)));
+    if (variant == 3) {
+      if (order == 1) O3D_DER((der_row_kernel<T, 1, true>), grid, nx, rows);
+      else O3D_DER((der_row_kernel<T, 2, true>), grid, nx, rows);
+    } else {
+      if (order == 1) O3D_DER((der_row_kernel<T, 1, false>), grid, nx, rows);
+      else O3D_DER((der_row_kernel<T, 2, false>), grid, nx, rows);
+    }
+  } else {
+    // Along y: lines (i, k), nx of them to a plane; along z: the nodes of a plane.
+    const int n = axis == 1 ? ny : nz, stride = axis == 1 ? nx : nx * ny;
+    const int per = axis == 1 ? nx : nx * ny, lines = axis == 1 ? nx * nz : nx * ny;
+    const dim3 grid(blocks(lines), (n + kDerRun - 1) / kDerRun);
+    if (order == 1) O3D_DER((der_line_kernel<T, 1>), grid, lines, per, nx * ny, n, stride);
+    else O3D_DER((der_line_kernel<T, 2>), grid, lines, per, nx * ny, n, stride);
+  }
 #undef O3D_DER
   return hipGetLastError();
 }

@@ -47,6 +47,18 @@ def test_derivatives_bit_exact(orc, shape):
         assert np.array_equal(df, exp), (which, np.abs(df - exp).max())
 
 
+# Lines of 16 nodes per thread along y and z, 4 rows per thread along x.
+@pytest.mark.parametrize("shape", [(16, 15, 65), (17, 32, 6), (33, 17, 7), (7, 6, 64)])
+def test_derivatives_at_run_edges(orc, shape):
+    f, = rand_fields(shape, 1, seed=18)
+    for which in range(18):
+        df = np.full_like(f, np.nan)
+        capi.der(which, df, f, 0.173)
+        axis, order, kind = which // 6, (which % 6) // 3 + 1, which % 3
+        exp = (orc.der1 if order == 1 else orc.der2)(f, axis, kind, 0.173)
+        assert np.array_equal(df, exp), which
+
+
 def test_derivatives_device_pointers(orc, gpu):
     torch = gpu
     f, = rand_fields((14, 18, 66), 1, seed=4)
