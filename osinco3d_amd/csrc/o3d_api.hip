@@ -1364,8 +1364,10 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
   double rmax = 0.0, rmax_old = 1609.0;
   while (rc == 0) {
     // r = rhs - L pp (FP64 arithmetic), colour-split in FP32, and e = 0.
-    if (launch_residual_norm_pair<double>(p, p, rhs_d, part, fin, nx, ny, nz, per, c.ox, c.oy,
-                                          c.oz, c.A, g_stream, R, E) != hipSuccess ||
+    // The coarse-grid correction writes all of e itself.
+    if (launch_residual_norm_pair<double>(nullptr, p, rhs_d, part, fin, nx, ny, nz, per, c.ox,
+                                          c.oy, c.oz, c.A, g_stream, R,
+                                          H.levels > 0 ? nullptr : E) != hipSuccess ||
         hipMemcpyAsync(hfin, fin, 4 * sizeof(double), hipMemcpyDeviceToHost, g_stream) !=
             hipSuccess ||
         hipStreamSynchronize(g_stream) != hipSuccess) {

@@ -178,8 +178,8 @@ hipError_t launch_fold_split(double *p, const float *e, int nx, int ny, int nz, 
 // FP64 residual norms of two iterates p0, p1 (r = rhs - L p) in one launch:
 // out (device, 4 doubles) = (max |r0|, sum r0^2, max |r1|, sum r1^2).  part
 // holds 4 * residual_blocks(nx, ny, nz) doubles.  With r1s (nx even), the
-// residual of p1 is also stored colour-split in FP32 and e1s is zeroed, as
-// launch_residual_split would do for p1.  With p0 null, the first pair
+// residual of p1 is also stored colour-split in FP32 and e1s (unless null) is
+// zeroed, as launch_residual_split would do for p1.  With p0 null, the first pair
 // comes from the part0 records launch_guess_residual wrote for the same p0
 // and rhs (bit-identical to computing them here).
 template <typename TR>

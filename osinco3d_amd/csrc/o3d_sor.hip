@@ -1026,7 +1026,7 @@ hipError_t launch_fold(double *p, const float *e, int n, hipStream_t s) {
 // Residual norms of two iterates against one rhs in one launch: per block
 // (max |r0|, sum r0^2, max |r1|, sum r1^2).  With r1s, the residual of p1 is
 // also stored colour-split in FP32 (r1s, the first correction solve's rhs
-// when p1 becomes the iterate) and e1s is zeroed.
+// when p1 becomes the iterate) and e1s, if given, is zeroed.
 template <typename TR>
 __global__ void __launch_bounds__(RNT) residual_norm_pair_kernel(
     const double *__restrict__ p0, const double *__restrict__ p1, const TR *__restrict__ rhs,
@@ -1049,7 +1049,7 @@ __global__ void __launch_bounds__(RNT) residual_norm_pair_kernel(
                       const size_t o = (size_t)(nx / 2) * (j + (size_t)ny * k) + (i >> 1) +
                                        (((i + j + k) & 1) ? half : 0);
                       r1s[o] = (float)r;
-                      e1s[o] = 0.0f;
+                      if (e1s) e1s[o] = 0.0f;
                     }
                   });
   m0 = block_max<RNT / O3D_WAVE>(m0, sc);
@@ -1092,8 +1092,7 @@ hipError_t launch_residual_norm_pair(const double *p0, const double *p1, const T
                                      const int per[3], double ox, double oy, double oz, double A,
                                      hipStream_t s, float *r1s, float *e1s,
                                      const double *part0) {
-  if (r1s && (nx % 2 != 0 || !e1s)) return hipErrorInvalidValue;
-  if (!p0 && !part0) return hipErrorInvalidValue;
+  if (r1s && nx % 2 != 0) return hipErrorInvalidValue;
   residual_norm_pair_kernel<TR><<<residual_grid(nx, ny, nz), RNT, 0, s>>>(
       p0, p1, rhs, part, r1s, e1s, nx, ny, nz, per[0], per[1], per[2], ox, oy, oz, A);
   residual_norm_final_kernel<<<1, 1024, 0, s>>>(part, p0 ? nullptr : part0,
