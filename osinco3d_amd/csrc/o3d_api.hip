@@ -2120,6 +2120,7 @@ int solver_poisson_mixed(Solver &S, o3d_step_info *info) {
   int capped = 0;  // consecutive correction solves that ended on their sweep cap
   // The judge sweep summed the p it wrote and nothing has changed p since.
   bool sum_ok = false;
+  bool fold_next = false;  // E[0] is still to be added to P[cur]
   while (total < p.kmax) {
     sum_ok = false;
     int per[3];
@@ -2131,9 +2132,20 @@ int solver_poisson_mixed(Solver &S, o3d_step_info *info) {
     if (split && cycles == 0 && S.r_ready) {
       // r and e = 0 already written by the warm-start acceptance check.
     } else if (split) {
-      HIPCHK(launch_residual_split<float>(S.P[S.cur], (const float *)S.rhs, S.R, S.E[0], p.nx,
-                                          p.ny, p.nz, per, S.sc.ox, S.sc.oy, S.sc.oz, S.sc.A,
-                                          g_stream));
+      // The coarse-grid correction writes all of e; without it e starts at 0.
+      if (fold_next) {
+        HIPCHK(launch_fold_residual_split<float>(S.P[S.cur], S.E[0], (const float *)S.rhs,
+                                                 S.P[1 - S.cur], S.R, mgc ? nullptr : S.E[1],
+                                                 p.nx, p.ny, p.nz, per, S.sc.ox, S.sc.oy, S.sc.oz,
+                                                 S.sc.A, g_stream));
+        S.cur = 1 - S.cur;
+        if (!mgc) std::swap(S.E[0], S.E[1]);
+        fold_next = false;
+      } else {
+        HIPCHK(launch_residual_split<float>(S.P[S.cur], (const float *)S.rhs, S.R,
+                                            mgc ? nullptr : S.E[0], p.nx, p.ny, p.nz, per,
+                                            S.sc.ox, S.sc.oy, S.sc.oz, S.sc.A, g_stream));
+      }
       if (mgc) {
         // The start of this correction solve: the coarse-grid correction of
         // its residual (cycle 0 starts from a guess that already had one).
@@ -2190,12 +2202,12 @@ int solver_poisson_mixed(Solver &S, o3d_step_info *info) {
     // p += e: with colour-split sweeps and a judge sweep next, folded into
     // the judge's loads (it reads p + e and writes the other buffer) instead
     // of a pass of its own; the sums are the same, so are the iterates.
+    // Before another correction solve (total < kmax there, so one follows) it joins
+    // that solve's residual.
     const bool fuse = split && to_judge;
-    if (!fuse) {
-      if (split) HIPCHK(launch_fold_split(S.P[S.cur], S.E[0], p.nx, p.ny, p.nz, g_stream));
-      else HIPCHK(launch_fold(S.P[S.cur], r.result(sweeps), n, g_stream));
-    }
+    if (!split) HIPCHK(launch_fold(S.P[S.cur], r.result(sweeps), n, g_stream));
     if (!to_judge) {
+      fold_next = split;
       ++capped;
       continue;
     }

@@ -169,11 +169,19 @@ hipError_t launch_guess_residual(const double *p, const float *e, const TR *rhs,
                                  float *r, int nx, int ny, int nz, const int per[3], double ox,
                                  double oy, double oz, double A, hipStream_t s,
                                  double *part0 = nullptr);
-// The same with r and e colour-split (red half-array, then black).
+// The same with r and e colour-split (red half-array, then black); e may be null
+// where the caller writes all of it.
 template <typename TR>
 hipError_t launch_residual_split(const double *p, const TR *rhs, float *r, float *e, int nx,
                                  int ny, int nz, const int per[3], double ox, double oy,
                                  double oz, double A, hipStream_t s);
+// q = p + e (e colour-split) and launch_residual_split's r of q in one pass; q and ez
+// (zeroed, may be null) are other buffers than p and e.
+template <typename TR>
+hipError_t launch_fold_residual_split(const double *p, const float *e, const TR *rhs, double *q,
+                                      float *r, float *ez, int nx, int ny, int nz,
+                                      const int per[3], double ox, double oy, double oz, double A,
+                                      hipStream_t s);
 hipError_t launch_fold_split(double *p, const float *e, int nx, int ny, int nz, hipStream_t s);
 // FP64 residual norms of two iterates p0, p1 (r = rhs - L p) in one launch:
 // out (device, 4 doubles) = (max |r0|, sum r0^2, max |r1|, sum r1^2).  part
@@ -181,7 +189,7 @@ hipError_t launch_fold_split(double *p, const float *e, int nx, int ny, int nz, 
 // residual of p1 is also stored colour-split in FP32 and e1s (unless null) is
 // zeroed, as launch_residual_split would do for p1.  With p0 null, the first pair
 // comes from the part0 records launch_guess_residual wrote for the same p0
-// and rhs (bit-identical to computing them here).
+// and rhs (bit-identical to computing them here), or is zero without them.
 template <typename TR>
 hipError_t launch_residual_norm_pair(const double *p0, const double *p1, const TR *rhs,
                                      double *part, double *out, int nx, int ny, int nz,

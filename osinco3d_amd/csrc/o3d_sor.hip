@@ -605,7 +605,7 @@ int residual_blocks(int nx, int ny, int nz) {
 // buffered (one barrier per plane); each thread keeps its own column's
 // planes k-1, k, k+1 (and k+2 in flight) and the rhs in registers.  A node
 // value is then loaded once per plane, plus the halo, instead of once per
-// neighbour reading it.  ld(o, v) fills v[0..NF) for node offset o;
+// neighbour reading it.  ld(o, d, v) fills v[0..NF) for node offset o of colour d;
 // f(o, i, j, k, nb, rh) receives, per field, the neighbour values
 // nb[f][0..6] = (x-1, x+1, y-1, y+1, z-1, z+1, centre) and the rhs, in the
 // operation order every residual kernel uses.  Every thread of the block
@@ -631,19 +631,26 @@ __device__ __forceinline__ void tile_march(LD &&ld, const TR *__restrict__ rhs, 
   const int cxr = act ? sor_ghost(i + 1, nx, px) + nx * j : 0;
   const int cyl = act ? i + nx * sor_ghost(j - 1, ny, py) : 0;
   const int cyr = act ? i + nx * sor_ghost(j + 1, ny, py) : 0;
-  auto zo = [&](int k) { return plane * (size_t)sor_ghost(k, nz, pz); };
+  // Colours (parity of i + j) of the same nodes.
+  const int dc = (i + j) & 1;
+  const int dxl = (sor_ghost(i - 1, nx, px) + j) & 1, dxr = (sor_ghost(i + 1, nx, px) + j) & 1;
+  const int dyl = (i + sor_ghost(j - 1, ny, py)) & 1, dyr = (i + sor_ghost(j + 1, ny, py)) & 1;
+  auto at = [&](int o, int d, int k, double *v) __attribute__((always_inline)) {
+    const int kk = sor_ghost(k, nz, pz);
+    ld(o + plane * (size_t)kk, (d + kk) & 1, v);
+  };
   double cm[NF], c0[NF], cp[NF], cn[NF], h[4][NF];
   double rh = 0.0, rn = 0.0;
   __syncthreads();  // a previous march of this block may still read the tile
   if (act) {
-    ld(c + zo(k0 - 1), cm);
-    ld(c + zo(k0), c0);
-    ld(c + zo(k0 + 1), cp);
+    at(c, dc, k0 - 1, cm);
+    at(c, dc, k0, c0);
+    at(c, dc, k0 + 1, cp);
     rh = (double)rhs[c + plane * k0];
-    if (hxl) ld(cxl + zo(k0), h[0]);
-    if (hxr) ld(cxr + zo(k0), h[1]);
-    if (hyl) ld(cyl + zo(k0), h[2]);
-    if (hyr) ld(cyr + zo(k0), h[3]);
+    if (hxl) at(cxl, dxl, k0, h[0]);
+    if (hxr) at(cxr, dxr, k0, h[1]);
+    if (hyl) at(cyl, dyl, k0, h[2]);
+    if (hyr) at(cyr, dyr, k0, h[3]);
 #pragma unroll
     for (int q = 0; q < NF; ++q) {
       tl[0][q][ty + 1][tx + 1] = c0[q];
@@ -660,13 +667,13 @@ __device__ __forceinline__ void tile_march(LD &&ld, const TR *__restrict__ rhs, 
     if (act) {
       // Loads for later planes first: the column's plane k+2, the rhs and
       // the halo of plane k+1.
-      ld(c + zo(k + 2), cn);
+      at(c, dc, k + 2, cn);
       if (more) {
         rn = (double)rhs[c + plane * (k + 1)];
-        if (hxl) ld(cxl + zo(k + 1), h[0]);
-        if (hxr) ld(cxr + zo(k + 1), h[1]);
-        if (hyl) ld(cyl + zo(k + 1), h[2]);
-        if (hyr) ld(cyr + zo(k + 1), h[3]);
+        if (hxl) at(cxl, dxl, k + 1, h[0]);
+        if (hxr) at(cxr, dxr, k + 1, h[1]);
+        if (hyl) at(cyl, dyl, k + 1, h[2]);
+        if (hyr) at(cyr, dyr, k + 1, h[3]);
       }
       double nb[NF][7];
 #pragma unroll
@@ -703,13 +710,13 @@ __device__ __forceinline__ void tile_march(LD &&ld, const TR *__restrict__ rhs, 
 }
 
 // f(offset of (i, j, k), i, j, k, p(i, j, k), residual) for every node of
-// the block's tile, the iterate's value at offset o being ld(o).
+// the block's tile, the iterate's value at offset o being ld(o, d), d its colour.
 template <typename TR, typename LD, typename F>
 __device__ __forceinline__ void residual_column_ld(LD &&ld, const TR *__restrict__ rhs, int nx,
                                                    int ny, int nz, int px, int py, int pz,
                                                    double ox, double oy, double oz, double A,
                                                    F &&f) {
-  tile_march<1>([&](size_t o, double *v) { v[0] = ld(o); }, rhs, nx, ny, nz, px, py, pz,
+  tile_march<1>([&](size_t o, int d, double *v) { v[0] = ld(o, d); }, rhs, nx, ny, nz, px, py, pz,
                 [&](size_t o, int i, int j, int k, const double (*nb)[7], double rh) {
                   const double lap = ox * (nb[0][0] + nb[0][1]) + oy * (nb[0][2] + nb[0][3]) +
                                      oz * (nb[0][4] + nb[0][5]) + A * nb[0][6];
@@ -722,7 +729,7 @@ __device__ __forceinline__ void residual_column(const double *__restrict__ p,
                                                 const TR *__restrict__ rhs, int nx, int ny,
                                                 int nz, int px, int py, int pz, double ox,
                                                 double oy, double oz, double A, F &&f) {
-  residual_column_ld([&](size_t o) { return p[o]; }, rhs, nx, ny, nz, px, py, pz, ox, oy, oz,
+  residual_column_ld([&](size_t o, int) { return p[o]; }, rhs, nx, ny, nz, px, py, pz, ox, oy, oz,
                      A, [&](size_t o, int i, int j, int k, double, double r) {
                        f(o, i, j, k, r);
                      });
@@ -971,9 +978,46 @@ __global__ void __launch_bounds__(RNT) residual_split_kernel(const double *__res
                     const size_t o = (size_t)(nx / 2) * (j + (size_t)ny * k) + (i >> 1) +
                                      (((i + j + k) & 1) ? half : 0);
                     r[o] = (float)res;
-                    e[o] = 0.0f;
+                    if (e) e[o] = 0.0f;
                   });
 }
+
+// The end of one correction solve and the start of the next in one pass: q = p + e
+// (e colour-split, fold_split_kernel's sums), r = rhs - L q colour-split as
+// residual_split_kernel gives it for that q, and ez = 0 where it is asked for.  q
+// and ez are other buffers than p and e, which neighbouring tiles still read.
+// Memory bounds it: 512x384x256 fold 181 us + residual 242 -> 379 us, 384x256x128
+// 53 + 64 -> 98; tiles of 8 rows and 32 planes take 356 and 101.
+template <typename TR>
+__global__ void __launch_bounds__(RNT) fold_residual_split_kernel(
+    const double *__restrict__ p, const float *__restrict__ e, const TR *__restrict__ rhs,
+    double *__restrict__ q, float *__restrict__ r, float *__restrict__ ez, int nx, int ny, int nz,
+    int px, int py, int pz, double ox, double oy, double oz, double A) {
+  const size_t half = (size_t)nx * ny * nz / 2;
+  residual_column_ld(
+      [&](size_t o, int d) { return p[o] + (double)e[(o >> 1) + (d ? half : 0)]; }, rhs, nx, ny,
+      nz, px, py, pz, ox, oy, oz, A, [&](size_t o, int i, int j, int k, double v, double res) {
+        const size_t s = (o >> 1) + (((i + j + k) & 1) ? half : 0);
+        q[o] = v;
+        r[s] = (float)res;
+        if (ez) ez[s] = 0.0f;
+      });
+}
+
+template <typename TR>
+hipError_t launch_fold_residual_split(const double *p, const float *e, const TR *rhs, double *q,
+                                      float *r, float *ez, int nx, int ny, int nz,
+                                      const int per[3], double ox, double oy, double oz, double A,
+                                      hipStream_t s) {
+  if (nx % 2 != 0 || q == p || ez == e) return hipErrorInvalidValue;
+  fold_residual_split_kernel<TR><<<residual_grid(nx, ny, nz), RNT, 0, s>>>(
+      p, e, rhs, q, r, ez, nx, ny, nz, per[0], per[1], per[2], ox, oy, oz, A);
+  return hipGetLastError();
+}
+template hipError_t launch_fold_residual_split<float>(const double *, const float *,
+                                                      const float *, double *, float *, float *,
+                                                      int, int, int, const int[3], double, double,
+                                                      double, double, hipStream_t);
 
 template <typename TR>
 hipError_t launch_residual_split(const double *p, const TR *rhs, float *r, float *e, int nx,

@@ -116,6 +116,28 @@ def test_mixed_precision_tracks_fp64():
     b.close()
 
 
+@pytest.mark.parametrize("opt", [{"inner_max": 7}, {"inner_max": 8},
+                                 {"inner_max": 5, "coarse_cycles": 1, "smooth_sweeps": 4}])
+def test_capped_correction_solves_reach_fp64(opt):
+    """Correction solves that end on their sweep cap: the next one's residual
+    pass adds their result to the pressure (partial tiles, both buffers)."""
+    cfg = tgv_config(40, 3, 3)
+    f = taylor_green(cfg)
+    a, b = Solver(cfg, FP64), Solver(cfg, MIXED, **opt)
+    a.upload(*f)
+    b.upload(*f)
+    for itime in range(1, 4):
+        a.step(itime)
+        ib = b.step(itime)
+        assert ib["sor_reason"] == 0 and ib["sor_dmax"] < cfg.eps
+        assert ib["refinements"] >= 2
+    # The tolerance of test_mixed_precision_tracks_fp64.
+    for x, y in zip(a.download()[:3], b.download()[:3]):
+        assert np.abs(x - y).max() <= 1e-5
+    a.close()
+    b.close()
+
+
 def _gold(name):
     import os
     return np.load(os.path.join(os.path.dirname(__file__), "golden", name), allow_pickle=False)
