@@ -481,10 +481,10 @@ __device__ __forceinline__ bf16x8 run_of(const bf16x8 *v, int c) {
   return o;
 }
 
-__global__ void __launch_bounds__(256) x_runs_kernel(const bf16 *__restrict__ x,
-                                                     bf16 *__restrict__ xt, Runs R, int C) {
+// The copy of x, 256 threads of which this is number idx.
+__device__ __forceinline__ void x_runs(const bf16 *__restrict__ x, bf16 *__restrict__ xt,
+                                       const Runs &R, int C, int idx) {
   const int G = C >> 3, nh = R.nr + 2;
-  const int idx = blockIdx.x * 256 + threadIdx.x;
   if (idx >= R.ny * R.nz * nh * G) return;
   const int cg = idx % G, q = idx / G;
   const int r = q % nh, row = q / nh;
@@ -618,14 +618,28 @@ inline WgradPlan wgrad_plan(const Runs &R, int ci, int co) {
   return p;
 }
 
-// dst[e] += sum_s part[s][e]: 64 entries per block, the slabs dealt to its 4
-// waves, the waves' sums added in wave order.
-__global__ void __launch_bounds__(256) reduce_parts_kernel(const float *__restrict__ part,
-                                                           int nparts, int entries,
-                                                           float *__restrict__ dst) {
+// dst[e] += sum_s part[s][e] of every weight, bias and head gradient in one launch:
+// 64 entries per block, the slabs dealt to its 4 waves, the waves' sums added in wave
+// order.  (A launch per set was 29 of them, 2.8 us each for a 32^3 network.)
+struct ReduceSet {
+  const float *part;
+  float *dst;
+  int nparts, entries, block0;  // first block of the set
+};
+constexpr int kReduceSets = 29;
+struct ReduceSets {
+  ReduceSet s[kReduceSets];
+  int n, blocks;
+};
+__global__ void __launch_bounds__(256) reduce_parts_kernel(const ReduceSets a) {
   __shared__ float sw[4][64];
+  int m = 0;
+  while (m + 1 < a.n && (int)blockIdx.x >= a.s[m + 1].block0) ++m;
+  const ReduceSet &t = a.s[m];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int e = blockIdx.x * 64 + lane;
+  const int e = ((int)blockIdx.x - t.block0) * 64 + lane;
+  const int entries = t.entries, nparts = t.nparts;
+  const float *part = t.part;
   float s = 0.f;
   if (e < entries) {
 #pragma unroll 8
@@ -633,7 +647,8 @@ __global__ void __launch_bounds__(256) reduce_parts_kernel(const float *__restri
   }
   sw[wv][lane] = s;
   __syncthreads();
-  if (wv == 0 && e < entries) dst[e] += ((sw[0][lane] + sw[1][lane]) + sw[2][lane]) + sw[3][lane];
+  if (wv == 0 && e < entries)
+    t.dst[e] += ((sw[0][lane] + sw[1][lane]) + sw[2][lane]) + sw[3][lane];
 }
 
 // ------------------------------------------------------- elementwise pieces
@@ -803,12 +818,21 @@ __global__ void __launch_bounds__(256) up_bwd_kernel(const float *__restrict__ g
 // value to an LDS word per channel: 45.5 us for 16 channels of 128x96x64,
 // now 37.6 us including the channel-major copy, and no gradient buffer needs
 // clearing.)
+// The blocks from nact on copy the layer's input x channel-major (x_runs): the
+// weight gradient needs both, neither fills the chip on the coarse levels, and a
+// launch costs as much as either does there.
 __global__ void __launch_bounds__(256) act_bwd_kernel(const float *__restrict__ g,
                                                       const bf16 *__restrict__ y,
                                                       bf16 *__restrict__ dz,
                                                       float *__restrict__ gskip,
                                                       bf16 *__restrict__ dzt,
-                                                      float *__restrict__ part, Runs R, int C) {
+                                                      float *__restrict__ part, Runs R, int C,
+                                                      int nact, const bf16 *__restrict__ x,
+                                                      bf16 *__restrict__ xt, int ci) {
+  if ((int)blockIdx.x >= nact) {
+    x_runs(x, xt, R, ci, ((int)blockIdx.x - nact) * 256 + (int)threadIdx.x);
+    return;
+  }
   __shared__ float sb[4][128];
   const int G = C >> 3;
   const int n = R.ny * R.nz * R.nr * G;
@@ -819,7 +843,7 @@ __global__ void __launch_bounds__(256) act_bwd_kernel(const float *__restrict__ 
   // The stride is a multiple of G (a power of two up to 16), so a thread's
   // channels stay the same.
   const int cg = threadIdx.x & (G - 1);
-  for (int idx = blockIdx.x * 256 + threadIdx.x; idx < n; idx += gridDim.x * 256) {
+  for (int idx = blockIdx.x * 256 + threadIdx.x; idx < n; idx += nact * 256) {
     const int q = idx / G;
     const int row = q / R.nr, r = q - row * R.nr;
     bf16x8 h[8];
@@ -1002,8 +1026,11 @@ struct Net {
   float *gbuf = nullptr;   // FP32 activation gradients (one arena)
   float *g_d0, *g_d0a, *g_u0, *g_d1, *g_d1a, *g_u1, *g_d2, *g_d2a, *g_u2, *g_e3, *g_e3a, *g_p3,
       *g_e2, *g_e2a, *g_p2, *g_e1, *g_e1a, *g_p1, *g_e0, *g_e0a;
-  float *part = nullptr;   // partial sums of the weight gradients
-  float *bpart = nullptr;  // partial sums of the bias and head gradients
+  float *part = nullptr;   // partial sums of the gradients (owns dzt and xt)
+  // Of each layer's weights and bias, and of the head: summed at the end of a
+  // backward pass.
+  float *wpart[14], *bpart[15];
+  ReduceSets sets;
   double *mse_part = nullptr;
   double *hpart = nullptr;
   void *act_arena = nullptr;
@@ -1071,6 +1098,11 @@ Runs runs_of(const Net &n, int level) {
 
 // Blocks of the bias and head gradient kernels, at most (their partial sums).
 constexpr int kBiasBlocks = 1024;
+// Blocks of act_bwd_kernel that work on a layer's output, and of head_bwd_kernel.
+int act_blocks(const Runs &R, int co) {
+  return std::min(kBiasBlocks, (R.rows() * R.nr * (co / 8) + 255) / 256);
+}
+int head_blocks(const Net &n) { return (int)std::min<size_t>(kBiasBlocks, (n.V[0] + 255) / 256); }
 
 int alloc_activations(Net &n, int nx, int ny, int nz) {
   if (nx % 8 || ny % 8 || nz % 8)
@@ -1117,23 +1149,34 @@ int alloc_activations(Net &n, int nx, int ny, int nz) {
     *g.p = (float *)p;
     p += ((n.V[g.level] * g.ch * 4 + 255) / 256) * 256;
   }
-  // The weight gradient's operands and partial sums, for its largest layer.
-  size_t zt = 0, xt = 0, np = 0;
-  for (const Conv &c : n.conv) {
+  // The weight gradient's operands, for its largest layer, and every layer's partial
+  // sums.
+  size_t zt = 0, xt = 0;
+  auto up = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+  size_t wb[14], bb[15];
+  total = 0;
+  for (int li = 0; li < 14; ++li) {
+    const Conv &c = n.conv[li];
     const Runs R = runs_of(n, c.level);
     const WgradPlan w = wgrad_plan(R, c.ci, c.co);
     zt = std::max(zt, R.dz_plane() * c.co);
     xt = std::max(xt, R.x_plane() * c.ci);
-    np = std::max(np, (size_t)w.slabs * c.co * 27 * c.ci);
+    wb[li] = up((size_t)w.slabs * c.co * 27 * c.ci * 4);
+    bb[li] = up((size_t)act_blocks(R, c.co) * c.co * 4);
+    total += wb[li] + bb[li];
   }
-  const size_t zb = (zt * sizeof(bf16) + 255) / 256 * 256, xb = (xt * sizeof(bf16) + 255) / 256 * 256;
-  const size_t pb = (np * 4 + 255) / 256 * 256;
+  bb[14] = up((size_t)head_blocks(n) * 17 * 4);
+  total += bb[14] + up(zt * sizeof(bf16)) + up(xt * sizeof(bf16));
   p = nullptr;
-  NNCHK(hipMalloc((void **)&p, zb + xb + pb + (size_t)kBiasBlocks * 128 * 4));
-  n.part = (float *)p;  // owns the four
-  n.bpart = (float *)(p + pb);
-  n.dzt = (bf16 *)(p + pb + (size_t)kBiasBlocks * 128 * 4);
-  n.xt = (bf16 *)((char *)n.dzt + zb);
+  NNCHK(hipMalloc((void **)&p, total));
+  n.part = (float *)p;
+  for (int li = 0; li < 15; ++li) {
+    if (li < 14) { n.wpart[li] = (float *)p; p += wb[li]; }
+    n.bpart[li] = (float *)p;
+    p += bb[li];
+  }
+  n.dzt = (bf16 *)p;
+  n.xt = (bf16 *)(p + up(zt * sizeof(bf16)));
   return 0;
 }
 
@@ -1222,8 +1265,10 @@ bool conv_fwd_up(Net &n, int li, const bf16 *xc, const bf16 *skip, bf16 *y, int 
   return true;
 }
 
-void reduce_parts(const float *part, int nparts, int entries, float *dst) {
-  reduce_parts_kernel<<<(entries + 63) / 64, 256, 0, st()>>>(part, nparts, entries, dst);
+// Adds a set to those the end of the backward pass sums.
+void reduce_parts(Net &n, const float *part, int nparts, int entries, float *dst) {
+  n.sets.s[n.sets.n++] = {part, dst, nparts, entries, n.sets.blocks};
+  n.sets.blocks += (entries + 63) / 64;
 }
 
 // Backward of y = act(conv(x) + b + skip): gy (FP32) -> dz; gskip = dz;
@@ -1233,26 +1278,23 @@ int conv_bwd(Net &n, int li, const float *gy, const bf16 *y, const bf16 *x, floa
   const Conv &c = n.conv[li];
   const int L = c.level;
   const Runs R = runs_of(n, L);
-  const int work = R.rows() * R.nr * (c.co / 8);
-  const int blocks = std::min(kBiasBlocks, (work + 255) / 256);
-  act_bwd_kernel<<<blocks, 256, 0, st()>>>(gy, y, gx ? n.dz : nullptr, gskip, n.dzt, n.bpart, R,
-                                           c.co);
+  const int blocks = act_blocks(R, c.co);
+  const int xw = (R.rows() * (R.nr + 2) * (c.ci / 8) + 255) / 256;
+  act_bwd_kernel<<<blocks + xw, 256, 0, st()>>>(gy, y, gx ? n.dz : nullptr, gskip, n.dzt,
+                                                n.bpart[li], R, c.co, blocks, x, n.xt, c.ci);
   NNCHK(hipGetLastError());
-  reduce_parts(n.bpart, blocks, c.co, n.G + c.boff);
+  reduce_parts(n, n.bpart[li], blocks, c.co, n.G + c.boff);
   // Weight gradient.
-  const int xw = R.rows() * (R.nr + 2) * (c.ci / 8);
-  x_runs_kernel<<<(xw + 255) / 256, 256, 0, st()>>>(x, n.xt, R, c.ci);
-  NNCHK(hipGetLastError());
+  float *part = n.wpart[li];
   const WgradPlan w = wgrad_plan(R, c.ci, c.co);
   const dim3 g1(w.tiles, w.slabs);
-  if (w.wc == 4) wgrad_kernel<4><<<g1, 256, 0, st()>>>(n.dzt, n.xt, n.part, R, c.ci, c.co, w.per);
+  if (w.wc == 4) wgrad_kernel<4><<<g1, 256, 0, st()>>>(n.dzt, n.xt, part, R, c.ci, c.co, w.per);
   else if (w.wc == 2)
-    wgrad_kernel<2><<<g1, 256, 0, st()>>>(n.dzt, n.xt, n.part, R, c.ci, c.co, w.per);
+    wgrad_kernel<2><<<g1, 256, 0, st()>>>(n.dzt, n.xt, part, R, c.ci, c.co, w.per);
   else
-    wgrad_kernel<1><<<g1, 256, 0, st()>>>(n.dzt, n.xt, n.part, R, c.ci, c.co, w.per);
+    wgrad_kernel<1><<<g1, 256, 0, st()>>>(n.dzt, n.xt, part, R, c.ci, c.co, w.per);
   NNCHK(hipGetLastError());
-  reduce_parts(n.part, w.slabs, c.co * 27 * c.ci, n.G + c.woff);
-  NNCHK(hipGetLastError());
+  reduce_parts(n, part, w.slabs, c.co * 27 * c.ci, n.G + c.woff);
   if (gx) {
     ConvArgs<float> a;
     a.x = n.dz; a.w = c.wb; a.bias = nullptr; a.skip = nullptr; a.y = gx;
@@ -1318,12 +1360,12 @@ int forward(Net &n, const float *in, float *out) {
 int backward(Net &n, const float *dout) {
   // Every activation gradient is written by its first reader's pass and only
   // added to by pool_bwd_kernel, so none needs clearing.
-  const int hb = (int)std::min<size_t>(kBiasBlocks, (n.V[0] + 255) / 256);
-  head_bwd_kernel<<<hb, 256, 0, st()>>>(dout, n.d0, n.W + n.head_off, n.g_d0, n.bpart,
+  const int hb = head_blocks(n);
+  n.sets.n = n.sets.blocks = 0;
+  head_bwd_kernel<<<hb, 256, 0, st()>>>(dout, n.d0, n.W + n.head_off, n.g_d0, n.bpart[14],
                                         (int)n.V[0]);
   NNCHK(hipGetLastError());
-  reduce_parts(n.bpart, hb, 17, n.G + n.head_off);
-  NNCHK(hipGetLastError());
+  reduce_parts(n, n.bpart[14], hb, 17, n.G + n.head_off);
   NCHK(conv_bwd(n, 13, n.g_d0, n.d0, n.d0a, nullptr, n.g_d0a));
   if (n.up_stale[0]) {  // the forward pass read d1 up-sampled without forming u0
     up_fwd_kernel<<<elem_blocks(n.V[0] * 4), 256, 0, st()>>>(n.d1, n.u0, n.nx[0], n.ny[0],
@@ -1367,6 +1409,7 @@ int backward(Net &n, const float *dout) {
     n.xin_stale = false;
   }
   NCHK(conv_bwd(n, 0, n.g_e0a, n.e0a, n.xin, nullptr, nullptr));
+  reduce_parts_kernel<<<n.sets.blocks, 256, 0, st()>>>(n.sets);
   NNCHK(hipGetLastError());
   return 0;
 }
