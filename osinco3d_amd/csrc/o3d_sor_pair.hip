@@ -39,9 +39,9 @@
 // every second launch marches from the other end, towards what the last one
 // left in the Infinity Cache (FP32 512x384x256 173 -> 156 us, FP64 320^3 199 ->
 // 188).  Per two iterations, launches of
-// one colour in place / this kernel: FP64 64^3 27.1 / 15.2 us, 128^3 36.7 /
-// 24.2, 256^3 186 / 106, 512x384x256 696 / 306; FP32 64^3 27.2 / 14.5, 256^3
-// 98 / 54, 384x256x128 93 / 38, 512x384x256 327 / 156 (the figures hold the
+// one colour in place / this kernel: FP64 128^3 36.7 / 24.2 us
+// (23 since the launch's maxima go by DPP), 256^3 186 / 106, 512x384x256 696 / 306;
+// FP32 256^3 98 / 54, 384x256x128 93 / 38, 512x384x256 327 / 156 (the figures hold the
 // host's share of a batch of launches, about 3 us).
 #include <algorithm>
 #include <utility>
@@ -243,6 +243,54 @@ __device__ __forceinline__ PairStep pair_decide(const SorSched &P, double da, do
   return s;
 }
 
+// What block 0 leaves of the launch's action: the result of the solve, or the
+// next launch's view of this one and its cleared dmax slots.
+template <typename T>
+__device__ __forceinline__ void pair_record(const PairStep &s, const SorPairArgs<T> &a, int tid,
+                                            int threads) {
+  SorState *st = a.st;
+  if (s.done) {
+    if (tid == 0) {
+      st->done = 1;
+      st->reason = s.reason;
+      st->exit_iter = s.reason == 2 ? a.kmax + 1 : s.sweeps;
+      st->sweeps = s.sweeps;
+      st->result = s.result;
+      st->dmax_final = s.dlast;
+      st->omega_final = s.omega;
+    }
+    return;
+  }
+  if (tid == 0) {
+    st->sched[(a.launch + 1) & 1] = {s.it0, s.n, s.src, 0, s.d_prev, s.om_a, s.om_b};
+    st->sweeps = s.it0 + s.n - 1;
+  }
+  unsigned long long *next =
+      a.dslot + (size_t)((a.launch + 1) % kPairSets) * 2 * kPairSlots * kPairStride;
+  for (int q = tid; q < 2 * kPairSlots; q += threads) next[(size_t)q * kPairStride] = 0ull;
+}
+
+// The block's dmax of both iterations into the launch's slots.
+template <int NT, typename T>
+__device__ __forceinline__ void pair_dmax(T ma, T mb, double (&scr)[2][NT / O3D_WAVE],
+                                          const SorPairArgs<T> &a, int tid) {
+  const double va = wave_max((double)ma), vb = wave_max((double)mb);
+  if (tid % O3D_WAVE == 0) {
+    scr[0][tid / O3D_WAVE] = va;
+    scr[1][tid / O3D_WAVE] = vb;
+  }
+  __syncthreads();
+  if (tid < 2) {
+    double v = scr[tid][0];
+#pragma unroll
+    for (int q = 1; q < NT / O3D_WAVE; ++q) v = fmax(v, scr[tid][q]);
+    if (v != 0.0)
+      atomicMax(&a.dslot[((size_t)(a.launch % kPairSets) * 2 * kPairSlots +
+                          (size_t)tid * kPairSlots + blockIdx.x % kPairSlots) * kPairStride],
+                (unsigned long long)__double_as_longlong(v));
+  }
+}
+
 template <int... K, typename F>
 __device__ __forceinline__ bool pair_group(std::integer_sequence<int, K...>, int m, int last,
                                            F &&f) {
@@ -407,27 +455,7 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
   s.done = __builtin_amdgcn_readfirstlane((int)s.done) != 0;
   s.n = __builtin_amdgcn_readfirstlane(s.n);
   s.src = __builtin_amdgcn_readfirstlane(s.src);
-  if (blockIdx.x == 0) {
-    if (s.done) {
-      if (tid == 0) {
-        st->done = 1;
-        st->reason = s.reason;
-        st->exit_iter = s.reason == 2 ? a.kmax + 1 : s.sweeps;
-        st->sweeps = s.sweeps;
-        st->result = s.result;
-        st->dmax_final = s.dlast;
-        st->omega_final = s.omega;
-      }
-    } else {
-      if (tid == 0) {
-        st->sched[(a.launch + 1) & 1] = {s.it0, s.n, s.src, 0, s.d_prev, s.om_a, s.om_b};
-        st->sweeps = s.it0 + s.n - 1;
-      }
-      unsigned long long *nx_ds =
-          a.dslot + (size_t)((a.launch + 1) % kPairSets) * 2 * kPairSlots * kPairStride;
-      for (int q = tid; q < 2 * kPairSlots; q += NT) nx_ds[(size_t)q * kPairStride] = 0ull;
-    }
-  }
+  if (blockIdx.x == 0) pair_record(s, a, tid, NT);
   if (s.done) return;
   if (s.src != src) {
     src = s.src;
@@ -500,24 +528,179 @@ __global__ void __launch_bounds__((PairShape<T, SHAPE>::NT))
       ma = dA[r] > ma ? dA[r] : ma;
       mb = dB[r] > mb ? dB[r] : mb;
     }
-  const double va = wave_max((double)ma), vb = wave_max((double)mb);
-  if (tid % O3D_WAVE == 0) {
-    scr[0][tid / O3D_WAVE] = va;
-    scr[1][tid / O3D_WAVE] = vb;
-  }
-  __syncthreads();
-  if (tid < 2) {
-    double v = scr[tid][0];
-#pragma unroll
-    for (int q = 1; q < NT / O3D_WAVE; ++q) v = fmax(v, scr[tid][q]);
-    if (v != 0.0)
-      atomicMax(&a.dslot[((size_t)(a.launch % kPairSets) * 2 * kPairSlots +
-                          (size_t)tid * kPairSlots + blockIdx.x % kPairSlots) * kPairStride],
-                (unsigned long long)__double_as_longlong(v));
-  }
+  pair_dmax<NT>(ma, mb, scr, a, tid);
 }
 
 // ------------------------------------------------------------- small grids
+// The same two iterations of a tile at rest: a block holds its tile and the
+// halo of 4 in registers, a thread a column of ZG planes of pairs, and every
+// half sweep updates all of it.  Where the march's first and last steps outweigh
+// its planes (a launch is never below 11 plane steps) this is the shorter one: a
+// launch is one round of loads and four half sweeps, however few planes there are.
+// Values, stop rule and records are sor_pair_kernel's.
+//   Neighbours: z from the thread's own registers, across threads and in y from
+// the colour's copy in LDS (one barrier per half sweep), x by DPP.  A wave holds
+// four rows of one parity, so that the side of a pair its node lies on is the same
+// in the whole wave; their LDS rows lie side by side (no bank conflicts).
+//   Half sweep h updates the tile and 3 - h nodes around it; planes outside are
+// left out, rows and lanes outside evolve unread.
+//   What bounds it: one round of loads, the stop decision and the block maximum, then
+// the vector units, 16 waves on a CU for 5 times the tile's own nodes.
+// Per launch, march / this: FP64 32^3 11.2 / 9.0 us, 64^3 12.4 / 10.1; FP32 32^3 12.6 / 8.0, 64^3 11.4 / 8.6.  A second round of blocks doubles it
+// (80^3 FP64 14.4 / 19): the line is one block per CU (tile_tiling).
+template <int ZG>
+struct TileShape {
+  static constexpr int LX = 16, LY = 16, LZ = 4 * ZG, NT = 4 * LX * LY;
+  static constexpr int OX = LX - 4, OY = LY - 8, OZ = LZ - 8;  // pairs, rows, planes
+};
+
+template <typename T, int ZG>
+__global__ void __launch_bounds__((TileShape<ZG>::NT)) sor_tile_kernel(const SorPairArgs<T> a) {
+  using S = TileShape<ZG>;
+  constexpr int LX = S::LX, LY = S::LY, LZ = S::LZ, NT = S::NT;
+  constexpr int PL = LX * LY;  // pairs of a plane
+  static_assert(ZG >= 4 && ZG % 2 == 0, "the halo of 4 planes ends inside the outer groups");
+  __shared__ T ex[2][LZ][PL];
+  __shared__ double scr[2][NT / O3D_WAVE];
+  const int tid = threadIdx.x;
+  const int lane = tid % LX;
+  // Rows of wave w of a group: parity w & 1, four of them from 8 (w >> 1) on.
+  const int zg = __builtin_amdgcn_readfirstlane(tid / PL);
+  const int w = __builtin_amdgcn_readfirstlane(tid / O3D_WAVE) & 3, par = w & 1;
+  const int row = 8 * (w >> 1) + 2 * ((tid / LX) & 3) + par;
+  SorState *st = a.st;
+  const int over = st->done;
+  const SorSched P = st->sched[a.launch & 1];
+  const unsigned long long *ds =
+      a.dslot + (size_t)((a.launch + kPairSets - 1) % kPairSets) * 2 * kPairSlots * kPairStride;
+  const size_t wl = (size_t)__lane_id() * kPairStride;
+  const unsigned long long dwa = ds[wl], dwb = ds[(size_t)kPairSlots * kPairStride + wl];
+
+  const int nx = a.nx, ny = a.ny, nz = a.nz, hx = nx / 2;
+  const int tile = pair_tile(blockIdx.x, gridDim.x);
+  const int tix = tile % a.ntx, rr = tile / a.ntx;
+  const int c0 = tix * S::OX, y0 = rr % a.nty * S::OY, z0 = rr / a.nty * S::OZ;
+  const T ox = T(a.ox), oy = T(a.oy), oz = T(a.oz), A = T(a.A), invA = T(a.invA);
+
+  const int c = c0 - 2 + lane, y = y0 - 4 + row;
+  const int rowo = hx * pair_ghost(y, ny, a.per[1]);
+  const int eL = pair_ghost(2 * c, nx, a.per[0]) >> 1, eR = pair_ghost(2 * c + 1, nx, a.per[0]) >> 1;
+  const unsigned vL = (unsigned)(rowo + eL) * (unsigned)sizeof(T);
+  const unsigned vR = (unsigned)(rowo + eR) * (unsigned)sizeof(T);
+  const bool own = lane >= 2 && lane < LX - 2 && c < hx && row >= 4 && row < LY - 4 && y < ny;
+  const int n = nx * ny * nz;
+  const unsigned planeB = (unsigned)(hx * ny) * (unsigned)sizeof(T);
+  const unsigned halfB = planeB * (unsigned)nz;
+  int src = a.launch & 1;
+  __amdgpu_buffer_rsrc_t rin = pair_rsrc(a.buf[src], n);
+  const __amdgpu_buffer_rsrc_t rrh = pair_rsrc(a.rhs, n);
+  // Planes zb + k, k < ZG.  The parity of row + plane of plane k is par + k: z0
+  // and y0 are even.
+  const int zb = z0 - 4 + zg * ZG;
+  T R[ZG], B[ZG], fR[ZG], fB[ZG];
+  const unsigned v0 = par ? vR : vL, v1 = par ? vL : vR;  // red, black node, even k
+  auto load_p = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < ZG; ++k) {
+      const unsigned so = planeB * (unsigned)pair_ghost(zb + k, nz, a.per[2]);
+      R[k] = pload<T>(rin, k & 1 ? v1 : v0, so);
+      B[k] = pload<T>(rin, k & 1 ? v0 : v1, so + halfB);
+    }
+  };
+  load_p();
+#pragma unroll
+  for (int k = 0; k < ZG; ++k) {
+    const unsigned so = planeB * (unsigned)pair_ghost(zb + k, nz, a.per[2]);
+    fR[k] = pload<T>(rrh, k & 1 ? v1 : v0, so);
+    fB[k] = pload<T>(rrh, k & 1 ? v0 : v1, so + halfB);
+  }
+  if (over) return;
+  PairStep s = pair_decide(P, wave_max(__longlong_as_double((long long)dwa)),
+                           wave_max(__longlong_as_double((long long)dwb)), a);
+  s.done = __builtin_amdgcn_readfirstlane((int)s.done) != 0;
+  s.n = __builtin_amdgcn_readfirstlane(s.n);
+  s.src = __builtin_amdgcn_readfirstlane(s.src);
+  if (blockIdx.x == 0) pair_record(s, a, tid, NT);
+  if (s.done) return;
+  if (s.src != src) {
+    src = s.src;
+    rin = pair_rsrc(a.buf[src], n);
+    load_p();
+  }
+  const __amdgpu_buffer_rsrc_t rout = pair_rsrc(a.buf[1 - src], n);
+  const double oma = s.it0 <= a.gs ? 1.0 : s.om_a, omb = s.it0 + 1 <= a.gs ? 1.0 : s.om_b;
+
+  // LDS place of a row: the rows of one parity are contiguous.
+  auto place = [&](int r) { return ((r & 1) * (LY / 2) + (r >> 1)) * LX + lane; };
+  const int me = place(row), lo = place(max(row - 1, 0)), hi = place(min(row + 1, LY - 1));
+  T dA = T(0), dB = T(0);
+  // Half sweep H of this group (GRP 0: the lowest, 2: the highest, 1: between), of
+  // rows of parity PAR: X (this colour) from Y (the other).
+  auto half = [&](auto H, auto GRP, auto PAR, T(&X)[ZG], const T(&Y)[ZG], const T(&F)[ZG], T om,
+                  T om1, T &dm) __attribute__((always_inline)) {
+    constexpr int h = decltype(H)::value, grp = decltype(GRP)::value;
+    constexpr int klo = grp == 0 ? 1 + h : 0, khi = grp == 2 ? ZG - 2 - h : ZG - 1;
+    constexpr int olo = grp == 0 ? 4 : 0, ohi = grp == 2 ? ZG - 5 : ZG - 1;
+    const T(*e)[PL] = ex[1 - (h & 1)];
+    T ym[ZG], yp[ZG], zl = T(0), zh = T(0);
+#pragma unroll
+    for (int k = klo; k <= khi; ++k) {
+      ym[k] = e[zg * ZG + k][lo];
+      yp[k] = e[zg * ZG + k][hi];
+    }
+    if constexpr (klo == 0) zl = e[zg * ZG - 1][me];
+    if constexpr (khi == ZG - 1) zh = e[zg * ZG + ZG][me];
+#pragma unroll
+    for (int k = klo; k <= khi; ++k) {
+      const bool right = ((decltype(PAR)::value + k + h) & 1) != 0;
+      const T side = right ? lane_next<1>(Y[k]) : lane_next<0>(Y[k]);
+      const T zm = k == 0 ? zl : Y[k == 0 ? 0 : k - 1];
+      const T zp = k == ZG - 1 ? zh : Y[k == ZG - 1 ? k : k + 1];
+      const T num = -ox * (side + Y[k]) - oy * (ym[k] + yp[k]) - oz * (zm + zp) + F[k];
+      const T pn = pair_div(num, A, invA);
+      if (k >= olo && k <= ohi) dm = max_abs(dm, zb + k < nz ? pn - X[k] : T(0));
+      X[k] = om1 * X[k] + om * pn;
+      if constexpr (h < 3) ex[h & 1][zg * ZG + k][me] = X[k];
+    }
+  };
+  auto sweep = [&](auto H, T om, T om1, T &dm) __attribute__((always_inline)) {
+    auto go = [&](auto GRP) __attribute__((always_inline)) {
+      constexpr int h = decltype(H)::value;
+      if constexpr (h & 1) {
+        if (par) half(H, GRP, PIC<1>{}, B, R, fB, om, om1, dm);
+        else half(H, GRP, PIC<0>{}, B, R, fB, om, om1, dm);
+      } else {
+        if (par) half(H, GRP, PIC<1>{}, R, B, fR, om, om1, dm);
+        else half(H, GRP, PIC<0>{}, R, B, fR, om, om1, dm);
+      }
+    };
+    if (zg == 0) go(PIC<0>{});
+    else if (zg == 3) go(PIC<2>{});
+    else go(PIC<1>{});
+    if constexpr (decltype(H)::value < 3) __syncthreads();
+  };
+#pragma unroll
+  for (int k = 0; k < ZG; ++k) ex[1][zg * ZG + k][me] = B[k];
+  __syncthreads();
+  sweep(PIC<0>{}, T(oma), T(1.0 - oma), dA);
+  sweep(PIC<1>{}, T(oma), T(1.0 - oma), dA);
+  if (s.n == 2) {
+    sweep(PIC<2>{}, T(omb), T(1.0 - omb), dB);
+    sweep(PIC<3>{}, T(omb), T(1.0 - omb), dB);
+  }
+  if (own) {
+#pragma unroll
+    for (int k = 0; k < ZG; ++k) {
+      const int q = zg * ZG + k;
+      if (q < 4 || q >= LZ - 4 || zb + k >= nz) continue;
+      const unsigned so = planeB * (unsigned)(zb + k);
+      pstore(R[k], rout, vL, so);
+      pstore(B[k], rout, vL, so + halfB);
+    }
+  }
+  pair_dmax<NT>(own ? dA : T(0), own ? dB : T(0), scr, a, tid);
+}
+
 // Whole iterations of a grid that fits one block's LDS, as many as the solve
 // takes (at most kBlockIters per launch, the state carried on in `sched`).  A
 // launch of the march costs 11 us however small its grid; here an iteration is two
@@ -696,6 +879,23 @@ double pair_tiling(SorPairArgs<T> &a) {
   return best;
 }
 
+// Tiles of sor_tile_kernel where they are one round of blocks (its comment has the
+// figures of both sides).
+constexpr int kTileShape = 16;
+template <typename T, int ZG>
+bool tile_tiling(SorPairArgs<T> &a) {
+  using S = TileShape<ZG>;
+  const int ntx = (a.nx / 2 + S::OX - 1) / S::OX, nty = (a.ny + S::OY - 1) / S::OY,
+            ntz = (a.nz + S::OZ - 1) / S::OZ;
+  if ((long long)ntx * nty * ntz > 256) return false;
+  a.shape = kTileShape + ZG;
+  a.ntx = ntx;
+  a.nty = nty;
+  a.ntz = ntz;
+  a.zc = S::OZ;
+  return true;
+}
+
 template <typename T, int SHAPE>
 void pair_launch(const SorPairArgs<T> &a, hipStream_t s) {
   using Shape = PairShape<T, SHAPE>;
@@ -723,6 +923,7 @@ bool pair_cached(const SorPairArgs<T> &a) {
 // 114, 320^3 188 / 198, 512x384x256 306 / 378.
 template <>
 void sor_pair_tiling<double>(SorPairArgs<double> &a) {
+  if (tile_tiling<double, 4>(a)) return;
   const double six = 0.86 * pair_tiling<double, 0>(a);
   if (!pair_cached(a)) return;
   SorPairArgs<double> b = a;
@@ -734,6 +935,7 @@ void sor_pair_tiling<double>(SorPairArgs<double> &a) {
 // 39.8 / 49.5, then 288^3 96.9 / 87.1, 320^3 114 / 107, 512x384x256 219 / 174.
 template <>
 void sor_pair_tiling<float>(SorPairArgs<float> &a) {
+  if (tile_tiling<float, 4>(a)) return;
   if (pair_cached(a)) pair_tiling<float, 0>(a);
   else pair_tiling<float, 1>(a);
 }
@@ -779,6 +981,8 @@ hipError_t launch_sor_pair(const SorPairArgs<T> &a, hipStream_t s) {
     if constexpr (sizeof(T) == 4) {
       if (per == 8) sor_block_kernel<T, 8><<<1, kBlockNT, 0, s>>>(a);
     }
+  } else if (a.shape == kTileShape + 4) {
+    sor_tile_kernel<T, 4><<<a.ntx * a.nty * a.ntz, TileShape<4>::NT, 0, s>>>(a);
   } else if (a.shape == 1) pair_launch<T, 1>(a, s);
   else pair_launch<T, 0>(a, s);
   return hipGetLastError();

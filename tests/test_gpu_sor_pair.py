@@ -11,12 +11,16 @@ from tests.helpers import rand_fields
 pytestmark = pytest.mark.gpu
 
 
-# FP64 tiles own 56 x 16 nodes and chunks of an even number of planes.
+# FP64 tiles own 56 x 16 nodes and chunks of an even number of planes; resting tiles
+# 24 x 8 x 8.
 @pytest.mark.parametrize("solver,shape", [("0000", (6, 6, 6)), ("0000", (8, 16, 56)),
                                           ("0000", (10, 18, 58)), ("0011", (8, 33, 114)),
                                           ("111111", (9, 17, 56)), ("0011", (42, 15, 10)),
                                           ("111111", (11, 7, 70)),
-                                          # Larger grids: the tile of 24 rows.
+                                          # One round of resting tiles, more: the
+                                          # march with 16 rows, with 24 rows.
+                                          ("0011", (40, 130, 58)), ("0000", (66, 66, 130)),
+                                          ("111111", (51, 67, 100)),
                                           ("0011", (130, 145, 116)), ("111111", (129, 128, 128))])
 @pytest.mark.parametrize("idyn", [0, 1])
 def test_pair_f64_equals_oracle(orc, solver, shape, idyn):
@@ -32,9 +36,11 @@ def test_pair_f64_equals_oracle(orc, solver, shape, idyn):
         assert np.array_equal(pg, po), (eps, kmax)
 
 
-# The narrow FP32 tile owns 56 x 40 nodes; the last shape is beyond the size
-# where the wide one (120 x 24) takes over.
-@pytest.mark.parametrize("solver,shape", [("0000", (10, 40, 56)), ("0011", (10, 81, 64)),
+# Resting tiles of 24 x 8 x 8 nodes, then the march: its narrow FP32 tile owns 56 x
+# 40 nodes; the last shape is beyond the size where the wide one (120 x 24) takes over.
+@pytest.mark.parametrize("solver,shape", [("0000", (20, 90, 264)), ("0011", (16, 121, 280)),
+                                          ("0000", (24, 40, 72)), ("111111", (25, 39, 128)),
+                                          ("0000", (10, 40, 56)), ("0011", (10, 81, 64)),
                                           ("111111", (13, 41, 120)),
                                           ("0011", (258, 289, 304))])
 def test_pair_f32_equals_single(solver, shape):
