@@ -661,6 +661,109 @@ __global__ void __launch_bounds__(kMgSmallThreads) mg_small_vcycle_kernel(
   for (int q = threadIdx.x; q < n0; q += kMgSmallThreads) u_out[q] = su[q];
 }
 
+// Two sweeps of a last level too large for one block, per launch.  The rows of a
+// tile of 8 x 8 (y, z) and a halo of 4 lie in LDS, whole in x (at most kBtX cells), and
+// four half sweeps shrink the halo.  A halo row is the stored row it is an image of and
+// keeps that row's colours, and a colour is read before it is written where two of its
+// cells meet (an odd axis that wraps), so every tile computes the same values; they
+// are those of lds_relax_any.  A thread takes a pair of cells (2t, 2t + 1), one of
+// each colour.  A launch per colour, 120 of them for 60 sweeps, is bound by the launches
+// at the sizes met here.  A V(1, 1) cycle over a last level, launches per colour / this:
+// 21^3 433 / 281 us, 25^3 407 / 298, 31^3 407 / 329.
+constexpr int kBtX = 40, kBtT = 8, kBtL = kBtT + 8, kBtNT = 1024;
+constexpr int kBtPer = kBtL * kBtL * (kBtX / 2) / kBtNT;
+template <bool ZERO>
+__global__ void __launch_bounds__(kBtNT) mg_bottom_kernel(float *__restrict__ uo,
+                                                          const float *__restrict__ u,
+                                                          const float *__restrict__ f, MgGrid g,
+                                                          int nty) {
+  constexpr int L = kBtL;
+  __shared__ float su[L * L * kBtX];
+  __shared__ int img[2][L];  // stored row of a local y, z; -1 outside
+  const int y0 = (int)(blockIdx.x % nty) * kBtT, z0 = (int)(blockIdx.x / nty) * kBtT;
+  const int tid = threadIdx.x;
+  if (tid < 2 * L) {
+    const int a = tid / L, l = tid % L;
+    const int q = (a ? z0 : y0) + l - 4, m = a ? g.mz : g.my;
+    img[a][l] = (a ? g.pz : g.py) ? ((q % m) + m) % m : (q < 0 || q >= m ? -1 : q);
+  }
+  __syncthreads();
+  const int hp = (g.mx + 1) >> 1, slots = hp * L * L;
+  const bool meet = mg_colours_meet(g);
+  // Per slot: LDS place of its left cell, row offsets of the y and z neighbours (0: the
+  // mirror), the x neighbours' offsets of both cells, the rows' distance to the edge.
+  int at[kBtPer], ym[kBtPer], yp[kBtPer], zm[kBtPer], zp[kBtPer], xl[kBtPer], xr[kBtPer],
+      par[kBtPer], rim[kBtPer];
+  float f0[kBtPer], f1[kBtPer];
+#pragma unroll
+  for (int s = 0; s < kBtPer; ++s) {
+    const int q = tid + s * kBtNT;
+    rim[s] = -1;
+    at[s] = ym[s] = yp[s] = zm[s] = zp[s] = xl[s] = xr[s] = par[s] = 0;
+    f0[s] = f1[s] = 0.f;
+    if (q >= slots) continue;
+    const int row = q / hp, t = q - row * hp, ly = row % L, lz = row / L;
+    const int y = img[0][ly], z = img[1][lz];
+    if (y < 0 || z < 0) continue;
+    const int x = 2 * t;
+    at[s] = row * kBtX + x;
+    const size_t o = x + (size_t)g.mx * (y + (size_t)g.my * z);
+    const bool two = x + 1 < g.mx;
+    su[at[s]] = ZERO ? 0.f : u[o];
+    f0[s] = f[o];
+    if (two) {
+      su[at[s] + 1] = ZERO ? 0.f : u[o + 1];
+      f1[s] = f[o + 1];
+    }
+    ym[s] = !g.py && y == 0 ? 0 : -kBtX;
+    yp[s] = !g.py && y == g.my - 1 ? 0 : kBtX;
+    zm[s] = !g.pz && z == 0 ? 0 : -L * kBtX;
+    zp[s] = !g.pz && z == g.mz - 1 ? 0 : L * kBtX;
+    // Before the left cell, after the last one of the pair.
+    xl[s] = x > 0 ? -1 : (g.px ? g.mx - 1 : 0);
+    const int last = two ? x + 1 : x;
+    xr[s] = last < g.mx - 1 ? last + 1 - x : (g.px ? -x : last - x);
+    par[s] = ((y + z) & 1) | (two ? 2 : 0);
+    rim[s] = min(min(ly, L - 1 - ly), min(lz, L - 1 - lz));
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int h = 0; h < 4; ++h) {
+    float v[kBtPer];
+#pragma unroll
+    for (int s = 0; s < kBtPer; ++s) {
+      const int right = (par[s] + h) & 1;
+      if (rim[s] > h && (!right || (par[s] & 2))) {
+        const float *c = su + at[s] + right;
+        const bool two = par[s] & 2;
+        const float a = right ? c[-1] : c[xl[s]];
+        const float b = right ? c[xr[s] - 1] : (two ? c[1] : c[xr[s]]);
+        v[s] = mg_relax_value(right ? f1[s] : f0[s], a + b, c[ym[s]] + c[yp[s]],
+                              c[zm[s]] + c[zp[s]], g);
+        if (!meet) su[at[s] + right] = v[s];
+      }
+    }
+    __syncthreads();
+    if (!meet) continue;
+#pragma unroll
+    for (int s = 0; s < kBtPer; ++s) {
+      const int right = (par[s] + h) & 1;
+      if (rim[s] > h && (!right || (par[s] & 2))) su[at[s] + right] = v[s];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int s = 0; s < kBtPer; ++s) {
+    if (rim[s] < 4) continue;
+    const int row = at[s] / kBtX, x = at[s] - row * kBtX;
+    const int y = y0 + row % L - 4, z = z0 + row / L - 4;
+    if (y >= g.my || z >= g.mz) continue;
+    float *o = uo + x + (size_t)g.mx * (y + (size_t)g.my * z);
+    o[0] = su[at[s]];
+    if (par[s] & 2) o[1] = su[at[s] + 1];
+  }
+}
+
 MgGrid grid_of(const MgHierarchy &H, int l) {
   MgGrid g;
   g.mx = H.m[l][0]; g.my = H.m[l][1]; g.mz = H.m[l][2];
@@ -728,6 +831,20 @@ hipError_t clear_level(const MgHierarchy &H, int l, hipStream_t s) {
   return hipGetLastError();
 }
 
+// An even number of sweeps of the last level, two per launch.
+hipError_t bottom(MgHierarchy &H, int l, int sweeps, bool zero, hipStream_t s) {
+  const MgGrid g = grid_of(H, l);
+  const int nty = (g.my + kBtT - 1) / kBtT, blocks = nty * ((g.mz + kBtT - 1) / kBtT);
+  for (int q = 0; q < sweeps; q += 2) {
+    if (zero && q == 0)
+      mg_bottom_kernel<true><<<blocks, kBtNT, 0, s>>>(H.r[l], H.u[l], H.f[l], g, nty);
+    else
+      mg_bottom_kernel<false><<<blocks, kBtNT, 0, s>>>(H.r[l], H.u[l], H.f[l], g, nty);
+    std::swap(H.u[l], H.r[l]);
+  }
+  return hipGetLastError();
+}
+
 // A V(nu1, nu2) cycle from level l down; zero: u starts from 0 (its array need
 // not be cleared).
 hipError_t vcycle(MgHierarchy &H, int l, int nu1, int nu2, bool zero, hipStream_t s) {
@@ -756,6 +873,7 @@ hipError_t vcycle(MgHierarchy &H, int l, int nu1, int nu2, bool zero, hipStream_
       mg_coarsest_kernel<<<1, threads, 0, s>>>(H.u[l], H.f[l], g, n <= 64 ? 30 : 60);
       return hipGetLastError();
     }
+    if (g.mx <= kBtX) return bottom(H, l, 60, zero, s);
     if (zero && (e = clear_level(H, l, s)) != hipSuccess) return e;
     return smooth(H, l, 60, s);
   }

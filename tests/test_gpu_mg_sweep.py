@@ -98,7 +98,10 @@ def _vcycle(u, f, h, per, top=True, inside=False):
 # (nz, ny, nx): one tile, partial tiles on every axis, several tiles of 4 and
 # of 8 planes (512 tiles of 8 planes and more), two levels only.
 @pytest.mark.parametrize("shape", [(4, 8, 32), (12, 20, 68), (40, 24, 48), (128, 64, 256),
-                                   (6, 6, 34)])
+                                   (6, 6, 34),
+                                   # Last levels of 17 x 18 x 25, 25 x 21 x 33 and
+                                   # 5 x 33 x 40 cells (more than a block holds).
+                                   (34, 36, 50), (50, 42, 66), (10, 66, 80)])
 @pytest.mark.parametrize("per", [(1, 1, 1), (1, 0, 1), (0, 0, 0)])
 def test_vcycles_equal_restatement(shape, per):
     f, = rand_fields(shape, 1, seed=71)
