@@ -426,42 +426,9 @@ __global__ void __launch_bounds__(256) mg_prolong_kernel(float *__restrict__ u,
   }
 }
 
-// An odd axis that wraps puts two cells of one colour beside each other, so a
-// colour relaxed in place would depend on which wave of the block comes first.
-// There all cells of a colour are read before any is written (with one barrier
-// more); elsewhere the cells of a colour do not meet.
+// Two cells of one colour are neighbours (an odd axis that wraps).
 __device__ __forceinline__ bool mg_colours_meet(const MgGrid &g) {
   return ((g.mx & g.px) | (g.my & g.py) | (g.mz & g.pz)) & 1;
-}
-
-// One colour of a level of at most kMgCoarsestCells cells in LDS, a cell per
-// thread at a time, by a block of at least 64 threads (1024 above 64 cells).
-__device__ __forceinline__ void lds_relax_any(float *u, const float *f, const MgGrid &g,
-                                              int colour, bool meet) {
-  const int n = g.mx * g.my * g.mz;
-  constexpr int kPer = kMgCoarsestCells / 1024;
-  float v[kPer];
-#pragma unroll
-  for (int s = 0; s < kPer; ++s) {
-    const int q = threadIdx.x + s * blockDim.x;
-    if (q < n) {
-      const int row = q / g.mx, i = q - row * g.mx;
-      const int k = row / g.my, j = row - k * g.my;
-      v[s] = u[q];
-      if (((i + j + k) & 1) == colour) {
-        v[s] = (f[q] - mg_lap_off(u, g, i, j, k)) * g.invd;
-        if (!meet) u[q] = v[s];
-      }
-    }
-  }
-  __syncthreads();
-  if (!meet) return;
-#pragma unroll
-  for (int s = 0; s < kPer; ++s) {
-    const int q = threadIdx.x + s * blockDim.x;
-    if (q < n) u[q] = v[s];
-  }
-  __syncthreads();
 }
 
 // The coarsest level: `sweeps` red-black Gauss-Seidel sweeps from u = 0 by
@@ -476,9 +443,15 @@ __global__ void __launch_bounds__(1024) mg_coarsest_kernel(float *__restrict__ u
     sf[q] = f[q];
   }
   __syncthreads();
-  const bool meet = mg_colours_meet(g);
   for (int s = 0; s < sweeps; ++s)
-    for (int colour = 0; colour < 2; ++colour) lds_relax_any(su, sf, g, colour, meet);
+    for (int colour = 0; colour < 2; ++colour) {
+      for (int q = threadIdx.x; q < n; q += blockDim.x) {
+        const int row = q / g.mx, i = q - row * g.mx;
+        const int k = row / g.my, j = row - k * g.my;
+        if (((i + j + k) & 1) == colour) mg_relax(su, sf, g, i, j, k, q);
+      }
+      __syncthreads();
+    }
   for (int q = threadIdx.x; q < n; q += blockDim.x) u[q] = su[q];
 }
 
@@ -511,10 +484,17 @@ struct SmallDiv {
 
 __device__ __forceinline__ void lds_smooth(float *u, const float *f, const MgGrid &g,
                                            int sweeps) {
-  const bool meet = mg_colours_meet(g);
   if (g.mx & 1) {
+    const int n = g.mx * g.my * g.mz;
     for (int s = 0; s < sweeps; ++s)
-      for (int colour = 0; colour < 2; ++colour) lds_relax_any(u, f, g, colour, meet);
+      for (int colour = 0; colour < 2; ++colour) {
+        for (int q = threadIdx.x; q < n; q += kMgSmallThreads) {
+          const int row = q / g.mx, i = q - row * g.mx;
+          const int k = row / g.my, j = row - k * g.my;
+          if (((i + j + k) & 1) == colour) mg_relax(u, f, g, i, j, k, q);
+        }
+        __syncthreads();
+      }
     return;
   }
   // Per cell pair of this thread: its offset and, for both of its cells, the
@@ -537,22 +517,14 @@ __device__ __forceinline__ void lds_smooth(float *u, const float *f, const MgGri
   }
   for (int sw = 0; sw < sweeps; ++sw)
     for (int colour = 0; colour < 2; ++colour) {
-      float v[kMgSmallPer];
 #pragma unroll
       for (int s = 0; s < kMgSmallPer; ++s)
         if (threadIdx.x + s * kMgSmallThreads < nh) {
           const int right = (base[s] + colour) & 1, l = base[s] >> 1, q = l + right;
           const float sx = u[right ? l : l + oxl[s]] + u[right ? l + oxr[s] : l + 1];
-          v[s] = mg_relax_value(f[q], sx, u[q + oym[s]] + u[q + oyp[s]],
+          u[q] = mg_relax_value(f[q], sx, u[q + oym[s]] + u[q + oyp[s]],
                                 u[q + ozm[s]] + u[q + ozp[s]], g);
-          if (!meet) u[q] = v[s];
         }
-      __syncthreads();
-      if (!meet) continue;
-#pragma unroll
-      for (int s = 0; s < kMgSmallPer; ++s)
-        if (threadIdx.x + s * kMgSmallThreads < nh)
-          u[(base[s] >> 1) + ((base[s] + colour) & 1)] = v[s];
       __syncthreads();
     }
 }
@@ -665,8 +637,9 @@ __global__ void __launch_bounds__(kMgSmallThreads) mg_small_vcycle_kernel(
 // tile of 8 x 8 (y, z) and a halo of 4 lie in LDS, whole in x (at most kBtX cells), and
 // four half sweeps shrink the halo.  A halo row is the stored row it is an image of and
 // keeps that row's colours, and a colour is read before it is written where two of its
-// cells meet (an odd axis that wraps), so every tile computes the same values; they
-// are those of lds_relax_any.  A thread takes a pair of cells (2t, 2t + 1), one of
+// cells meet (an odd axis that wraps), so every tile computes the same values: those
+// of mg_smooth_kernel where the colours do not meet, one of the orders its launches may
+// take where they do.  A thread takes a pair of cells (2t, 2t + 1), one of
 // each colour.  A launch per colour, 120 of them for 60 sweeps, is bound by the launches
 // at the sizes met here.  A V(1, 1) cycle over a last level, launches per colour / this:
 // 21^3 433 / 281 us, 25^3 407 / 298, 31^3 407 / 329.
