@@ -888,9 +888,19 @@ __global__ void __launch_bounds__(256) mg_sum_kernel(const float *__restrict__ f
                                                      double *__restrict__ part) {
   __shared__ double sc[4];
   double s = 0.0;
-  // Eight loads in flight, added in order.
-#pragma unroll 8
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) s += (double)f[i];
+  // 32 loads in flight, added in order (256x192x128 cells 26 us with 8, now 6.8).
+  const int step = gridDim.x * 256;
+  for (long long i0 = blockIdx.x * 256 + threadIdx.x; i0 < n; i0 += 32ll * step) {
+    float v[32];
+#pragma unroll
+    for (int q = 0; q < 32; ++q) {
+      const long long i = i0 + (long long)q * step;
+      v[q] = f[min(i, (long long)n - 1)];
+    }
+#pragma unroll
+    for (int q = 0; q < 32; ++q)
+      if (i0 + (long long)q * step < n) s += (double)v[q];
+  }
   s = block_sum<4>(s, sc);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
@@ -1011,7 +1021,7 @@ hipError_t mg_solve(MgHierarchy &H, int cycles, int nu1, int nu2, hipStream_t s,
     double *part = reinterpret_cast<double *>(H.r[0]);
     const int nb = std::max(1, std::min(kMgMeanBlocks, n0 / 2));
     mg_sum_kernel<<<nb, 256, 0, s>>>(H.f[0], n0, part);
-    mg_center_kernel<<<nb, 256, 0, s>>>(H.f[0], n0, part, nb);
+    mg_center_kernel<<<std::min(1024, (n0 + 255) / 256), 256, 0, s>>>(H.f[0], n0, part, nb);
   }
   hipError_t e = hipGetLastError();
   if (cycles < 1 && from_zero) e = clear_level(H, 0, s);
