@@ -578,8 +578,10 @@ __global__ void __launch_bounds__(kMgSmallThreads) mg_small_vcycle_kernel(
     su[q] = 0.f;
   }
   __syncthreads();
-  // Down: smooth, then the averaged residual as the next level's f.
-#pragma unroll
+  // Down: smooth, then the averaged residual as the next level's f.  (One copy of
+  // the code for all levels: every launch meets it cold, and with a copy per level
+  // 24x16x8 cells took 21.4 us, now 19.8.)
+#pragma unroll 1
   for (int l = 0; l < kMgSmallLevels - 1; ++l) {
     if (l >= S.levels - 1) break;
     const MgGrid &g = S.g[l], &c = S.g[l + 1];
@@ -597,7 +599,7 @@ __global__ void __launch_bounds__(kMgSmallThreads) mg_small_vcycle_kernel(
     __syncthreads();
   }
   // Coarsest.
-#pragma unroll
+#pragma unroll 1
   for (int l = 1; l < kMgSmallLevels; ++l)
     if (l == S.levels - 1) {
       const MgGrid &g = S.g[l];
@@ -607,7 +609,7 @@ __global__ void __launch_bounds__(kMgSmallThreads) mg_small_vcycle_kernel(
         lds_smooth(su + S.off[l], sf + S.off[l], g, S.coarse_sweeps);
     }
   // Up: prolong, smooth.
-#pragma unroll
+#pragma unroll 1
   for (int l = kMgSmallLevels - 2; l >= 0; --l) {
     if (l >= S.levels - 1) continue;
     const MgGrid &g = S.g[l], &c = S.g[l + 1];
