@@ -443,6 +443,44 @@ __global__ void __launch_bounds__(1024) mg_coarsest_kernel(float *__restrict__ u
     sf[q] = f[q];
   }
   __syncthreads();
+  if (!mg_colours_meet(g)) {
+    // The cells of this thread and their neighbours, worked out once (a V-cycle over 9 x
+    // 15 x 24 cells, y and z mirrored, 383 -> 81 us).  Where colours meet, the order of
+    // the loop below stays.
+    constexpr int kPer = kMgCoarsestCells / 1024;
+    int nb[kPer][6], col[kPer];
+    float fq[kPer];
+#pragma unroll
+    for (int s = 0; s < kPer; ++s) {
+      const int q = threadIdx.x + s * blockDim.x;
+      col[s] = -1;
+      fq[s] = 0.f;
+      if (q >= n) continue;
+      const int row = q / g.mx, i = q - row * g.mx;
+      const int k = row / g.my, j = row - k * g.my;
+      const int pl = g.mx * g.my;
+      nb[s][0] = q - i + mg_nb(i - 1, g.mx, g.px);
+      nb[s][1] = q - i + mg_nb(i + 1, g.mx, g.px);
+      nb[s][2] = q + g.mx * (mg_nb(j - 1, g.my, g.py) - j);
+      nb[s][3] = q + g.mx * (mg_nb(j + 1, g.my, g.py) - j);
+      nb[s][4] = q + pl * (mg_nb(k - 1, g.mz, g.pz) - k);
+      nb[s][5] = q + pl * (mg_nb(k + 1, g.mz, g.pz) - k);
+      col[s] = (i + j + k) & 1;
+      fq[s] = sf[q];
+    }
+    for (int sw = 0; sw < sweeps; ++sw)
+      for (int colour = 0; colour < 2; ++colour) {
+#pragma unroll
+        for (int s = 0; s < kPer; ++s)
+          if (col[s] == colour)
+            su[threadIdx.x + s * blockDim.x] =
+                mg_relax_value(fq[s], su[nb[s][0]] + su[nb[s][1]], su[nb[s][2]] + su[nb[s][3]],
+                               su[nb[s][4]] + su[nb[s][5]], g);
+        __syncthreads();
+      }
+    for (int q = threadIdx.x; q < n; q += blockDim.x) u[q] = su[q];
+    return;
+  }
   for (int s = 0; s < sweeps; ++s)
     for (int colour = 0; colour < 2; ++colour) {
       for (int q = threadIdx.x; q < n; q += blockDim.x) {

@@ -125,6 +125,22 @@ def test_vcycles_equal_restatement(shape, per):
         assert np.abs(u - ref).max() <= 1e-5 * np.abs(ref).max()
 
 
+# Levels of one block whose cells of a colour do not meet: axes that wrap are even.
+@pytest.mark.parametrize("shape,per", [((36, 30, 48), (1, 0, 0)), ((20, 60, 98), (0, 1, 0)),
+                                       ((16, 24, 90), (0, 1, 1))])
+def test_one_block_last_level(shape, per):
+    f, = rand_fields(shape, 1, seed=73)
+    f = f.astype(F)
+    u = np.zeros(shape, F)
+    capi.multigrid(u, f, (0.1, 0.12, 0.11), per, 2)
+    f = f - F(f.astype(np.float64).sum() / f.size)
+    ref = np.zeros(shape, F)
+    for _ in range(2):
+        ref = _vcycle(ref, f, (0.1, 0.12, 0.11), per)
+    # As above: the mean's last bit.
+    assert np.abs(u - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("solver,shape", [("0000", (16, 16, 64)), ("0011", (24, 40, 72)),
                                           ("111111", (16, 12, 16))])
 def test_v11_solves(orc, solver, shape):
