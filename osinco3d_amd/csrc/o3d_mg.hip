@@ -378,7 +378,49 @@ __global__ void __launch_bounds__(256) mg_smooth_kernel(float *__restrict__ u,
   mg_relax(u, f, g, i, j, k, i + g.mx * row);
 }
 
-// The same for mx odd: one thread per cell, the other colour idle.
+// Two cells of one colour are neighbours (an odd axis that wraps): cells 0 and m - 1
+// of such an axis.  Relaxed in place, which of them reads the other's new value would
+// depend on waves and blocks that nothing orders, and with it the free constant of the
+// solution (by some 1e-3 of it) from run to run.  So every kernel of a level whose
+// colours meet reads all cells of a colour before it writes any of them: the values do
+// not depend on the kernel, its tiles or the block's size.  (One wave does so by
+// itself, and so did in practice the launches per colour and small blocks, whose loads
+// are all on their way before the first store.)  A V(2, 2) cycle where they meet / where
+// no axis wraps: a last level of 20 x 15 x 9 cells in one block 82 / 73 us (one barrier
+// more per colour), 36 x 9 x 13 in rows 322 / 268 us, 104 x 87 x 33 by launches per
+// colour 442 / 424 us.
+__device__ __host__ __forceinline__ bool mg_colours_meet(const MgGrid &g) {
+  return ((g.mx & g.px) | (g.my & g.py) | (g.mz & g.pz)) & 1;
+}
+
+// One colour of a sweep where the colours meet: the new values go to uo.  un holds the
+// other colour's latest values (uo itself for the second colour of a sweep), u the
+// values before the sweep; a neighbour of the cell's own colour (across the wrap, or
+// the cell itself at a mirrored edge) is read from u.
+__global__ void __launch_bounds__(256) mg_smooth_meet_kernel(float *uo, const float *un,
+                                                             const float *u,
+                                                             const float *__restrict__ f,
+                                                             MgGrid g, int colour) {
+  const int hx = (g.mx + 1) >> 1;
+  const int p = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  if (p >= hx * g.my * g.mz) return;
+  const int row = p / hx, t = p - row * hx;
+  const int k = row / g.my, j = row - k * g.my;
+  const int i = 2 * t + ((j + k + colour) & 1);
+  if (i >= g.mx) return;
+  const int pl = g.mx * g.my, q = i + g.mx * row;
+  const int xm = mg_nb(i - 1, g.mx, g.px), xp = mg_nb(i + 1, g.mx, g.px);
+  const int ym = mg_nb(j - 1, g.my, g.py), yp = mg_nb(j + 1, g.my, g.py);
+  const int zm = mg_nb(k - 1, g.mz, g.pz), zp = mg_nb(k + 1, g.mz, g.pz);
+  // The value d places from the cell, across so many indices of an axis.
+  auto at = [&](int across, int d) { return ((across & 1) ? un : u)[q + d]; };
+  const float sx = at(xm - i, xm - i) + at(xp - i, xp - i);
+  const float sy = at(ym - j, g.mx * (ym - j)) + at(yp - j, g.mx * (yp - j));
+  const float sz = at(zm - k, pl * (zm - k)) + at(zp - k, pl * (zp - k));
+  uo[q] = mg_relax_value(f[q], sx, sy, sz, g);
+}
+
+// The same in place for mx odd: one thread per cell, the other colour idle.
 __global__ void __launch_bounds__(256) mg_smooth_any_kernel(float *__restrict__ u,
                                                             const float *__restrict__ f,
                                                             MgGrid g, int colour) {
@@ -426,11 +468,6 @@ __global__ void __launch_bounds__(256) mg_prolong_kernel(float *__restrict__ u,
   }
 }
 
-// Two cells of one colour are neighbours (an odd axis that wraps).
-__device__ __forceinline__ bool mg_colours_meet(const MgGrid &g) {
-  return ((g.mx & g.px) | (g.my & g.py) | (g.mz & g.pz)) & 1;
-}
-
 // The coarsest level: `sweeps` red-black Gauss-Seidel sweeps from u = 0 by
 // one block, the level staged in LDS.
 __global__ void __launch_bounds__(1024) mg_coarsest_kernel(float *__restrict__ u,
@@ -443,51 +480,44 @@ __global__ void __launch_bounds__(1024) mg_coarsest_kernel(float *__restrict__ u
     sf[q] = f[q];
   }
   __syncthreads();
-  if (!mg_colours_meet(g)) {
-    // The cells of this thread and their neighbours, worked out once (a V-cycle over 9 x
-    // 15 x 24 cells, y and z mirrored, 383 -> 81 us).  Where colours meet, the order of
-    // the loop below stays.
-    constexpr int kPer = kMgCoarsestCells / 1024;
-    int nb[kPer][6], col[kPer];
-    float fq[kPer];
+  // The cells of this thread and their neighbours, worked out once (a V-cycle over 9 x
+  // 15 x 24 cells, y and z mirrored, 383 -> 81 us).
+  const bool meet = mg_colours_meet(g);
+  constexpr int kPer = kMgCoarsestCells / 1024;
+  int nb[kPer][6], col[kPer];
+  float fq[kPer], v[kPer];
 #pragma unroll
-    for (int s = 0; s < kPer; ++s) {
-      const int q = threadIdx.x + s * blockDim.x;
-      col[s] = -1;
-      fq[s] = 0.f;
-      if (q >= n) continue;
-      const int row = q / g.mx, i = q - row * g.mx;
-      const int k = row / g.my, j = row - k * g.my;
-      const int pl = g.mx * g.my;
-      nb[s][0] = q - i + mg_nb(i - 1, g.mx, g.px);
-      nb[s][1] = q - i + mg_nb(i + 1, g.mx, g.px);
-      nb[s][2] = q + g.mx * (mg_nb(j - 1, g.my, g.py) - j);
-      nb[s][3] = q + g.mx * (mg_nb(j + 1, g.my, g.py) - j);
-      nb[s][4] = q + pl * (mg_nb(k - 1, g.mz, g.pz) - k);
-      nb[s][5] = q + pl * (mg_nb(k + 1, g.mz, g.pz) - k);
-      col[s] = (i + j + k) & 1;
-      fq[s] = sf[q];
-    }
-    for (int sw = 0; sw < sweeps; ++sw)
-      for (int colour = 0; colour < 2; ++colour) {
-#pragma unroll
-        for (int s = 0; s < kPer; ++s)
-          if (col[s] == colour)
-            su[threadIdx.x + s * blockDim.x] =
-                mg_relax_value(fq[s], su[nb[s][0]] + su[nb[s][1]], su[nb[s][2]] + su[nb[s][3]],
-                               su[nb[s][4]] + su[nb[s][5]], g);
-        __syncthreads();
-      }
-    for (int q = threadIdx.x; q < n; q += blockDim.x) u[q] = su[q];
-    return;
+  for (int s = 0; s < kPer; ++s) {
+    const int q = threadIdx.x + s * blockDim.x;
+    col[s] = -1;
+    fq[s] = 0.f;
+    if (q >= n) continue;
+    const int row = q / g.mx, i = q - row * g.mx;
+    const int k = row / g.my, j = row - k * g.my;
+    const int pl = g.mx * g.my;
+    nb[s][0] = q - i + mg_nb(i - 1, g.mx, g.px);
+    nb[s][1] = q - i + mg_nb(i + 1, g.mx, g.px);
+    nb[s][2] = q + g.mx * (mg_nb(j - 1, g.my, g.py) - j);
+    nb[s][3] = q + g.mx * (mg_nb(j + 1, g.my, g.py) - j);
+    nb[s][4] = q + pl * (mg_nb(k - 1, g.mz, g.pz) - k);
+    nb[s][5] = q + pl * (mg_nb(k + 1, g.mz, g.pz) - k);
+    col[s] = (i + j + k) & 1;
+    fq[s] = sf[q];
   }
-  for (int s = 0; s < sweeps; ++s)
+  for (int sw = 0; sw < sweeps; ++sw)
     for (int colour = 0; colour < 2; ++colour) {
-      for (int q = threadIdx.x; q < n; q += blockDim.x) {
-        const int row = q / g.mx, i = q - row * g.mx;
-        const int k = row / g.my, j = row - k * g.my;
-        if (((i + j + k) & 1) == colour) mg_relax(su, sf, g, i, j, k, q);
-      }
+#pragma unroll
+      for (int s = 0; s < kPer; ++s)
+        if (col[s] == colour) {
+          v[s] = mg_relax_value(fq[s], su[nb[s][0]] + su[nb[s][1]], su[nb[s][2]] + su[nb[s][3]],
+                                su[nb[s][4]] + su[nb[s][5]], g);
+          if (!meet) su[threadIdx.x + s * blockDim.x] = v[s];
+        }
+      __syncthreads();
+      if (!meet) continue;
+#pragma unroll
+      for (int s = 0; s < kPer; ++s)
+        if (col[s] == colour) su[threadIdx.x + s * blockDim.x] = v[s];
       __syncthreads();
     }
   for (int q = threadIdx.x; q < n; q += blockDim.x) u[q] = su[q];
@@ -522,14 +552,30 @@ struct SmallDiv {
 
 __device__ __forceinline__ void lds_smooth(float *u, const float *f, const MgGrid &g,
                                            int sweeps) {
+  const bool meet = mg_colours_meet(g);
   if (g.mx & 1) {
     const int n = g.mx * g.my * g.mz;
+    constexpr int kPer = kMgCoarsestCells / kMgSmallThreads;
     for (int s = 0; s < sweeps; ++s)
       for (int colour = 0; colour < 2; ++colour) {
-        for (int q = threadIdx.x; q < n; q += kMgSmallThreads) {
+        float v[kPer];
+#pragma unroll
+        for (int c = 0; c < kPer; ++c) {
+          const int q = threadIdx.x + c * kMgSmallThreads;
+          if (q >= n) continue;
           const int row = q / g.mx, i = q - row * g.mx;
           const int k = row / g.my, j = row - k * g.my;
-          if (((i + j + k) & 1) == colour) mg_relax(u, f, g, i, j, k, q);
+          v[c] = u[q];
+          if (((i + j + k) & 1) != colour) continue;
+          v[c] = (f[q] - mg_lap_off(u, g, i, j, k)) * g.invd;
+          if (!meet) u[q] = v[c];
+        }
+        __syncthreads();
+        if (!meet) continue;
+#pragma unroll
+        for (int c = 0; c < kPer; ++c) {
+          const int q = threadIdx.x + c * kMgSmallThreads;
+          if (q < n) u[q] = v[c];
         }
         __syncthreads();
       }
@@ -555,14 +601,22 @@ __device__ __forceinline__ void lds_smooth(float *u, const float *f, const MgGri
   }
   for (int sw = 0; sw < sweeps; ++sw)
     for (int colour = 0; colour < 2; ++colour) {
+      float v[kMgSmallPer];
 #pragma unroll
       for (int s = 0; s < kMgSmallPer; ++s)
         if (threadIdx.x + s * kMgSmallThreads < nh) {
           const int right = (base[s] + colour) & 1, l = base[s] >> 1, q = l + right;
           const float sx = u[right ? l : l + oxl[s]] + u[right ? l + oxr[s] : l + 1];
-          u[q] = mg_relax_value(f[q], sx, u[q + oym[s]] + u[q + oyp[s]],
+          v[s] = mg_relax_value(f[q], sx, u[q + oym[s]] + u[q + oyp[s]],
                                 u[q + ozm[s]] + u[q + ozp[s]], g);
+          if (!meet) u[q] = v[s];
         }
+      __syncthreads();
+      if (!meet) continue;
+#pragma unroll
+      for (int s = 0; s < kMgSmallPer; ++s)
+        if (threadIdx.x + s * kMgSmallThreads < nh)
+          u[(base[s] >> 1) + ((base[s] + colour) & 1)] = v[s];
       __syncthreads();
     }
 }
@@ -677,9 +731,8 @@ __global__ void __launch_bounds__(kMgSmallThreads) mg_small_vcycle_kernel(
 // tile of 8 x 8 (y, z) and a halo of 4 lie in LDS, whole in x (at most kBtX cells), and
 // four half sweeps shrink the halo.  A halo row is the stored row it is an image of and
 // keeps that row's colours, and a colour is read before it is written where two of its
-// cells meet (an odd axis that wraps), so every tile computes the same values: those
-// of mg_smooth_kernel where the colours do not meet, one of the orders its launches may
-// take where they do.  A thread takes a pair of cells (2t, 2t + 1), one of
+// cells meet (mg_colours_meet), so every tile computes the same values: those of the
+// launches per colour.  A thread takes a pair of cells (2t, 2t + 1), one of
 // each colour.  A launch per colour, 120 of them for 60 sweeps, is bound by the launches
 // at the sizes met here.  A V(1, 1) cycle over a last level, launches per colour / this:
 // 21^3 433 / 281 us, 25^3 407 / 298, 31^3 407 / 329.
@@ -789,9 +842,20 @@ MgGrid grid_of(const MgHierarchy &H, int l) {
 
 unsigned blocks_for(long long threads) { return (unsigned)((threads + 255) / 256); }
 
-hipError_t smooth(const MgHierarchy &H, int l, int sweeps, hipStream_t s) {
+hipError_t smooth(MgHierarchy &H, int l, int sweeps, hipStream_t s) {
   const MgGrid g = grid_of(H, l);
   const long long n = (long long)g.mx * g.my * g.mz;
+  if (mg_colours_meet(g)) {
+    // A sweep goes from H.u[l] into H.r[l], which then trade places.
+    const unsigned blocks = blocks_for((long long)((g.mx + 1) / 2) * g.my * g.mz);
+    for (int q = 0; q < sweeps; ++q) {
+      for (int colour = 0; colour < 2; ++colour)
+        mg_smooth_meet_kernel<<<blocks, 256, 0, s>>>(H.r[l], colour ? H.r[l] : H.u[l], H.u[l],
+                                                     H.f[l], g, colour);
+      std::swap(H.u[l], H.r[l]);
+    }
+    return hipGetLastError();
+  }
   for (int q = 0; q < sweeps; ++q)
     for (int colour = 0; colour < 2; ++colour) {
       if (g.mx & 1)
