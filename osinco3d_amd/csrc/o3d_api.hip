@@ -1369,10 +1369,11 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
   CHK(s.scratch(mg_plan(H, m0, h, per), &mgbuf));
   mg_bind(H, mgbuf);
   H.levels = std::min(H.levels, std::max(nlevels - 1, 0));
-  float *R, *E, *E2;
+  const bool pairs = sor_buffer_fits<float, float>(nx, ny, nz);
+  float *R, *E, *E2 = nullptr;
   CHK(s.scratch(n, &R));
   CHK(s.scratch(n, &E));
-  CHK(s.scratch(n, &E2));
+  if (pairs) CHK(s.scratch(n, &E2));
   const int nb = residual_blocks(nx, ny, nz);
   double *part;
   CHK(s.scratch((size_t)4 * nb + 4, &part));
@@ -1436,11 +1437,16 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
         break;
       }
     }
-    int sweeps = 0;
-    if ((rc = run.run(1.0, npre + npost, &sweeps)) != 0) break;
-    if (run.hst->result == 1) {
-      std::swap(E, E2);
-      std::swap(run.pa.buf[0], run.pa.buf[1]);
+    if (pairs) {
+      int sweeps = 0;
+      if ((rc = run.run(1.0, npre + npost, &sweeps)) != 0) break;
+      if (run.hst->result == 1) {
+        std::swap(E, E2);
+        std::swap(run.pa.buf[0], run.pa.buf[1]);
+      }
+    } else if (launch_gs_split<float>(run.pa, E, npre + npost, g_stream) != hipSuccess) {
+      rc = fail("multigrid: smoothing failed");
+      break;
     }
     if (launch_fold_split(p, E, nx, ny, nz, g_stream) != hipSuccess) {
       rc = fail("multigrid: fold failed");

@@ -136,6 +136,10 @@ template <typename T>
 hipError_t launch_sor_pair_init(const SorPairArgs<T> &a, double omega, hipStream_t s);
 template <typename T>
 hipError_t launch_sor_pair(const SorPairArgs<T> &a, hipStream_t s);
+// `sweeps` red-black Gauss-Seidel sweeps of `field` (colour-split) in place, for grids of
+// any size: the pair kernel's grids are those of sor_buffer_fits.
+template <typename T>
+hipError_t launch_gs_split(const SorPairArgs<T> &a, T *field, int sweeps, hipStream_t s);
 
 // Natural <-> colour-split storage (nx even).
 template <typename T>

@@ -818,6 +818,33 @@ __global__ void __launch_bounds__(kBlockNT) sor_block_kernel(const SorPairArgs<T
   }
 }
 
+// One colour of a Gauss-Seidel sweep (omega = 1) in place, the updates of
+// sor_pair_kernel, with 64-bit addresses and no stop rule: the multigrid smoother of
+// grids beyond what buffer descriptors address (2 GiB of FP32).  One thread per node of
+// the colour; memory bounds it.
+template <typename T>
+__global__ void __launch_bounds__(256) gs_split_kernel(T *__restrict__ x,
+                                                       const T *__restrict__ y,
+                                                       const T *__restrict__ rhs, int colour,
+                                                       int nx, int ny, int nz, int px, int py,
+                                                       int pz, T ox, T oy, T oz, T A, T invA) {
+  const int hx = nx / 2;
+  const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= (size_t)hx * ny * nz) return;
+  const int row = (int)(e / hx), c = (int)(e - (size_t)row * hx);
+  const int k = row / ny, j = row - k * ny;
+  const bool right = ((j + k + colour) & 1) != 0;
+  const size_t plane = (size_t)hx * ny, yb = plane * k + c, zb = (size_t)hx * j + c;
+  const int out = pair_ghost(right ? 2 * c + 2 : 2 * c - 1, nx, px) >> 1;
+  const T side = y[(size_t)row * hx + out];
+  const T ym = y[yb + (size_t)hx * pair_ghost(j - 1, ny, py)];
+  const T yp = y[yb + (size_t)hx * pair_ghost(j + 1, ny, py)];
+  const T zm = y[zb + plane * pair_ghost(k - 1, nz, pz)];
+  const T zp = y[zb + plane * pair_ghost(k + 1, nz, pz)];
+  const T num = -ox * (side + y[e]) - oy * (ym + yp) - oz * (zm + zp) + rhs[e];
+  x[e] = T(0) * x[e] + T(1) * pair_div(num, A, invA);
+}
+
 __global__ void __launch_bounds__(256) sor_pair_init_kernel(SorState *st, double omega,
                                                             unsigned long long *dslot,
                                                             int words) {
@@ -988,6 +1015,20 @@ hipError_t launch_sor_pair(const SorPairArgs<T> &a, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <typename T>
+hipError_t launch_gs_split(const SorPairArgs<T> &a, T *field, int sweeps, hipStream_t s) {
+  if (a.nx % 2 != 0 || a.nx < 6 || a.ny < 6 || a.nz < 6) return hipErrorInvalidValue;
+  const size_t half = (size_t)(a.nx / 2) * a.ny * a.nz;
+  T *c[2] = {field, field + half};
+  const T *f[2] = {a.rhs, a.rhs + half};
+  for (int q = 0; q < 2 * sweeps; ++q)
+    gs_split_kernel<T><<<(unsigned)((half + 255) / 256), 256, 0, s>>>(
+        c[q & 1], c[1 - (q & 1)], f[q & 1], q & 1, a.nx, a.ny, a.nz, a.per[0], a.per[1], a.per[2],
+        T(a.ox), T(a.oy), T(a.oz), T(a.A), T(a.invA));
+  return hipGetLastError();
+}
+
+template hipError_t launch_gs_split<float>(const SorPairArgs<float> &, float *, int, hipStream_t);
 template bool sor_whole<float>(SorPairArgs<float> &);
 template bool sor_whole<double>(SorPairArgs<double> &);
 template hipError_t launch_sor_pair_init<float>(const SorPairArgs<float> &, double, hipStream_t);
