@@ -506,7 +506,7 @@ struct SorRun {
       }
       if (hst->done) break;
       // At most two launches per iteration (a pair and its first sweep again).
-      if (pa.launch > 2 * pa.kmax + 16) return fail("SOR state did not close after kmax");
+      if (pa.launch > 2ll * pa.kmax + 16) return fail("SOR state did not close after kmax");
       first = false;
       batch = pa.whole ? 1 : 8;
     }
