@@ -211,7 +211,8 @@ __device__ __forceinline__ PairStep pair_decide(const SorSched &P, double da, do
       s.om_b = s.om_a;
       return s;
     }
-    if (!stop && P.n == 2 && om != P.om_b) {  // the pair with its own omegas
+    // The pair with its own omegas (bits: a NaN omega is no change either).
+    if (!stop && P.n == 2 && __double_as_longlong(om) != __double_as_longlong(P.om_b)) {
       s.n = 2;
       s.om_b = om;
       return s;

@@ -20,3 +20,21 @@ def test_any_kmax(shape, kmax):
         got.append((capi.poisson(p, rhs, (0.3, 0.35, 0.4), 1.6, 1e-6, k, 0, "0000"), p))
     assert got[0][0] == got[1][0] and 20 < got[0][0][0] < 5000
     assert np.array_equal(got[0][1], got[1][1])
+
+
+# One block, resting tiles, the march.  The one-iteration kernel's largest update leaves
+# out NaN, so a solve with omega = NaN ends on eps once the field is NaN.
+@pytest.mark.parametrize("shape", [(12, 12, 16), (20, 24, 40), (20, 90, 264)])
+@pytest.mark.parametrize("idyn", [0, 1])
+@pytest.mark.parametrize("omega", [np.nan, np.inf])
+def test_omega_not_finite(shape, idyn, omega):
+    rhs, p0 = [a.astype(np.float32) for a in rand_fields(shape, 2, seed=78)]
+    got = []
+    for variant in (0, 2):
+        p = p0.copy()
+        it, dmax, reason, om = capi.poisson_f32(p, rhs, (0.3, 0.35, 0.4), omega, 1e-6, 12, idyn,
+                                                "0000", variant=variant)
+        got.append((it, dmax, reason, p, om))
+    assert got[0][:3] == got[1][:3]
+    assert np.array_equal(got[0][3], got[1][3], equal_nan=True)
+    assert np.array_equal(got[0][4], got[1][4], equal_nan=True)
