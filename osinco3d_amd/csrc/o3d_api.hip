@@ -1049,12 +1049,14 @@ int poisson_dev(T *pp, const T *rhs, double dx, double dy, double dz, int nx, in
     const int h = n / 2;
     HIPCHK(launch_split<T>(pp, other, other + h, nx, ny, nz, g_stream));
     HIPCHK(launch_split<T>(rhs, rs, rs + h, nx, ny, nz, g_stream));
-    // pp is free while its split copy is the iterate.
+    // pp is written once the solve has ended: one that fails leaves it as it was.
+    T *b1;
+    CHK(s.scratch(n, &b1));
     r.pair = true;
-    r.pa = pair_args<T>(a, other, pp, rs, dslot);
+    r.pa = pair_args<T>(a, other, b1, rs, dslot);
     rc = r.run(*omega, 16, &sweeps);
-    if (rc == 0 && r.hst->result == 1) HIPCHK(launch_copy<T>(other, pp, n, g_stream));
-    if (rc == 0) HIPCHK(launch_unsplit<T>(pp, other, other + h, nx, ny, nz, g_stream));
+    const T *q = r.hst->result == 1 ? b1 : other;
+    if (rc == 0) HIPCHK(launch_unsplit<T>(pp, q, q + h, nx, ny, nz, g_stream));
   }
   if (!r.pair) {
     rc = r.run(*omega, 16, &sweeps);
