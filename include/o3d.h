@@ -357,7 +357,8 @@ int o3d_copy(void *dst, const void *src, size_t bytes);
  * last step: total ms of complete sweep batches, the number of sweeps
  * (iterations) and of kernel launches in them, per precision (index 0 FP64,
  * 1 FP32; a launch is one iteration in the fused kernel and two with
- * colour-split storage).
+ * colour-split storage, fewer where idyn = 1 changes omega within a pair; a
+ * solve that runs in one launch is not timed).
  * launches2 may be NULL. */
 int o3d_solver_sor_timing(void *handle, double *ms2, int *sweeps2, int *launches2);
 /* Mixed form with colour-split sweeps: `iterations` back-to-back FP32

@@ -477,6 +477,7 @@ struct SorRun {
     if (pa.whole) batch = 1;
     pa.launch = 0;
     bool first = true;
+    int before = 0;  // iterations at the end of the last batch
     while (true) {
       hipEvent_t e0 = (*events)[0], e1 = (*events)[1];
       bool mid_set = false;
@@ -492,16 +493,19 @@ struct SorRun {
       HIPCHK(hipEventRecord(e1, g_stream));
       HIPCHK(hipMemcpyAsync(hst, st, sizeof(SorState), hipMemcpyDeviceToHost, g_stream));
       HIPCHK(hipStreamSynchronize(g_stream));
-      // Timed are launches that ran two iterations each: a batch the solve
-      // did not end in, or the Gauss-Seidel opening.
-      const int timed = pa.whole     ? 0
-                        : !hst->done ? batch - 1
-                                   : (mid_set && hst->sweeps >= pa.gs ? pa.gs / 2 - 1 : 0);
+      // Timed are launches that all ran: of a batch the solve did not end in, or of the
+      // Gauss-Seidel opening.  They count with their share of the iterations the batch
+      // brought (two each, less where a change of omega had a pair run again).
+      const bool opening = mid_set && hst->sweeps >= pa.gs && pa.idyn != 1;
+      const int timed = pa.whole ? 0 : !hst->done ? batch - 1 : (opening ? pa.gs / 2 - 1 : 0);
+      const int brought = hst->done ? 2 * timed
+                                    : (int)((long long)(hst->sweeps - before) * timed / batch);
+      before = hst->sweeps;
       if (timed > 0) {
         float ms = 0.f;
         HIPCHK(hipEventElapsedTime(&ms, e0, hst->done ? mid : e1));
         ms_full += ms;
-        sweeps_full += 2 * timed;
+        sweeps_full += brought;
         launches_full += timed;
       }
       if (hst->done) break;
@@ -3146,10 +3150,12 @@ extern "C" int o3d_solver_sor_period(void *handle, int iterations, double *us) {
     if (r.pa.launch == 0) HIPCHK(hipEventRecord(e0, g_stream));
   }
   HIPCHK(hipEventRecord(e1, g_stream));
-  HIPCHK(hipEventSynchronize(e1));
+  HIPCHK(hipMemcpyAsync(S.hst, S.st, sizeof(SorState), hipMemcpyDeviceToHost, g_stream));
+  HIPCHK(hipStreamSynchronize(g_stream));
   float ms = 0.f;
   HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-  *us = 1e3 * (double)ms / (2 * (launches - 1));
+  // The timed launches' share of the iterations (two a launch unless idyn = 1).
+  *us = 1e3 * (double)ms / (S.hst->sweeps * (double)(launches - 1) / launches);
   return 0;
 }
 

@@ -38,3 +38,19 @@ def test_omega_not_finite(shape, idyn, omega):
     assert got[0][:3] == got[1][:3]
     assert np.array_equal(got[0][3], got[1][3], equal_nan=True)
     assert np.array_equal(got[0][4], got[1][4], equal_nan=True)
+
+
+# idyn = 1: where omega changes after a pair's first iteration the next launch runs the
+# pair again; the timing counts each iteration of the solve once.
+def test_timed_iterations_of_changing_omega():
+    from osinco3d_amd.config import tgv_config
+    from osinco3d_amd.solver import FP64, Solver, taylor_green
+    cfg = tgv_config(48, 1, 2, kmax=40)
+    cfg.idyn, cfg.omega = 1, 4.0  # above 2 the updates grow, and omega falls with each
+    s = Solver(cfg, FP64)
+    s.upload(*taylor_green(cfg))
+    done = s.step(1)["sor_exit_iter"] - 1
+    ms, sweeps, launches = s.sor_timing(launches=True)
+    print(f"iterations {done}, timed {sweeps[0]} in {launches[0]} launches, {ms[0]:.3f} ms")
+    assert done == 40 and 0 < sweeps[0] <= done and ms[0] > 0
+    s.close()
