@@ -727,7 +727,8 @@ extern "C" int o3d_stream_probe(size_t bytes_per_buffer, int reps, double *gbs, 
   hipEvent_t e0 = nullptr, e1 = nullptr;
   int rc = 0;
   for (int q = 0; q < 3 && rc == 0; ++q)
-    if (hipMalloc((void **)&buf[q], n4 * 16) != hipSuccess) rc = fail("stream probe: hipMalloc");
+    if (!(buf[q] = (float4 *)ScratchPool::get().allocate(n4 * 16)))
+      rc = fail("stream probe: hipMalloc");
   if (rc == 0 && (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess))
     rc = fail("stream probe: events");
   if (rc == 0) {
@@ -2455,7 +2456,8 @@ struct LwSums {
 
 int lw_sums_alloc(LwSums &w) {
   if (w.part) return 0;
-  HIPCHK(hipMalloc((void **)&w.part, 2 * kLwBlocks * sizeof(double)));
+  w.part = (double *)ScratchPool::get().allocate(2 * kLwBlocks * sizeof(double));
+  if (!w.part) return fail("out of device memory (%zu bytes)", 2 * kLwBlocks * sizeof(double));
   HIPCHK(hipHostMalloc((void **)&w.hpart, 2 * kLwBlocks * sizeof(double)));
   return 0;
 }
@@ -2835,6 +2837,10 @@ double solver_omega(void *s) { return ((Solver *)s)->omega; }
 double solver_eps(void *s) { return ((Solver *)s)->p.eps; }
 hipStream_t current_stream() { return g_stream; }
 int set_error(const char *msg) { return fail("%s", msg); }
+hipError_t device_malloc(void **p, size_t bytes) {
+  *p = ScratchPool::get().allocate(bytes);
+  return *p ? hipSuccess : hipErrorOutOfMemory;
+}
 }  // namespace o3d
 
 extern "C" int o3d_solver_create(const o3d_params *p, void **handle) {

@@ -16,5 +16,7 @@ double solver_omega(void *s);
 double solver_eps(void *s);
 hipStream_t current_stream();
 int set_error(const char *msg);
+// hipMalloc, once more without the scratch kept between calls when it fails.
+hipError_t device_malloc(void **p, size_t bytes);
 }  // namespace o3d
 

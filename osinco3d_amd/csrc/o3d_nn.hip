@@ -1129,7 +1129,7 @@ int alloc_activations(Net &n, int nx, int ny, int nz) {
                     {&n.d0, 0, 16}, {&n.dz, 0, 32}};
   size_t total = 0;
   for (const A &a : acts) total += ((n.V[a.level] * a.ch * sizeof(bf16) + 255) / 256) * 256;
-  NNCHK(hipMalloc(&n.act_arena, total));
+  NNCHK(o3d::device_malloc(&n.act_arena, total));
   char *p = (char *)n.act_arena;
   for (const A &a : acts) {
     *a.p = (bf16 *)p;
@@ -1143,7 +1143,7 @@ int alloc_activations(Net &n, int nx, int ny, int nz) {
                      {&n.g_e1a, 1, 32}, {&n.g_p1, 1, 16}, {&n.g_e0, 0, 16}, {&n.g_e0a, 0, 16}};
   total = 0;
   for (const G &g : grads) total += ((n.V[g.level] * g.ch * 4 + 255) / 256) * 256;
-  NNCHK(hipMalloc((void **)&n.gbuf, total));
+  NNCHK(o3d::device_malloc((void **)&n.gbuf, total));
   p = (char *)n.gbuf;
   for (const G &g : grads) {
     *g.p = (float *)p;
@@ -1168,7 +1168,7 @@ int alloc_activations(Net &n, int nx, int ny, int nz) {
   bb[14] = up((size_t)head_blocks(n) * 17 * 4);
   total += bb[14] + up(zt * sizeof(bf16)) + up(xt * sizeof(bf16));
   p = nullptr;
-  NNCHK(hipMalloc((void **)&p, total));
+  NNCHK(o3d::device_malloc((void **)&p, total));
   n.part = (float *)p;
   for (int li = 0; li < 15; ++li) {
     if (li < 14) { n.wpart[li] = (float *)p; p += wb[li]; }
@@ -1426,7 +1426,7 @@ extern "C" int o3d_nn_create(int nx, int ny, int nz, unsigned long long seed, vo
   int rc = 0;
   auto al = [&](void **p, size_t bytes) {
     if (rc) return;
-    if (hipMalloc(p, bytes) != hipSuccess) { rc = o3d::set_error("hipMalloc failed"); return; }
+    if (o3d::device_malloc(p, bytes) != hipSuccess) { rc = o3d::set_error("hipMalloc failed"); return; }
     n->allocs.push_back(*p);
     if (hipMemset(*p, 0, bytes) != hipSuccess) rc = o3d::set_error("hipMemset failed");
   };

@@ -1,0 +1,41 @@
+"""Allocations of the library's own give back the scratch it keeps between calls
+before they fail: a network is created on a device whose last memory that scratch
+holds."""
+import numpy as np
+import pytest
+
+from osinco3d_amd import capi, warmstart
+
+pytestmark = pytest.mark.gpu
+
+
+def test_network_takes_the_kept_scratch():
+    import torch
+    lib = capi.load()
+    lib.o3d_release_scratch()
+    # Idle scratch of about 0.8 GB: the tendency and the sums of a 100 M-node field.
+    phi = torch.zeros((100, 1000, 1000), dtype=torch.float64, device="cuda")
+    f = torch.zeros((1,) + phi.shape, dtype=torch.float64, device="cuda")
+    capi.transeq(phi, [phi, phi, phi], phi, f, 100.0, 0.7, [0.01] * 3, [0.0] * 3, [0.0] * 3, 1, 1,
+                 (0.1, 0.2, 0.3), 0, None, (0, 0, 0))
+    del phi, f
+    torch.cuda.empty_cache()
+    # A 96x96x48 network takes about 0.6 GB; leave less than that free.
+    warmstart.Network(16, 16, 16).close()
+    hold, left = [], torch.cuda.mem_get_info()[0]
+    for _ in range(4):  # memory of the calls before comes back with a delay
+        if left <= 256 << 20:
+            break
+        hold.append(torch.empty(left - (192 << 20), dtype=torch.uint8, device="cuda"))
+        left = torch.cuda.mem_get_info()[0]
+    print(f"left free {left >> 20} MB")
+    assert left <= 256 << 20
+    net = warmstart.Network(96, 96, 48)
+    x = torch.zeros((2, 96 * 96 * 48), dtype=torch.float32, device="cuda")
+    out = torch.empty_like(x[0])
+    net.forward(x, out)
+    assert np.isfinite(float(out.sum()))
+    net.close()
+    del hold
+    torch.cuda.empty_cache()
+    lib.o3d_release_scratch()
