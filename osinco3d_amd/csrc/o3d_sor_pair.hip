@@ -24,12 +24,16 @@
 // of a pair is a guess that the first does not end the solve or change omega.
 // The next launch checks it; when it was wrong the source buffer still holds
 // the iterate before the pair, and that launch runs the first iteration (or
-// the pair with the right omegas) again.
+// the pair with the right omegas) again.  With idyn = 1 that costs a launch per change
+// of omega, of which solves have few: 400 iterations from omega 1.5 or 1.99 take 53.0
+// to 53.2 us each at FP64 256^3 (52.8 with idyn = 0), 12.0 at 128^3 (11.6), 6.7 to 6.9
+// at 64^3 (6.4).
 //
 // What bounds it: small grids by the plane step, 0.85 us (0.95 us with the
 // tests of the first steps as branches inside the march, which kept the
 // compiler from interleaving the half sweeps: 64^3 16.7 -> 15.2 us a launch);
-// large ones by memory, at 4.3 TB/s of the traffic that reaches the fabric (the
+// large ones by memory, at 4.3 TB/s (FP64, FP32 4.9) of the traffic that reaches the
+// fabric, 1.16 (1.26) times the algorithmic bytes at 256^3 (the
 // same kernel without its arithmetic takes as long), and there by the halos,
 // which neighbouring tiles find in their XCD's L2 only while they march side by
 // side.  So tiles are handed to the XCDs in
@@ -126,11 +130,12 @@ __device__ __forceinline__ double max_abs(double m, double d) {
   return r;
 }
 
-// num / A.  FP64 divides as the reference does: the correction step of a
-// correctly rounded division from the reciprocal invA (quotient, exact
-// remainder by fma, corrected quotient), the last part of what the compiler
-// emits for num / A, whose refinement of 1 / A per node is left out; zero,
-// infinite and NaN numerators by div_fixup.  FP32 multiplies by 1 / A.
+// num / A.  FP64 divides as the reference does: from the correctly rounded reciprocal
+// invA, the quotient, its exact remainder by fma and the quotient corrected by it are
+// correctly rounded (Markstein's theorem), as long as the remainder is a normal number
+// or exact: for |num| above 2^-968.  Below, the last bit may differ from num / A; such
+// a numerator is a sum of pressures and rhs all under 1e-291.  Zero, infinite and NaN
+// numerators by div_fixup.  FP32 multiplies by 1 / A.
 __device__ __forceinline__ double pair_div(double num, double A, double invA) {
   const double q = num * invA;
   const double r = __builtin_fma(-q, A, num);
