@@ -7,9 +7,10 @@
 // the trilinear interpolation of the result to the guess.  The SOR solve
 // that follows still decides convergence (same stop rule), so the
 // correction only changes where SOR starts.  The grids are small (128^3 and
-// below at 256^3): the per-level kernels give each thread one cell of the
-// colour being relaxed (or a pair of cells), and the levels of at most 16^3
-// cells run as one V-cycle in one block's LDS; the launch count dominates.
+// below at 256^3) and the launch count dominates: a level above the last takes
+// one launch per sweep, the levels of at most 16^3 cells run as one V-cycle in
+// one block's LDS, and a larger last level takes two sweeps per launch or, where
+// its rows are too wide for that, one launch per colour.
 #include <algorithm>
 #include <utility>
 
