@@ -128,8 +128,9 @@ int o3d_predict_velocity(double *ux_pred, double *uy_pred, double *uz_pred, cons
  * the reference).  omega is in/out
  * (dynamic omega persists, idyn = 1).  exit_iter = the iteration the
  * reference prints on exit (kmax+1 when kmax ran out); reason 0 = dmax < eps,
- * 1 = stagnation, 2 = kmax.  Any of the three out pointers may be NULL.  pp
- * is written once the solve has ended on a grid with nx even. */
+ * 1 = stagnation, 2 = kmax.  Any of the three out pointers may be NULL.  With
+ * nx even and memory for three fields pp is written once the solve has
+ * ended. */
 int o3d_poisson(double *pp, const double *rhs, double dx, double dy, double dz, int nx, int ny,
                 int nz, double *omega, double eps, int kmax, int idyn, int solver,
                 int *exit_iter, double *dmax, int *reason);

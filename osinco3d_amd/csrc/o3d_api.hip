@@ -1055,13 +1055,18 @@ int poisson_dev(T *pp, const T *rhs, double dx, double dy, double dz, int nx, in
     HIPCHK(launch_split<T>(pp, other, other + h, nx, ny, nz, g_stream));
     HIPCHK(launch_split<T>(rhs, rs, rs + h, nx, ny, nz, g_stream));
     // pp is written once the solve has ended: one that fails leaves it as it was.
+    // (Without memory for that it is the second buffer itself.)
     T *b1;
-    CHK(s.scratch(n, &b1));
+    if (s.scratch(n, &b1) != 0) b1 = pp;
     r.pair = true;
     r.pa = pair_args<T>(a, other, b1, rs, dslot);
     rc = r.run(*omega, 16, &sweeps);
-    const T *q = r.hst->result == 1 ? b1 : other;
-    if (rc == 0) HIPCHK(launch_unsplit<T>(pp, q, q + h, nx, ny, nz, g_stream));
+    if (rc == 0) {
+      const bool second = r.hst->result == 1;
+      if (second && b1 == pp) HIPCHK(launch_copy<T>(other, pp, n, g_stream));
+      const T *q = second && b1 != pp ? b1 : other;
+      HIPCHK(launch_unsplit<T>(pp, q, q + h, nx, ny, nz, g_stream));
+    }
   }
   if (!r.pair) {
     rc = r.run(*omega, 16, &sweeps);
