@@ -1381,11 +1381,9 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
   CHK(s.scratch(mg_plan(H, m0, h, per), &mgbuf));
   mg_bind(H, mgbuf);
   H.levels = std::min(H.levels, std::max(nlevels - 1, 0));
-  const bool pairs = sor_buffer_fits<float, float>(nx, ny, nz);
   float *R, *E, *E2 = nullptr;
   CHK(s.scratch(n, &R));
   CHK(s.scratch(n, &E));
-  if (pairs) CHK(s.scratch(n, &E2));
   const int nb = residual_blocks(nx, ny, nz);
   double *part;
   CHK(s.scratch((size_t)4 * nb + 4, &part));
@@ -1415,6 +1413,9 @@ extern "C" int o3d_poisson_multigrid(double *pp, const double *rhs, double dx, d
   a.idyn = 0;
   a.it = 0;
   a.gs = npre + npost;
+  // Beyond the pair kernel's grids, or without memory for its second buffer, the
+  // smoother in place.
+  const bool pairs = sor_buffer_fits<float, float>(nx, ny, nz) && s.scratch(n, &E2) == 0;
   run.pair = true;
   run.pa = pair_args<float>(a, E, E2, R, dslot);
   int rc = 0, done = 0, why = 2;

@@ -41,9 +41,10 @@ def test_network_takes_the_kept_scratch():
     lib.o3d_release_scratch()
 
 
-# The solve asks for three fields of scratch and does with two, for an even and an odd
-# number of launches.
-def test_sor_with_two_fields_of_scratch():
+# The SOR solve asks for three fields of scratch and does with two, for an even and an
+# odd number of launches; the multigrid solve for three FP32 fields and the levels (3.4
+# fields of 64 MiB) and does with one less.
+def test_solves_with_a_field_less_of_scratch():
     import torch
     lib = capi.load()
     g = torch.Generator(device="cuda").manual_seed(80)
@@ -51,7 +52,10 @@ def test_sor_with_two_fields_of_scratch():
     runs = [((0.3, 0.35, 0.4), 1.6, 1e-30, kmax, 0, "0000") for kmax in (5, 8)]
     ref = [torch.zeros_like(rhs) for _ in runs]
     want = [capi.poisson(p, rhs, *args) for p, args in zip(ref, runs)]
-    p = [torch.zeros_like(rhs) for _ in runs]
+    mg = ((0.3, 0.35, 0.4), "0000")
+    ref.append(torch.zeros_like(rhs))
+    want.append(capi.poisson_multigrid(ref[2], rhs, *mg, tol=0.0, max_cycles=2))
+    p = [torch.zeros_like(rhs) for _ in ref]
     torch.cuda.synchronize()
     lib.o3d_release_scratch()
     torch.cuda.empty_cache()
@@ -64,6 +68,12 @@ def test_sor_with_two_fields_of_scratch():
     print(f"left free {left >> 20} MB")
     assert 260 << 20 < left <= 380 << 20
     got = [capi.poisson(a, rhs, *args) for a, args in zip(p, runs)]
+    lib.o3d_release_scratch()
+    left = torch.cuda.mem_get_info()[0]
+    hold.append(torch.empty(left - (190 << 20), dtype=torch.uint8, device="cuda"))
+    print(f"then {torch.cuda.mem_get_info()[0] >> 20} MB")
+    assert torch.cuda.mem_get_info()[0] < 216 << 20
+    got.append(capi.poisson_multigrid(p[2], rhs, *mg, tol=0.0, max_cycles=2))
     del hold
     torch.cuda.empty_cache()
     assert got == want
